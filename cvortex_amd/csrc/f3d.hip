@@ -499,84 +499,204 @@ F3Fn f3_reduce(int mask) {
 }
 // Influence matrix (cvtx_F3D_inf_mtrx, reference src/F3D.cpp:204-227):
 //   out[i * n_fil + j] = vel(filament j, point i) . dir_i
-// with the filament's own strength, the velocity term of f3d_kernel (same
-// well-conditioned formula and the same flush of non-finite terms).  Each
-// lane owns INF_NJ consecutive filaments (columns) of its workgroup's
-// block and the workgroup walks `rows` consecutive points, whose
-// coordinates and directions are the same in every lane.  Where a lane's
-// filaments form a polyline (each starts, bit for bit, where the previous
-// one ends, as the spanwise segments of a vortex lattice do) and every lane
-// of the wave has that, the shared end point's distance terms are computed
-// once per row: the same values the unshared form gives, with one rsq and
-// seven other instructions fewer per element.  16384 x 16384 lattice:
-// 0.362 -> 0.348 ms (three A/B pairs on one box).  Four filaments per lane
-// were slower (0.41 ms: a wave's stores then cover 1 KiB at a 16-byte
-// stride), and two columns written as one 8-byte store gained nothing.
-constexpr int INF_NJ = 2;
+// with the filament's own strength and, as in f3d_kernel, non-finite terms
+// flushed to zero.  Each lane owns NF adjacent filaments (columns) of its
+// workgroup's block and the workgroup walks `rows` consecutive points, staged
+// in LDS (a broadcast read puts them in VGPRs; an SGPR operand would halve
+// the issue rate of every instruction that reads it).
+//
+// Two forms of the element.  inf_general is f3d_pair's, right for any point.
+// The far form holds where S^2 >= 2 L^2 for S = |r1| + |r2| and the
+// filament's length L (then r1.r2 >= 0 and no term is infinite): with
+// S^2 - L^2 = 2 (|r1||r2| + r1.r2),
+//   k = (Gamma/4pi) (y1 + y2) / (|r1||r2| + r1.r2) = (Gamma/2pi) S y1 y2 / (S^2 - L^2)
+// needs neither r1.r2 nor |c|^2 nor the selects, and c = r0 x r1 (r0 = b - a,
+// kept in registers) is, away from the segment, the better conditioned
+// product.  S^2 - L^2 loses at most one bit there.  S is at least twice the
+// distance D of the point from the filament, so D^2 >= L^2 / 2 is enough, and
+// a wave decides it for its 64 NF filaments and all its rows at once: lane l
+// compares row l's distance from the box around the wave's filaments with
+// their longest, and a ballot gives one bit per row (a test per element
+// instead: 222 against 217 us on the matrix below).  Where the filaments of
+// every lane of the wave form a polyline (each starts, bit for bit, where the
+// previous one ends, as the spanwise segments of a vortex lattice do), a
+// shared end point's distance terms are computed once per row.
+//
+// What bounds it: the matrix's write and the vector units about equally.  For
+// 16384 x 16384 (1 GiB) the kernel takes 217-225 us, 4.8-4.9 TB/s of writes
+// (294 us before: every element by the general form, two columns per lane,
+// points in SGPRs); with the element arithmetic left out it takes 167 us
+// with 8 rows per workgroup and 213 with 32.  127 x 130 columns 322 -> 260
+// us, 127 x 129 318 -> 262 us.
+template <int NF>
+struct InfCols {
+  float3 a[NF], b[NF], r0[NF];
+  float g[NF], L2[NF];  // Gamma / (2 pi), |r0|^2
+};
 
+__device__ __forceinline__ float3 sub3(float4 x, float3 a) {
+  return make_float3(x.x - a.x, x.y - a.y, x.z - a.z);
+}
+__device__ __forceinline__ float dot3(float3 a, float3 b) {
+  return __builtin_fmaf(a.x, b.x, __builtin_fmaf(a.y, b.y, a.z * b.z));
+}
+__device__ __forceinline__ float3 cross3(float3 a, float3 b) {
+  return make_float3(__builtin_fmaf(a.y, b.z, -a.z * b.y), __builtin_fmaf(a.z, b.x, -a.x * b.z),
+                     __builtin_fmaf(a.x, b.y, -a.y * b.x));
+}
+
+// One element by f3d_pair's formula, projected on e (g = Gamma / (4 pi)).
+__device__ __forceinline__ float inf_general(float3 r1, float3 r2, float g, float3 e) {
+  const float3 c = cross3(r1, r2);
+  const float cc = dot3(c, c);
+  const float n1s = dot3(r1, r1), n2s = dot3(r2, r2);
+  const float n1 = n1s * __builtin_amdgcn_rsqf(n1s);
+  const float n2 = n2s * __builtin_amdgcn_rsqf(n2s);
+  const float P = n1 * n2;
+  const float sum = n1 + n2;
+  const float d12 = dot3(r1, r2);
+  const bool same_side = d12 >= 0.f;
+  const float den = same_side ? P * (P + d12) : P * cc;
+  const float num = same_side ? sum : sum * (P - d12);
+  float kk = g * num * __builtin_amdgcn_rcpf(den);
+  kk = (__builtin_fabsf(kk) < __builtin_inff()) ? kk : 0.f;
+  return kk * dot3(c, e);
+}
+
+constexpr long INF_STREAM_ELEMENTS = 64l << 20;  // 256 MiB of floats
+constexpr int INF_ROWS = 32;  // rows a workgroup stages at most
+
+// The rows of one workgroup.  WHOLE: the lane's columns are all inside the
+// matrix and may be written as one NF * 4-byte store
+// (STREAM: past the caches).
+template <int NF, bool SHARE, bool WHOLE, bool STREAM>
+__device__ __forceinline__ void inf_rows(const InfCols<NF>& c, const float4* s_x, const float4* s_e,
+                                         unsigned long long far_rows, int nr, int j0, int n_fil,
+                                         float* __restrict__ o) {
+  using Vec = float __attribute__((ext_vector_type(NF)));
+  using Vec4 = float __attribute__((ext_vector_type(NF), aligned(4)));  // any float's address
+  int iv = in_vgpr(0);
+  float4 xn = s_x[iv], en = s_e[iv];
+  for (int i = 0; i < nr; ++i, o += n_fil) {
+    const float4 x = xn;
+    const float3 e = make_float3(en.x, en.y, en.z);
+    ++iv;
+    // the next row's point is read while this row's elements are computed
+    // (the arrays have a slot past the last row)
+    xn = s_x[iv];
+    en = s_e[iv];
+    Vec v;
+    if ((far_rows >> i) & 1) {
+      float3 r2;
+      float y2, n2;
+#pragma unroll
+      for (int f = 0; f < NF; ++f) {
+        float3 r1 = r2;
+        float y1 = y2, n1 = n2;
+        if (f == 0 || !SHARE) {
+          r1 = sub3(x, c.a[f]);
+          const float ns = dot3(r1, r1);
+          y1 = __builtin_amdgcn_rsqf(ns);
+          n1 = ns * y1;
+        }
+        r2 = sub3(x, c.b[f]);
+        const float ns = dot3(r2, r2);
+        y2 = __builtin_amdgcn_rsqf(ns);
+        n2 = ns * y2;
+        const float S = n1 + n2;
+        const float den = __builtin_fmaf(S, S, -c.L2[f]);
+        const float ce = dot3(cross3(c.r0[f], r1), e);
+        v[f] = ((c.g[f] * (S * y1)) * y2) * (ce * __builtin_amdgcn_rcpf(den));
+      }
+    } else {
+#pragma unroll
+      for (int f = 0; f < NF; ++f) v[f] = inf_general(sub3(x, c.a[f]), sub3(x, c.b[f]), 0.5f * c.g[f], e);
+    }
+    if constexpr (WHOLE) {
+      if constexpr (STREAM) __builtin_nontemporal_store(v, reinterpret_cast<Vec*>(o + j0));
+      else *reinterpret_cast<Vec4*>(o + j0) = v;
+    } else {
+#pragma unroll
+      for (int f = 0; f < NF; ++f)
+        if (j0 + f < n_fil) o[j0 + f] = v[f];
+    }
+  }
+}
+
+template <int NF, bool STREAM>
 __global__ __launch_bounds__(256) void f3d_inf_kernel(const float4* __restrict__ fa,
                                                       const float4* __restrict__ fb, int n_fil,
                                                       const float4* __restrict__ mes,
                                                       const float4* __restrict__ dir, int n_mes,
                                                       int rows, float* __restrict__ out) {
-  const int j0 = (blockIdx.x * 256 + threadIdx.x) * INF_NJ;
-  float3 a[INF_NJ], b[INF_NJ];
-  float g[INF_NJ];
+  __shared__ float4 s_x[INF_ROWS + 1], s_e[INF_ROWS + 1];
+  const int tid = threadIdx.x;
+  const int j0 = (blockIdx.x * 256 + tid) * NF;
+  const int i0 = blockIdx.y * rows;
+  const int nr = min(rows, n_mes - i0);
+  if (tid <= nr) {
+    const bool in = tid < nr;
+    s_x[tid] = in ? mes[i0 + tid] : make_float4(0.f, 0.f, 0.f, 0.f);
+    s_e[tid] = in ? dir[i0 + tid] : make_float4(0.f, 0.f, 0.f, 0.f);
+  }
+  InfCols<NF> c;
   bool linked = true;
 #pragma unroll
-  for (int k = 0; k < INF_NJ; ++k) {
-    const int j = min(j0 + k, n_fil - 1);
+  for (int f = 0; f < NF; ++f) {
+    const int j = min(j0 + f, n_fil - 1);
     const float4 fa4 = fa[j], fb4 = fb[j];
-    a[k] = make_float3(fa4.x, fa4.y, fa4.z);
-    b[k] = make_float3(fb4.x, fb4.y, fb4.z);
-    g[k] = fa4.w * (float)(1.0 / (4.0 * M_PI));
-    if (k > 0)
-      linked = linked && __float_as_uint(a[k].x) == __float_as_uint(b[k - 1].x) &&
-               __float_as_uint(a[k].y) == __float_as_uint(b[k - 1].y) &&
-               __float_as_uint(a[k].z) == __float_as_uint(b[k - 1].z);
+    c.a[f] = make_float3(fa4.x, fa4.y, fa4.z);
+    c.b[f] = make_float3(fb4.x, fb4.y, fb4.z);
+    c.r0[f] = make_float3(fb4.x - fa4.x, fb4.y - fa4.y, fb4.z - fa4.z);
+    c.L2[f] = dot3(c.r0[f], c.r0[f]);
+    c.g[f] = 2.f * (fa4.w * (float)(1.0 / (4.0 * M_PI)));
+    if (f > 0)
+      linked = linked && __float_as_uint(c.a[f].x) == __float_as_uint(c.b[f - 1].x) &&
+               __float_as_uint(c.a[f].y) == __float_as_uint(c.b[f - 1].y) &&
+               __float_as_uint(c.a[f].z) == __float_as_uint(c.b[f - 1].z);
   }
+  const bool whole = ((int)blockIdx.x + 1) * (256 * NF) <= n_fil;
+  __syncthreads();
+  float* o = out + (size_t)i0 * (size_t)n_fil;
   // one answer for the whole wave, so the row loop branches uniformly
   const bool share = __all(linked);
-  const int i0 = blockIdx.y * rows;
-  const int i1 = min(i0 + rows, n_mes);
-  for (int i = i0; i < i1; ++i) {
-    const float4 x = mes[i];
-    const float4 e = dir[i];
-    float r1x = x.x - a[0].x, r1y = x.y - a[0].y, r1z = x.z - a[0].z;
-    float n1s = __builtin_fmaf(r1x, r1x, __builtin_fmaf(r1y, r1y, r1z * r1z));
-    float n1 = n1s * __builtin_amdgcn_rsqf(n1s);
+  // bit i: row i is far from all the wave's filaments (see above), and every
+  // distance is finite and normal
+  Box<3> wb;
+  float l2 = 0.f;
+  wb.finite = true;
 #pragma unroll
-    for (int k = 0; k < INF_NJ; ++k) {
-      if (k > 0 && !share) {
-        r1x = x.x - a[k].x;
-        r1y = x.y - a[k].y;
-        r1z = x.z - a[k].z;
-        n1s = __builtin_fmaf(r1x, r1x, __builtin_fmaf(r1y, r1y, r1z * r1z));
-        n1 = n1s * __builtin_amdgcn_rsqf(n1s);
-      }
-      const float r2x = x.x - b[k].x, r2y = x.y - b[k].y, r2z = x.z - b[k].z;
-      const float cx = __builtin_fmaf(r1y, r2z, -r1z * r2y);
-      const float cy = __builtin_fmaf(r1z, r2x, -r1x * r2z);
-      const float cz = __builtin_fmaf(r1x, r2y, -r1y * r2x);
-      const float cc = __builtin_fmaf(cx, cx, __builtin_fmaf(cy, cy, cz * cz));
-      const float n2s = __builtin_fmaf(r2x, r2x, __builtin_fmaf(r2y, r2y, r2z * r2z));
-      const float n2 = n2s * __builtin_amdgcn_rsqf(n2s);
-      const float P = n1 * n2;
-      const float sum = n1 + n2;
-      const float d12 = __builtin_fmaf(r1x, r2x, __builtin_fmaf(r1y, r2y, r1z * r2z));
-      const bool same_side = d12 >= 0.f;
-      const float den = same_side ? P * (P + d12) : P * cc;
-      const float num = same_side ? sum : sum * (P - d12);
-      float kk = g[k] * num * __builtin_amdgcn_rcpf(den);
-      kk = (__builtin_fabsf(kk) < __builtin_inff()) ? kk : 0.f;
-      const float v = kk * __builtin_fmaf(cx, e.x, __builtin_fmaf(cy, e.y, cz * e.z));
-      if (j0 + k < n_fil) out[(size_t)i * (size_t)n_fil + j0 + k] = v;
-      // the next filament starts at this one's end point
-      r1x = r2x;
-      r1y = r2y;
-      r1z = r2z;
-      n1 = n2;
+  for (int d = 0; d < 3; ++d) { wb.lo[d] = __builtin_inff(); wb.hi[d] = -__builtin_inff(); }
+#pragma unroll
+  for (int f = 0; f < NF; ++f) {
+    const float pa[3] = {c.a[f].x, c.a[f].y, c.a[f].z}, pb[3] = {c.b[f].x, c.b[f].y, c.b[f].z};
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      wb.lo[d] = fminf(wb.lo[d], fminf(pa[d], pb[d]));
+      wb.hi[d] = fmaxf(wb.hi[d], fmaxf(pa[d], pb[d]));
+      wb.finite = wb.finite && __builtin_isfinite(pa[d]) && __builtin_isfinite(pb[d]);
     }
+    wb.finite = wb.finite && __builtin_isfinite(c.g[f]);
+    l2 = fmaxf(l2, c.L2[f]);
+  }
+#pragma unroll
+  for (int d = 0; d < 3; ++d) { wb.lo[d] = wave_min(wb.lo[d]); wb.hi[d] = wave_max(wb.hi[d]); }
+  l2 = wave_max(l2);
+  wb.finite = __all(wb.finite);
+  const float4 xr = s_x[min(tid & 63, nr)];  // (slot nr is zero)
+  Box<3> pb;
+  pb.lo[0] = pb.hi[0] = xr.x; pb.lo[1] = pb.hi[1] = xr.y; pb.lo[2] = pb.hi[2] = xr.z;
+  float dmin2, dmax2;
+  box_dist2<3>(wb, pb, dmin2, dmax2);
+  const bool fin = __builtin_isfinite(xr.x) && __builtin_isfinite(xr.y) && __builtin_isfinite(xr.z);
+  const unsigned long long far_rows =
+      __ballot(fin && wb.finite && dmin2 >= 0.51f * l2 && dmin2 >= 1e-30f && dmax2 <= 1e30f);
+  if (whole) {
+    if (share) inf_rows<NF, true, true, STREAM>(c, s_x, s_e, far_rows, nr, j0, n_fil, o);
+    else inf_rows<NF, false, true, STREAM>(c, s_x, s_e, far_rows, nr, j0, n_fil, o);
+  } else {
+    if (share) inf_rows<NF, true, false, STREAM>(c, s_x, s_e, far_rows, nr, j0, n_fil, o);
+    else inf_rows<NF, false, false, STREAM>(c, s_x, s_e, far_rows, nr, j0, n_fil, o);
   }
 }
 
@@ -586,12 +706,22 @@ hipError_t launch_f3d_inf(const float4* fa, const float4* fb, int n_fil, const f
                           const float4* dir, int n_mes, float* out, hipStream_t s) {
   if (n_fil <= 0 || n_mes <= 0) return hipSuccess;
   if (!fa || !fb || !mes || !dir || !out) return hipErrorInvalidValue;
-  // rows per workgroup: enough workgroups to fill the chip several times
-  const int gx = (n_fil + 256 * INF_NJ - 1) / (256 * INF_NJ);
+  // A matrix that outgrows the last-level cache, with rows of whole 128-byte
+  // lines, is written past the caches in 16-byte stores: 16384 x 16384 237 us
+  // with two columns per lane and cached stores, 217 us so.  Where it fits
+  // (3280 x 1149, 15 MB) streaming takes 21 us against 10, and where lines are
+  // shared between rows (127 x 130 columns) 345 us against 260.
+  const bool stream = n_fil % 32 == 0 && ((uintptr_t)out & 127) == 0 &&
+                      (size_t)n_fil * n_mes >= (size_t)INF_STREAM_ELEMENTS;
+  const int per = 256 * (stream ? 4 : 2);
+  // rows per workgroup: two workgroups per CU at least, so that each has rows
+  // to spread its prologue over (3280 x 1149: 22 us with 16 per CU, 9.9 with 2)
+  const int gx = (n_fil + per - 1) / per;
   int rows = 1;
-  while (rows < 64 && (long long)gx * ((n_mes + 2 * rows - 1) / (2 * rows)) >= 4096) rows *= 2;
-  hipLaunchKernelGGL(f3d_inf_kernel, dim3(gx, (n_mes + rows - 1) / rows), dim3(256), 0, s, fa, fb,
-                     n_fil, mes, dir, n_mes, rows, out);
+  while (rows < INF_ROWS && (long long)gx * ((n_mes + 2 * rows - 1) / (2 * rows)) >= 512) rows *= 2;
+  const auto k = stream ? f3d_inf_kernel<4, true> : f3d_inf_kernel<2, false>;
+  hipLaunchKernelGGL(k, dim3(gx, (n_mes + rows - 1) / rows), dim3(256), 0, s, fa, fb, n_fil, mes,
+                     dir, n_mes, rows, out);
   return hipGetLastError();
 }
 
