@@ -2,7 +2,8 @@
 //
 // Filaments stream through LDS in tiles; when a tile is staged each
 // filament is expanded once per workgroup into
-//   { a (start), Gamma/(4pi) },  { b (end), 3 Gamma/(4pi |r0|) },  { r0 = b - a },
+//   { a (start), Gamma/(4pi) },  { b (end), -6 Gamma/(4pi |r0|) },
+//   { r0 = b - a, |r0|^2 / 2 },
 // so the per-pair work only involves the target-dependent quantities.
 //
 // Per pair (x the target): r1 = x - a, r2 = x - b, c = r1 x r2 (= r0 x r1),
@@ -63,8 +64,8 @@ __device__ __forceinline__ void f3d_finish(const double* a, float3 at, const F3D
 }
 
 // One pair by the general formula (any target position): accumulates into
-// acc[0..NA) of one target.  sa = {a, Gamma/(4pi)}, sb = {b, 3 Gamma/(4pi|r0|)},
-// f0 = {r0}.
+// acc[0..NA) of one target.  fa = {a, Gamma/(4pi)}, fb = {b, -6 Gamma/(4pi|r0|)},
+// f0 = {r0, |r0|^2 / 2}.
 template <int MASK>
 __device__ __forceinline__ void f3d_pair(const float4 fa, const float4 fb, const float4 f0,
                                          const float3 xt, const float fin, float* acc) {
@@ -93,7 +94,7 @@ __device__ __forceinline__ void f3d_pair(const float4 fa, const float4 fb, const
     const float rcc = __builtin_amdgcn_rsqf(cc);
     const float cn = cc * rcc;  // |c|; 0 * inf = NaN when c = 0
     const float p12 = __builtin_fmaf(f0.x, r1x + r2x, __builtin_fmaf(f0.y, r1y + r2y, f0.z * (r1z + r2z)));
-    float B = -fb.w * cn * p12 * __builtin_amdgcn_rcpf(P * sum);
+    float B = fb.w * cn * (0.5f * p12) * __builtin_amdgcn_rcpf(P * sum);
     // B is NaN whenever c = 0 (target on the filament's line), so the
     // finiteness of B also drops those pairs
     const bool ok = (__builtin_fabsf(kk) < __builtin_inff()) &&
@@ -121,33 +122,38 @@ __device__ __forceinline__ void f3d_pair(const float4 fa, const float4 fb, const
 // Far tiles (tile_cull.hpp).  When every target of the block is at least
 // half the longest filament of the tile away from the tile's box, every
 // pair has r1.r2 = |x - m|^2 - |r0|^2/4 >= 0 (m the filament's midpoint),
-// so the same-side form holds for all of them, with y_i = 1/|r_i|:
-//   k = (Gamma/4pi) (|r1| + |r2|) / (|r1||r2| (|r1||r2| + r1.r2))
-//     = (Gamma/4pi) (y1 + y2) / (P + r1.r2),           P = |r1||r2|,
-//   1/|r1| - 1/|r2| = -r0.(r1 + r2) y1 y2 / (|r1| + |r2|),
-// and no pair's terms can be infinite.  The reciprocals of P + r1.r2 (and,
-// for the stretching, of |r1| + |r2|) of the group's pairs come from one
-// shared reciprocal (batch_rcp).  The stretching terms of a pair with c = 0
-// (a target on the extension of a filament's line) are dropped, as the
-// general form does (there |c| = 0 and the reference's terms are NaN).
+// so the same-side form holds for all of them and no pair's terms can be
+// infinite.  With y_i = 1/|r_i|, S = |r1| + |r2|, L = |r0| and
+// h = |r1||r2| + r1.r2 = (S^2 - L^2) / 2 (which loses at most a bit or two
+// at the nearest targets):
+//   k = (Gamma/4pi) S / (|r1||r2| h) = (Gamma/4pi) (y1 + y2) / h,
+//   1/|r1| - 1/|r2| = -r0.(r1 + r2) y1 y2 / S,  r0.(r1 + r2) / 2 = r0.r1 - L^2/2,
+// and c = r0 x r1, the better conditioned product away from the segment.
+// The stretching takes 1/h and 1/S from one value, 1/(S h):
+//   k = (Gamma/4pi) S^2 z,  B = -(3 Gamma/4pi L) |c| r0.(r1 + r2) h z,
+//   z = y1 y2 / (S h);
+// the reciprocals of a group's pairs come from one (batch_rcp).  Against the
+// form with r1.r2 and one reciprocal each for h and S it saves three
+// operations of 30 per pair for the velocity and ten of 58 for both outputs.
+// The stretching terms of a pair with c = 0 (a target on the extension of a
+// filament's line) are dropped, as the general form does (there |c| = 0 and
+// the reference's terms are NaN).
+// Bound by vector issue: 2.25 transcendentals per pair along a chain (rsq of
+// the new end point, sqrt of |c|^2, half a rcp), 1.5 for the velocity.
+// 16384 filaments in chains of 128 x 2^20 targets, ms, old form -> this:
+// fused 18.44 -> 14.95, stretching 17.08 -> 14.18, velocity 9.96 -> 9.04.
+// Two pairs per group: the velocity with four takes 9.99 ms (more registers:
+// 12.35 held to 6 waves per SIMD, with spills), with one 12.2.
 template <int MASK, int T>
 struct F3DFar {
-  // pairs per group and reciprocals per pair
-  static constexpr int G = (MASK == OUT_VEL) ? 4 : 2;
-  static constexpr int U = G >= T ? G / T : 1;  // filaments per group
-  static constexpr int NP = U * T;              // pairs per group
-  static constexpr int NR = (MASK & OUT_DVORT) ? 2 : 1;
-  static constexpr int N = NP * NR;             // values per shared reciprocal
+  static constexpr int U = T >= 2 ? 1 : 2;  // filaments per group
+  static constexpr int NP = U * T;          // pairs per group
 };
 
-// Waves per SIMD the register allocation must leave room for.  The fused
-// kernel with one target per lane is held to 5 (at most 96 VGPRs; it takes
-// 103 and 4 waves unbounded, and spills 16 bytes held to 5): 16384
-// filaments x 2^20 targets, 21.29 -> 19.69 ms.  The velocity alone is held
-// to 6 (80 VGPRs instead of 89; 20 bytes spilled outside the source loops):
-// 10.37 -> 10.20 ms (three A/B pairs on one box); held to 7 it was slower.
-// The stretching alone runs best unbounded (5 waves; 17.24 ms against 17.73
-// held to 6).
+// Waves per SIMD the register allocation must leave room for: the fused
+// kernel with one target per lane is held to 5 (96 VGPRs; held to 4 it takes
+// 15.25 ms against 14.98), the velocity to 6 (5, 7 and 8: 9.09, 9.10, 9.17
+// ms against 9.04); the stretching takes 93 and 5 waves unbounded.
 template <int MASK, int T>
 constexpr int f3d_min_waves() {
   if constexpr (T != 1) return 1;
@@ -163,6 +169,7 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
   __shared__ float4 s_a[WG];
   __shared__ float4 s_b[WG];
   __shared__ float4 s_r0[WG];
+  __shared__ unsigned long long s_link[WAVES];
   __shared__ BoxPartials<3, WAVES> s_box;
   const int tid = threadIdx.x;
   const int base = blockIdx.x * (WG * T);
@@ -210,16 +217,16 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
     __syncthreads();
     {
       float4 a = make_float4(0.f, 0.f, 0.f, 0.f), b = a;
+      // link: this filament ends where the next one of the tile starts,
+      // bit for bit (a polyline), so the two can share that point's
+      // distance terms in the far loop
+      int link = 0;
       if (tid < cnt) {
         a = p.fa[ts + tid];
         b = p.fb[ts + tid];
         const float rx = b.x - a.x, ry = b.y - a.y, rz = b.z - a.z;
         const float g = a.w * k4pi;
-        const float len = __builtin_sqrtf(rx * rx + ry * ry + rz * rz);
-        // link: this filament ends where the next one of the tile starts,
-        // bit for bit (a polyline), so the two can share that point's
-        // distance terms in the far loop
-        int link = 0;
+        const float l2 = rx * rx + ry * ry + rz * rz;
         if (tid + 1 < cnt) {
           const float4 an = p.fa[ts + tid + 1];
           link = (int)(__float_as_uint(an.x) == __float_as_uint(b.x)) &
@@ -227,9 +234,11 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
                  (int)(__float_as_uint(an.z) == __float_as_uint(b.z));
         }
         s_a[tid] = make_float4(a.x, a.y, a.z, g);
-        s_b[tid] = make_float4(b.x, b.y, b.z, 3.f * g / len);
-        s_r0[tid] = make_float4(rx, ry, rz, __int_as_float(link));
+        s_b[tid] = make_float4(b.x, b.y, b.z, -6.f * g / __builtin_sqrtf(l2));
+        s_r0[tid] = make_float4(rx, ry, rz, 0.5f * l2);
       }
+      const unsigned long long links = __ballot(link != 0);
+      if ((tid & 63) == 0) s_link[tid >> 6] = links;
       // the tile's box holds both ends of every filament; extra: the
       // longest filament's squared length
       const float l3[3] = {fminf(a.x, b.x), fminf(a.y, b.y), fminf(a.z, b.z)};
@@ -261,15 +270,18 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
     const float c126 = in_vgpr(0x1p126f);
     float l2max;
     const Box<3> fbox = box_combine<3, WAVES>(s_box, &l2max);
-    // every pair same-side and finite, and each of the N values that share
-    // a reciprocal (P + r1.r2 in [dmin^2, 2 dmax^2], |r1| + |r2| in
-    // [2 dmin, 2 dmax]) within 2^(+-120/N), so their products stay normal
+    // every pair same-side and finite, and the product of the NP values that
+    // share a reciprocal normal: h is in [dmin^2, 2 dmax^2], S, by which the
+    // stretching multiplies it, in [2 dmin, 2 dmax], so the product of two
+    // S h or of four h is within 2^(+-124) in the wide range, that of four
+    // S h in the narrow one
     bool far = false;
     if (tbox.finite && fbox.finite) {
       float dmin2, dmax2;
       box_dist2<3>(tbox, fbox, dmin2, dmax2);
-      const float lo_ok = FF::N <= 4 ? 9.3e-10f : 3.1e-5f;   // 2^-30, 2^-15
-      const float hi_ok = FF::N <= 4 ? 5.3e8f : 1.6e4f;      // 2^29, 2^14
+      constexpr bool few = FF::NP <= 2 || (MASK & OUT_DVORT) == 0;
+      const float lo_ok = few ? 9.3e-10f : 3.1e-5f;   // 2^-30, 2^-15
+      const float hi_ok = few ? 5.3e8f : 1.6e4f;      // 2^29, 2^14
       far = dmin2 >= 0.2501f * l2max && dmin2 >= lo_ok && dmax2 <= hi_ok;
     }
     if (far) {
@@ -277,16 +289,18 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
       int j = 0;
       // the last end point of a group, kept for the next group when the
       // chain runs on into it (its first filament starts there, bit for bit,
-      // so the values are those the next group would compute).  With the
-      // stretching (two filaments per group) this saves a quarter of the end
-      // points' rsq: lattice dvort 18.67 -> 17.94 ms, fused 19.74 -> 19.22;
-      // both paths leave the point, which keeps the register allocator from
-      // copying it around the branch (dvort 18.07 -> 17.23, fused 19.14 ->
-      // 18.62), and then the velocity alone (four filaments per group, a
-      // fifth of its rsq saved) gains too: 10.87 -> 10.58 ms.
-      float lpx[T], lpy[T], lpz[T], lpns[T], lpy1[T];
+      // so the values are those the next group would compute): a third of the
+      // end points of a chain's groups of two.  Both paths leave the point,
+      // which keeps the register allocator from copying it around the branch.
+      float lpx[T], lpy[T], lpz[T], lpn[T], lpy1[T];
       bool carry = false;
+      unsigned long long links = 0;
       for (; j + U <= cnt; j += U, jv += U) {
+        if ((j & 63) == 0) {
+          const unsigned long long m = s_link[j >> 6];
+          links = ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(m >> 32)) << 32) |
+                  (unsigned)__builtin_amdgcn_readfirstlane((int)m);
+        }
         float4 fa[U], fb[U], f0[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -294,40 +308,36 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
           fb[u] = s_b[jv + u];
           f0[u] = s_r0[jv + u];
         }
-        float cx[FF::NP], cy[FF::NP], cz[FF::NP], ys[FF::NP], y12[FF::NP], p12[FF::NP],
-            cn[FF::NP], den[FF::N], inv[FF::N];
-        // the terms of pair q (filament u, target k) from r1 = x - a,
-        // r2 = x - b, their squared norms and reciprocal norms
-        auto terms = [&](int q, int u, float r1x, float r1y, float r1z, float r2x, float r2y,
-                         float r2z, float n1s, float n2s, float y1, float y2) {
-          cx[q] = __builtin_fmaf(r1y, r2z, -r1z * r2y);
-          cy[q] = __builtin_fmaf(r1z, r2x, -r1x * r2z);
-          cz[q] = __builtin_fmaf(r1x, r2y, -r1y * r2x);
-          const float n1 = n1s * y1, n2 = n2s * y2;
-          const float d12 = __builtin_fmaf(r1x, r2x, __builtin_fmaf(r1y, r2y, r1z * r2z));
-          ys[q] = y1 + y2;
-          den[q] = __builtin_fmaf(n1, n2, d12);  // P + r1.r2
+        float cx[FF::NP], cy[FF::NP], cz[FF::NP], ys[FF::NP], S2[FF::NP], p12[FF::NP],
+            cn[FF::NP], den[FF::NP], X[FF::NP], inv[FF::NP];
+        // the terms of pair q (filament u) from r1 = x - a, the norms of r1
+        // and r2 and their reciprocals
+        auto terms = [&](int q, int u, float r1x, float r1y, float r1z, float n1, float n2,
+                         float y1, float y2) {
+          cx[q] = __builtin_fmaf(f0[u].y, r1z, -f0[u].z * r1y);
+          cy[q] = __builtin_fmaf(f0[u].z, r1x, -f0[u].x * r1z);
+          cz[q] = __builtin_fmaf(f0[u].x, r1y, -f0[u].y * r1x);
+          const float S = n1 + n2;
+          S2[q] = S * S;
+          den[q] = __builtin_fmaf(0.5f, S2[q], -f0[u].w);  // |r1||r2| + r1.r2
           if constexpr ((MASK & OUT_DVORT) != 0) {
-            y12[q] = y1 * y2;
-            den[FF::NP + q] = n1 + n2;
+            ys[q] = y1 * y2;
+            X[q] = S * den[q];
             const float cc = __builtin_fmaf(cx[q], cx[q], __builtin_fmaf(cy[q], cy[q], cz[q] * cz[q]));
             cn[q] = __builtin_amdgcn_sqrtf(cc);
-            p12[q] = __builtin_fmaf(f0[u].x, r1x + r2x,
-                                    __builtin_fmaf(f0[u].y, r1y + r2y, f0[u].z * (r1z + r2z)));
+            // r0.(r1 + r2) / 2
+            p12[q] = __builtin_fmaf(f0[u].x, r1x, __builtin_fmaf(f0[u].y, r1y,
+                                                                 __builtin_fmaf(f0[u].z, r1z, -f0[u].w)));
+          } else {
+            ys[q] = y1 + y2;
+            X[q] = den[q];
           }
         };
         // a chained group (each filament ends where the next begins) has
         // U + 1 distinct end points: each point's distance and rsq serve
-        // the two filaments that meet there (same formulas as below).
-        // Lattice of 16384 filaments in chains of 128 x 2^20 targets:
-        // vel 13.22 -> 10.65 ms, dvort 19.23 -> 18.67, fused 20.41 -> 19.69
-        bool chained = false;
-        if constexpr (U > 1) {
-          int f = __float_as_int(f0[0].w);
-#pragma unroll
-          for (int u = 1; u + 1 < U; ++u) f &= __float_as_int(f0[u].w);
-          chained = __builtin_amdgcn_readfirstlane(f) != 0;
-        }
+        // the two filaments that meet there (same formulas as below)
+        constexpr unsigned in_group = (1u << (U - 1)) - 1u;
+        const bool chained = U > 1 && ((unsigned)links & in_group) == in_group;
         if (chained) {
           if (!carry) {
 #pragma unroll
@@ -335,26 +345,27 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
               lpx[k] = xt[k].x - fa[0].x;
               lpy[k] = xt[k].y - fa[0].y;
               lpz[k] = xt[k].z - fa[0].z;
-              lpns[k] = __builtin_fmaf(lpx[k], lpx[k], __builtin_fmaf(lpy[k], lpy[k], lpz[k] * lpz[k]));
-              lpy1[k] = __builtin_amdgcn_rsqf(lpns[k]);
+              const float ns = __builtin_fmaf(lpx[k], lpx[k], __builtin_fmaf(lpy[k], lpy[k], lpz[k] * lpz[k]));
+              lpy1[k] = __builtin_amdgcn_rsqf(ns);
+              lpn[k] = ns * lpy1[k];
             }
           }
 #pragma unroll
           for (int k = 0; k < T; ++k) {
             // walk the points: each filament's terms as soon as its end is known
-            float px = lpx[k], py = lpy[k], pz = lpz[k], pns = lpns[k], py1 = lpy1[k];
+            float px = lpx[k], py = lpy[k], pz = lpz[k], pn = lpn[k], py1 = lpy1[k];
 #pragma unroll
             for (int u = 0; u < U; ++u) {
               const float4 pt = u + 1 < U ? fa[u + 1] : fb[U - 1];
               const float qx = xt[k].x - pt.x, qy = xt[k].y - pt.y, qz = xt[k].z - pt.z;
               const float qns = __builtin_fmaf(qx, qx, __builtin_fmaf(qy, qy, qz * qz));
               const float qy1 = __builtin_amdgcn_rsqf(qns);
-              terms(u * T + k, u, px, py, pz, qx, qy, qz, pns, qns, py1, qy1);
-              px = qx; py = qy; pz = qz; pns = qns; py1 = qy1;
+              const float qn = qns * qy1;
+              terms(u * T + k, u, px, py, pz, pn, qn, py1, qy1);
+              px = qx; py = qy; pz = qz; pn = qn; py1 = qy1;
             }
-            lpx[k] = px; lpy[k] = py; lpz[k] = pz; lpns[k] = pns; lpy1[k] = py1;
+            lpx[k] = px; lpy[k] = py; lpz[k] = pz; lpn[k] = pn; lpy1[k] = py1;
           }
-          carry = __builtin_amdgcn_readfirstlane(__float_as_int(f0[U - 1].w)) != 0;
         } else {
 #pragma unroll
           for (int u = 0; u < U; ++u)
@@ -364,37 +375,43 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
               const float r2x = xt[k].x - fb[u].x, r2y = xt[k].y - fb[u].y, r2z = xt[k].z - fb[u].z;
               const float n1s = __builtin_fmaf(r1x, r1x, __builtin_fmaf(r1y, r1y, r1z * r1z));
               const float n2s = __builtin_fmaf(r2x, r2x, __builtin_fmaf(r2y, r2y, r2z * r2z));
-              const float y2 = __builtin_amdgcn_rsqf(n2s);
-              terms(u * T + k, u, r1x, r1y, r1z, r2x, r2y, r2z, n1s, n2s,
-                    __builtin_amdgcn_rsqf(n1s), y2);
+              const float y1 = __builtin_amdgcn_rsqf(n1s), y2 = __builtin_amdgcn_rsqf(n2s);
+              const float n2 = n2s * y2;
+              terms(u * T + k, u, r1x, r1y, r1z, n1s * y1, n2, y1, y2);
               if (u == U - 1) {
                 // the group's last end point, as the chained walk leaves it
-                lpx[k] = r2x; lpy[k] = r2y; lpz[k] = r2z; lpns[k] = n2s; lpy1[k] = y2;
+                lpx[k] = r2x; lpy[k] = r2y; lpz[k] = r2z; lpn[k] = n2; lpy1[k] = y2;
               }
             }
-          carry = __builtin_amdgcn_readfirstlane(__float_as_int(f0[U - 1].w)) != 0;
         }
-        batch_rcp<FF::N>(den, inv);
+        carry = (links >> (U - 1)) & 1;
+        links >>= U;
+        batch_rcp<FF::NP>(X, inv);
 #pragma unroll
         for (int u = 0; u < U; ++u)
 #pragma unroll
           for (int k = 0; k < T; ++k) {
             const int q = u * T + k;
-            const float kk = fa[u].w * ys[q] * inv[q];
+            float kk;
+            if constexpr ((MASK & OUT_DVORT) != 0) {
+              const float z = ys[q] * inv[q];  // y1 y2 / (S (P + r1.r2))
+              kk = fa[u].w * S2[q] * z;
+              acc[k][D + 0] = __builtin_fmaf(fb[u].w, cn[q] * p12[q] * (den[q] * z), acc[k][D + 0]);
+            } else {
+              kk = fa[u].w * ys[q] * inv[q];
+            }
             if constexpr ((MASK & OUT_VEL) != 0) {
               acc[k][0] = __builtin_fmaf(kk, cx[q], acc[k][0]);
               acc[k][1] = __builtin_fmaf(kk, cy[q], acc[k][1]);
               acc[k][2] = __builtin_fmaf(kk, cz[q], acc[k][2]);
             }
             if constexpr ((MASK & OUT_DVORT) != 0) {
-              const float B = -fb[u].w * cn[q] * p12[q] * y12[q] * inv[FF::NP + q];
               // kk, or 0 when c = 0: |c| is 0 or at least 2^-75 (the root
               // of a float), so |c| 2^126 clamped to [0, 1] is 0 or 1 (one
               // multiplication with the clamp modifier, where a compare does
               // not dual-issue): lattice fused 19.18 -> 19.03 ms
               // (kk is finite in far tiles, so kk * 0 is 0)
               const float kd = kk * __builtin_amdgcn_fmed3f(cn[q] * c126, 0.f, 1.f);
-              acc[k][D + 0] += B;
               acc[k][D + 1] = __builtin_fmaf(kd, f0[u].x, acc[k][D + 1]);
               acc[k][D + 2] = __builtin_fmaf(kd, f0[u].y, acc[k][D + 2]);
               acc[k][D + 3] = __builtin_fmaf(kd, f0[u].z, acc[k][D + 3]);
