@@ -529,22 +529,22 @@ F3Fn f3_reduce(int mask) {
 //   k = (Gamma/4pi) (y1 + y2) / (|r1||r2| + r1.r2) = (Gamma/2pi) S y1 y2 / (S^2 - L^2)
 // needs neither r1.r2 nor |c|^2 nor the selects, and c = r0 x r1 (r0 = b - a,
 // kept in registers) is, away from the segment, the better conditioned
-// product.  S^2 - L^2 loses at most one bit there.  S is at least twice the
-// distance D of the point from the filament, so D^2 >= L^2 / 2 is enough, and
-// a wave decides it for its 64 NF filaments and all its rows at once: lane l
-// compares row l's distance from the box around the wave's filaments with
-// their longest, and a ballot gives one bit per row (a test per element
-// instead: 222 against 217 us on the matrix below).  Where the filaments of
+// product.  S^2 - L^2 loses at most one bit there.  A row for which any lane
+// of the wave fails the test (or has a NaN) is computed again by the general
+// form.  (One test per wave and row against the box around the wave's
+// filaments, decided for all rows by one ballot, gave 217 us instead of 222
+// on the matrix below, but its wave reductions cost every workgroup more than
+// a small matrix's rows: 1786 x 2069 8.4 -> 11.9 us.)  Where the filaments of
 // every lane of the wave form a polyline (each starts, bit for bit, where the
 // previous one ends, as the spanwise segments of a vortex lattice do), a
 // shared end point's distance terms are computed once per row.
 //
 // What bounds it: the matrix's write and the vector units about equally.  For
-// 16384 x 16384 (1 GiB) the kernel takes 217-225 us, 4.8-4.9 TB/s of writes
-// (294 us before: every element by the general form, two columns per lane,
-// points in SGPRs); with the element arithmetic left out it takes 167 us
-// with 8 rows per workgroup and 213 with 32.  127 x 130 columns 322 -> 260
-// us, 127 x 129 318 -> 262 us.
+// 16384 x 16384 (1 GiB) the kernel takes 222 us, 4.8 TB/s of writes (294 us
+// before: every element by the general form, two columns per lane, points in
+// SGPRs); with the element arithmetic left out it takes 167 us with 8 rows
+// per workgroup and 213 with 32.  16383 x 16384 320 -> 263 us, 4096 x 4096
+// 23.4 -> 19.3, 3280 x 1149 10.3 -> 8.6, 923 x 18510 26.6 -> 25.0.
 template <int NF>
 struct InfCols {
   float3 a[NF], b[NF], r0[NF];
@@ -588,8 +588,7 @@ constexpr int INF_ROWS = 32;  // rows a workgroup stages at most
 // (STREAM: past the caches).
 template <int NF, bool SHARE, bool WHOLE, bool STREAM>
 __device__ __forceinline__ void inf_rows(const InfCols<NF>& c, const float4* s_x, const float4* s_e,
-                                         unsigned long long far_rows, int nr, int j0, int n_fil,
-                                         float* __restrict__ o) {
+                                         int nr, int j0, int n_fil, float* __restrict__ o) {
   using Vec = float __attribute__((ext_vector_type(NF)));
   using Vec4 = float __attribute__((ext_vector_type(NF), aligned(4)));  // any float's address
   int iv = in_vgpr(0);
@@ -603,29 +602,30 @@ __device__ __forceinline__ void inf_rows(const InfCols<NF>& c, const float4* s_x
     xn = s_x[iv];
     en = s_e[iv];
     Vec v;
-    if ((far_rows >> i) & 1) {
-      float3 r2;
-      float y2, n2;
+    bool far = true;
+    float3 r2;
+    float y2, n2;
 #pragma unroll
-      for (int f = 0; f < NF; ++f) {
-        float3 r1 = r2;
-        float y1 = y2, n1 = n2;
-        if (f == 0 || !SHARE) {
-          r1 = sub3(x, c.a[f]);
-          const float ns = dot3(r1, r1);
-          y1 = __builtin_amdgcn_rsqf(ns);
-          n1 = ns * y1;
-        }
-        r2 = sub3(x, c.b[f]);
-        const float ns = dot3(r2, r2);
-        y2 = __builtin_amdgcn_rsqf(ns);
-        n2 = ns * y2;
-        const float S = n1 + n2;
-        const float den = __builtin_fmaf(S, S, -c.L2[f]);
-        const float ce = dot3(cross3(c.r0[f], r1), e);
-        v[f] = ((c.g[f] * (S * y1)) * y2) * (ce * __builtin_amdgcn_rcpf(den));
+    for (int f = 0; f < NF; ++f) {
+      float3 r1 = r2;
+      float y1 = y2, n1 = n2;
+      if (f == 0 || !SHARE) {
+        r1 = sub3(x, c.a[f]);
+        const float ns = dot3(r1, r1);
+        y1 = __builtin_amdgcn_rsqf(ns);
+        n1 = ns * y1;
       }
-    } else {
+      r2 = sub3(x, c.b[f]);
+      const float ns = dot3(r2, r2);
+      y2 = __builtin_amdgcn_rsqf(ns);
+      n2 = ns * y2;
+      const float S = n1 + n2;
+      const float den = __builtin_fmaf(S, S, -c.L2[f]);
+      far = far && den >= c.L2[f];
+      const float ce = dot3(cross3(c.r0[f], r1), e);
+      v[f] = ((c.g[f] * (S * y1)) * y2) * (ce * __builtin_amdgcn_rcpf(den));
+    }
+    if (!__all(far)) {
 #pragma unroll
       for (int f = 0; f < NF; ++f) v[f] = inf_general(sub3(x, c.a[f]), sub3(x, c.b[f]), 0.5f * c.g[f], e);
     }
@@ -677,43 +677,12 @@ __global__ __launch_bounds__(256) void f3d_inf_kernel(const float4* __restrict__
   float* o = out + (size_t)i0 * (size_t)n_fil;
   // one answer for the whole wave, so the row loop branches uniformly
   const bool share = __all(linked);
-  // bit i: row i is far from all the wave's filaments (see above), and every
-  // distance is finite and normal
-  Box<3> wb;
-  float l2 = 0.f;
-  wb.finite = true;
-#pragma unroll
-  for (int d = 0; d < 3; ++d) { wb.lo[d] = __builtin_inff(); wb.hi[d] = -__builtin_inff(); }
-#pragma unroll
-  for (int f = 0; f < NF; ++f) {
-    const float pa[3] = {c.a[f].x, c.a[f].y, c.a[f].z}, pb[3] = {c.b[f].x, c.b[f].y, c.b[f].z};
-#pragma unroll
-    for (int d = 0; d < 3; ++d) {
-      wb.lo[d] = fminf(wb.lo[d], fminf(pa[d], pb[d]));
-      wb.hi[d] = fmaxf(wb.hi[d], fmaxf(pa[d], pb[d]));
-      wb.finite = wb.finite && __builtin_isfinite(pa[d]) && __builtin_isfinite(pb[d]);
-    }
-    wb.finite = wb.finite && __builtin_isfinite(c.g[f]);
-    l2 = fmaxf(l2, c.L2[f]);
-  }
-#pragma unroll
-  for (int d = 0; d < 3; ++d) { wb.lo[d] = wave_min(wb.lo[d]); wb.hi[d] = wave_max(wb.hi[d]); }
-  l2 = wave_max(l2);
-  wb.finite = __all(wb.finite);
-  const float4 xr = s_x[min(tid & 63, nr)];  // (slot nr is zero)
-  Box<3> pb;
-  pb.lo[0] = pb.hi[0] = xr.x; pb.lo[1] = pb.hi[1] = xr.y; pb.lo[2] = pb.hi[2] = xr.z;
-  float dmin2, dmax2;
-  box_dist2<3>(wb, pb, dmin2, dmax2);
-  const bool fin = __builtin_isfinite(xr.x) && __builtin_isfinite(xr.y) && __builtin_isfinite(xr.z);
-  const unsigned long long far_rows =
-      __ballot(fin && wb.finite && dmin2 >= 0.51f * l2 && dmin2 >= 1e-30f && dmax2 <= 1e30f);
   if (whole) {
-    if (share) inf_rows<NF, true, true, STREAM>(c, s_x, s_e, far_rows, nr, j0, n_fil, o);
-    else inf_rows<NF, false, true, STREAM>(c, s_x, s_e, far_rows, nr, j0, n_fil, o);
+    if (share) inf_rows<NF, true, true, STREAM>(c, s_x, s_e, nr, j0, n_fil, o);
+    else inf_rows<NF, false, true, STREAM>(c, s_x, s_e, nr, j0, n_fil, o);
   } else {
-    if (share) inf_rows<NF, true, false, STREAM>(c, s_x, s_e, far_rows, nr, j0, n_fil, o);
-    else inf_rows<NF, false, false, STREAM>(c, s_x, s_e, far_rows, nr, j0, n_fil, o);
+    if (share) inf_rows<NF, true, false, STREAM>(c, s_x, s_e, nr, j0, n_fil, o);
+    else inf_rows<NF, false, false, STREAM>(c, s_x, s_e, nr, j0, n_fil, o);
   }
 }
 
@@ -731,11 +700,12 @@ hipError_t launch_f3d_inf(const float4* fa, const float4* fb, int n_fil, const f
   const bool stream = n_fil % 32 == 0 && ((uintptr_t)out & 127) == 0 &&
                       (size_t)n_fil * n_mes >= (size_t)INF_STREAM_ELEMENTS;
   const int per = 256 * (stream ? 4 : 2);
-  // rows per workgroup: two workgroups per CU at least, so that each has rows
-  // to spread its prologue over (3280 x 1149: 22 us with 16 per CU, 9.9 with 2)
+  // rows per workgroup: eight workgroups per CU at least (3280 x 1149, us with
+  // 2 / 4 / 8 / 16 per CU: 8.5 / 8.3 / 8.6 / 10.7; 923 x 18510: 25.6 / 25.9 /
+  // 25.0 / 24.0; 1786 x 2069: 9.9 / 8.8 / 8.4 / 8.4)
   const int gx = (n_fil + per - 1) / per;
   int rows = 1;
-  while (rows < INF_ROWS && (long long)gx * ((n_mes + 2 * rows - 1) / (2 * rows)) >= 512) rows *= 2;
+  while (rows < INF_ROWS && (long long)gx * ((n_mes + 2 * rows - 1) / (2 * rows)) >= 2048) rows *= 2;
   const auto k = stream ? f3d_inf_kernel<4, true> : f3d_inf_kernel<2, false>;
   hipLaunchKernelGGL(k, dim3(gx, (n_mes + rows - 1) / rows), dim3(256), 0, s, fa, fb, n_fil, mes,
                      dir, n_mes, rows, out);
