@@ -47,6 +47,7 @@ struct RegConsts {
   float c2;        // gaussian: sqrt(2/pi)
   float q_far = 208.f;  // gaussian: rho^2 beyond which exp(-rho^2/2) is 0 in FP32
   float q_tab = (float)(GTAB_RHO_MAX * GTAB_RHO_MAX);  // gaussian: table range in rho^2
+  float xs = 1.f;  // 3D winckelmans: power of two that positions are multiplied by
 };
 
 // A uniform value that a pair loop reads on every pair, held in a VGPR.  On
@@ -108,7 +109,7 @@ __device__ __forceinline__ void two_sum_add(float& hi, float& lo, float x) {
 }
 
 // ---- regularisation kernels (reduced form) -------------------------------
-// eval<SELF>(r2, K, lds_table, Kv, Kh, eta)
+// eval<SELF>(r2, K, lds_table, Kv, Kh, eta) (Winckelmans: see there)
 //   Kv: velocity / stretching kernel, zero when r2 == 0 (self and
 //       coincident pairs are excluded, reference src/P3D.cpp:58,94,127)
 //   Kh: gradient kernel; Kh * 0 must be 0 when r2 == 0
@@ -139,30 +140,25 @@ struct RegKernel<REG_SINGULAR> {
 
 template <>
 struct RegKernel<REG_WINCKELMANS> {
-  // Reduced units (q = rho^2, s = q + 1, y = s^-1/2); the epilogue applies
-  // |sigma|^-3 to Kv, 3 |sigma|^-5 to Kh and 52.5 to eta:
-  //   Kv  = G(rho)     = (q + 2.5) y^5
-  //   Kh  = H(rho) / 3 = (q + 3.5) y^7
+  // Positions come multiplied by a power of two (RegConsts::xs, exact) that
+  // puts sigma in [1, 2), so that S = r^2 + sigma^2 can be formed in three
+  // multiply-adds started from sigma^2 (rather than r^2 and then r^2/sigma^2
+  // + 1) and its powers stay in range.  With y = S^-1/2, in those units:
+  //   Kv  = (r^2 + 2.5 sigma^2) y^5 = y^3 (1 + 1.5 sigma^2 y^2)
+  //   Kh  = (r^2 + 3.5 sigma^2) y^7 = (Kv + sigma^2 y^5) y^2
   //   eta = y^9
-  template <bool SELF = true>
-  static __device__ __forceinline__ void eval(float r2, const RegConsts& k, const float4*,
-                                              float& Kv, float& Kh, float& eta) {
-    float s = __builtin_fmaf(r2, k.inv_s2, 1.f);
-    float y = __builtin_amdgcn_rsqf(s);
-    float y2 = y * y;
-    float y3 = y2 * y;
-    float y5 = y3 * y2;
-    float kv = (s + 1.5f) * y5;
-    Kh = (kv + y5) * y2;  // (s + 2.5) y^7 from Kv: two operations instead of three
-    float e = (y5 * y2) * y2;
-    if constexpr (SELF) {
-      bool z = (r2 == 0.f);
-      Kv = z ? 0.f : kv;
-      eta = z ? 0.f : e;
-    } else {
-      Kv = kv;
-      eta = e;
-    }
+  // (x 3 and x 52.5 sigma^9 in the epilogue).  None is zero at r = 0: the
+  // caller drops coincident pairs where that matters.  k: s2 = sigma^2, c1 =
+  // 1.5 sigma^2.
+  static __device__ __forceinline__ void eval(float S, const RegConsts& k, float& Kv, float& Kh,
+                                              float& eta) {
+    const float y = __builtin_amdgcn_rsqf(S);
+    const float y2 = y * y;
+    const float y3 = y2 * y;
+    Kv = y3 * __builtin_fmaf(k.c1, y2, 1.f);
+    const float y5 = y3 * y2;
+    Kh = __builtin_fmaf(k.s2, y5, Kv) * y2;
+    eta = (y5 * y2) * y2;
   }
 };
 

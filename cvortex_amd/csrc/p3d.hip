@@ -96,6 +96,14 @@ bool p3d_supported(int reg, int mask) {
   return true;
 }
 
+// Winckelmans: the exponent e for which sigma 2^e is in [1, 2) (0 for a radius
+// that is zero, infinite or NaN).
+static int winckelmans_exponent(float sigma) {
+  const double s = std::fabs((double)sigma);
+  if (!(s > 0.0) || !std::isfinite(s)) return 0;
+  return std::min(126, std::max(-126, -std::ilogb(s)));
+}
+
 RegConsts p3d_consts(int reg, float sigma) {
   RegConsts k{};
   const double s = std::fabs((double)sigma);
@@ -104,6 +112,15 @@ RegConsts p3d_consts(int reg, float sigma) {
   if (reg == REG_GAUSSIAN) {
     k.c1 = (float)(-0.5 / std::log(2.0));
     k.c2 = (float)std::sqrt(2.0 / M_PI);
+  }
+  if (reg == REG_WINCKELMANS) {
+    k.xs = (float)std::ldexp(1.0, winckelmans_exponent(sigma));
+    const double t = s * (double)k.xs;
+    // no field of a radius that is no length: 0 and NaN give NaN; an infinite
+    // one is scaled by 0 below
+    const double t2 = std::isinf(s) ? 1.0 : (s == 0.0 ? std::nan("") : t * t);
+    k.s2 = (float)t2;
+    k.c1 = (float)(1.5 * t2);
   }
   return k;
 }
@@ -121,12 +138,17 @@ Scales p3d_scales(int reg, float sigma, float nu) {
       sc.dH = 3.0 * sgn * k4pi / s5;
       sc.visc = 2.0 * (double)nu / (s * s);
       break;
-    case REG_WINCKELMANS:
-      sc.vel = -k4pi / s3;
-      sc.dG = sgn * k4pi / s3;
-      sc.dH = 3.0 * sgn * k4pi / s5;
-      sc.visc = 2.0 * (double)nu / (s * s) * 52.5;
+    case REG_WINCKELMANS: {
+      // in positions multiplied by x: Kv is x^-3 of the dimensional one, each
+      // position factor x
+      const double x = std::ldexp(1.0, winckelmans_exponent(sigma)), t = s * x;
+      const double on = std::isinf(s) ? 0.0 : 1.0;
+      sc.vel = -k4pi * x * x * on;
+      sc.dG = sgn * k4pi * x * x * x * on;
+      sc.dH = 3.0 * sc.dG;
+      sc.visc = std::isinf(s) ? 0.0 : 2.0 * (double)nu / (s * s) * 52.5 * std::pow(t, 9);
       break;
+    }
     case REG_PLANETARY:
       sc.vel = -k4pi / s3;
       sc.dG = sgn * k4pi / s3;

@@ -68,18 +68,35 @@ struct P3DKParams {
   Scales sc;
 };
 
-template <int REG, int MASK, int ACC>
+// How a Winckelmans pair with equal coordinates is dropped (the other
+// regularisations test r^2 == 0 in their own kernels).  SELF_NONE: it need
+// not be, the velocity term being Kv (d x a_s) with d = 0.  SELF_TEST: a
+// compare per pair.  SELF_WATCH: only the smallest S = r^2 + sigma^2 of the
+// tile is kept, a third as many instructions; where it is sigma^2 the caller
+// repeats the tile with SELF_TEST (see p3d_block).
+enum SelfMode : int { SELF_NONE, SELF_TEST, SELF_WATCH };
+
+template <int REG, int MASK, int ACC, int SELF>
 __device__ __forceinline__ void p3d_pair(const float4 sp, const float4 sa, const double2* pxy,
                                          const double2* pzv, const float3 xt, const float3 at,
                                          const RegConsts& rc, const float4* tab, float* acc,
-                                         double* dacc) {
+                                         double* dacc, float& smin) {
   using R = P3DRegs<REG, MASK, ACC>;
   const float dx = xt.x - sp.x;
   const float dy = xt.y - sp.y;
   const float dz = xt.z - sp.z;
-  const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, dz * dz));
+  const float r2 = __builtin_fmaf(
+      dx, dx, __builtin_fmaf(dy, dy, REG == REG_WINCKELMANS ? __builtin_fmaf(dz, dz, rc.s2) : dz * dz));
   float Kv, Kh, eta, Kfar = 0.f;
-  if constexpr (R::SPLIT && (MASK & OUT_DVORT) != 0) {
+  if constexpr (REG == REG_WINCKELMANS) {
+    RegKernel<REG_WINCKELMANS>::eval(r2, rc, Kv, Kh, eta);
+    if constexpr (SELF == SELF_WATCH) smin = fminf(smin, r2);
+    if constexpr (SELF == SELF_TEST) {
+      const bool same = (__float_as_uint(dx) | __float_as_uint(dy) | __float_as_uint(dz)) == 0u;
+      Kv = same ? 0.f : Kv;
+      eta = same ? 0.f : eta;
+    }
+  } else if constexpr (R::SPLIT && (MASK & OUT_DVORT) != 0) {
     RegKernel<REG_GAUSSIAN>::eval_split(r2, rc, tab, Kv, Kh, eta,
                                         [&](float kn, float en) {
       const double2 sxy = *pxy, szv = *pzv;
@@ -239,7 +256,8 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
     i = i < tgt_end ? i : tgt_end - 1;
     if (p.tgt_perm) i = p.tgt_perm[i];
     const float4 q = p.tgt_pv[i];
-    xt[k] = make_float3(q.x, q.y, q.z);
+    xt[k] = REG == REG_WINCKELMANS ? make_float3(q.x * rc.xs, q.y * rc.xs, q.z * rc.xs)
+                                   : make_float3(q.x, q.y, q.z);
     vt[k] = q.w;
     if constexpr (L::NEED_TA) {
       const float4 w = p.tgt_a[i];
@@ -266,8 +284,13 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
     const int cnt = min(WG, s1 - ts);
     __syncthreads();
     if (tid < cnt) {
-      const float4 q = p.src_pv[ts + tid];
+      float4 q = p.src_pv[ts + tid];
       const float4 w = p.src_a[ts + tid];
+      if constexpr (REG == REG_WINCKELMANS) {
+        q.x *= rc.xs;
+        q.y *= rc.xs;
+        q.z *= rc.xs;
+      }
       sm.xa[tid] = make_float4(q.x, q.y, q.z, w.x);
       if constexpr (P3DSmem<REG, MASK, ACC, WG>::VOL)
         sm.tl[tid] = make_float4(w.y, w.z, q.w, 0.f);
@@ -279,15 +302,6 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
       }
     }
     __syncthreads();
-    if constexpr (ACC != ACC_PLAIN) {
-#pragma unroll
-      for (int k = 0; k < T; ++k)
-#pragma unroll
-        for (int a = 0; a < NF; ++a) acc[k][a] = 0.f;
-    }
-    // the LDS index runs in a VGPR too: an SGPR index would cost an
-    // SGPR-reading move per source to form the ds_read address
-    int jv = in_vgpr(0);
     // two sources per iteration, except around the velocity-only Gaussian's
     // pinned near-range branch, which cannot be unrolled, and four for the
     // short velocity-only pair with one target per lane (uniform cube of
@@ -296,18 +310,58 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
     constexpr int kUnroll = (R::SPLIT && (MASK & (OUT_DVORT | OUT_VISC)) == 0)
                                 ? 1
                                 : ((MASK == OUT_VEL && T == 1) ? 4 : 2);
+    float smin = __builtin_inff();
+    auto tile = [&](auto mode) {
+      if constexpr (ACC != ACC_PLAIN) {
+#pragma unroll
+        for (int k = 0; k < T; ++k)
+#pragma unroll
+          for (int a = 0; a < NF; ++a) acc[k][a] = 0.f;
+      }
+      // the LDS index runs in a VGPR too: an SGPR index would cost an
+      // SGPR-reading move per source to form the ds_read address
+      int jv = in_vgpr(0);
 #pragma unroll kUnroll
-    for (int j = 0; j < cnt; ++j, ++jv) {
-      const float4 xa = sm.xa[jv];
-      const auto tl = sm.tl[jv];
-      float vol = 0.f;
-      if constexpr (P3DSmem<REG, MASK, ACC, WG>::VOL) vol = tl.z;
-      const float4 sp = make_float4(xa.x, xa.y, xa.z, vol);
-      const float4 sa = make_float4(xa.w, tl.x, tl.y, 0.f);
+      for (int j = 0; j < cnt; ++j, ++jv) {
+        const float4 xa = sm.xa[jv];
+        const auto tl = sm.tl[jv];
+        float vol = 0.f;
+        if constexpr (P3DSmem<REG, MASK, ACC, WG>::VOL) vol = tl.z;
+        const float4 sp = make_float4(xa.x, xa.y, xa.z, vol);
+        const float4 sa = make_float4(xa.w, tl.x, tl.y, 0.f);
+#pragma unroll
+        for (int k = 0; k < T; ++k)
+          p3d_pair<REG, MASK, ACC, decltype(mode)::value>(sp, sa, &sm.xy[DBL_ ? jv : 0],
+                                                          &sm.zv[DBL_ ? jv : 0], xt[k], at[k], rv,
+                                                          sm.tab, acc[k], dacc[k], smin);
+      }
+    };
+    // Winckelmans with stretching or viscous terms: a target meets itself (or
+    // another particle at its place) in one tile of many, so the tile's sums
+    // are formed without a test and formed again with it only where some
+    // pair's S was sigma^2 (r below 2^-12 sigma).  Both give the same value
+    // for every other pair.  One FP32 running sum cannot be taken back.
+    // With S formed from sigma^2 (RegKernel) 36 issue slots per pair instead
+    // of 41, ms: 128 clouds, tile-compensated 51.1 -> 46.6; 64 clouds, FP64
+    // stretching 32.1 -> 30.8; 400000 particles with the viscous term 147.4 ->
+    // 141.0; velocity of 100000 (S alone) 4.38 -> 4.06.
+    constexpr bool WATCH = REG == REG_WINCKELMANS && ACC != ACC_PLAIN && (MASK & (OUT_DVORT | OUT_VISC)) != 0;
+    if constexpr (WATCH) {
+      double before[T][ND];
 #pragma unroll
       for (int k = 0; k < T; ++k)
-        p3d_pair<REG, MASK, ACC>(sp, sa, &sm.xy[DBL_ ? jv : 0], &sm.zv[DBL_ ? jv : 0], xt[k], at[k],
-                                 rv, sm.tab, acc[k], dacc[k]);
+#pragma unroll
+        for (int a = 0; a < ND; ++a) before[k][a] = dacc[k][a];
+      tile(std::integral_constant<int, SELF_WATCH>());
+      if (__any(smin <= rc.s2)) {
+#pragma unroll
+        for (int k = 0; k < T; ++k)
+#pragma unroll
+          for (int a = 0; a < ND; ++a) dacc[k][a] = before[k][a];
+        tile(std::integral_constant<int, SELF_TEST>());
+      }
+    } else {
+      tile(std::integral_constant<int, MASK == OUT_VEL ? SELF_NONE : SELF_TEST>());
     }
     if constexpr (ACC != ACC_PLAIN) {
 #pragma unroll
