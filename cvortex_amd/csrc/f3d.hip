@@ -160,8 +160,12 @@ constexpr int f3d_min_waves() {
   return MASK == (OUT_VEL | OUT_DVORT) ? 5 : (MASK == OUT_VEL ? 6 : 1);
 }
 
-template <int MASK, int ACC, int T, int WG>
+// Q > 1 (T = 1): 64 targets per workgroup, the same in all Q waves, each of
+// which takes 1/Q of every tile's filaments; their FP64 sums are added at the
+// end (see narrow_cfg).
+template <int MASK, int ACC, int T, int WG, int Q = 1>
 __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3DKParams p) {
+  static_assert(Q == 1 || (T == 1 && WG == 64 * Q), "a group of shared targets is one wave wide");
   constexpr int NA = ((MASK & OUT_VEL) ? 3 : 0) + ((MASK & OUT_DVORT) ? 4 : 0);
   constexpr int D = (MASK & OUT_VEL) ? 3 : 0;
   constexpr int WAVES = WG / 64;
@@ -171,12 +175,15 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
   __shared__ float4 s_r0[WG];
   __shared__ unsigned long long s_link[WAVES];
   __shared__ BoxPartials<3, WAVES> s_box;
+  __shared__ double s_share[Q > 1 ? Q - 1 : 1][Q > 1 ? NA : 1][64];
   const int tid = threadIdx.x;
-  const int base = blockIdx.x * (WG * T);
+  const int tl = Q == 1 ? tid : tid & 63;               // target within the group
+  const int part = Q == 1 ? 0 : (tid >> 6) * (WG / Q);  // first filament of this wave's part
+  const int base = blockIdx.x * (WG * T / Q);
   float3 xt[T], at[T];
 #pragma unroll
   for (int k = 0; k < T; ++k) {
-    int i = base + k * WG + tid;
+    int i = base + k * WG + tl;
     i = i < p.n_tgt ? i : p.n_tgt - 1;
     if (p.tgt_perm) i = p.tgt_perm[i];
     const float4 q = p.tgt_pv[i];
@@ -257,7 +264,8 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
 #pragma unroll
         for (int a = 0; a < NA; ++a) acc[k][a] = 0.f;
     }
-    int jv = in_vgpr(0);  // LDS index in a VGPR (no SGPR operand per filament)
+    int jv = in_vgpr(part);  // LDS index in a VGPR (no SGPR operand per filament)
+    const int end = Q == 1 ? cnt : min(cnt, part + WG / Q);
     // velocity only: +inf in a VGPR, so |kk| < fin is a VGPR compare (against
     // the literal the compiler emits a class test whose mask operand is an
     // SGPR).  Measured on 16384 filaments x 2^20 targets: vel 16.79 -> 16.54
@@ -286,7 +294,7 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
     }
     if (far) {
       constexpr int U = FF::U;
-      int j = 0;
+      int j = part;
       // the last end point of a group, kept for the next group when the
       // chain runs on into it (its first filament starts there, bit for bit,
       // so the values are those the next group would compute): a third of the
@@ -295,7 +303,7 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
       float lpx[T], lpy[T], lpz[T], lpn[T], lpy1[T];
       bool carry = false;
       unsigned long long links = 0;
-      for (; j + U <= cnt; j += U, jv += U) {
+      for (; j + U <= end; j += U, jv += U) {
         if ((j & 63) == 0) {
           const unsigned long long m = s_link[j >> 6];
           links = ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(m >> 32)) << 32) |
@@ -418,14 +426,14 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
             }
           }
       }
-      for (; j < cnt; ++j, ++jv) {
+      for (; j < end; ++j, ++jv) {
         const float4 fa = s_a[jv], fb = s_b[jv], f0 = s_r0[jv];
 #pragma unroll
         for (int k = 0; k < T; ++k) f3d_pair<MASK>(fa, fb, f0, xt[k], fin, acc[k]);
       }
     } else {
 #pragma unroll 2
-      for (int j = 0; j < cnt; ++j, ++jv) {
+      for (int j = part; j < end; ++j, ++jv) {
         const float4 fa = s_a[jv];
         const float4 fb = s_b[jv];
         const float4 f0 = s_r0[jv];
@@ -443,12 +451,25 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
 
 #pragma unroll
   for (int k = 0; k < T; ++k) {
-    const int i = base + k * WG + tid;
-    if (i >= p.n_tgt) continue;
+    const int i = base + k * WG + tl;
+    if (Q == 1 && i >= p.n_tgt) continue;
     double d[NA];
 #pragma unroll
     for (int a = 0; a < NA; ++a)
       d[a] = (ACC == ACC_COMP) ? (double)hi[k][a] + (double)lo[k][a] : (double)acc[k][a];
+    if constexpr (Q > 1) {
+      const int w = tid >> 6;
+      if (w > 0) {
+#pragma unroll
+        for (int a = 0; a < NA; ++a) s_share[w - 1][a][tl] = d[a];
+      }
+      __syncthreads();
+      if (w > 0 || i >= p.n_tgt) return;
+#pragma unroll
+      for (int v = 0; v < Q - 1; ++v)
+#pragma unroll
+        for (int a = 0; a < NA; ++a) d[a] += s_share[v][a][tl];
+    }
     if (p.n_split == 1) {
       f3d_finish<MASK>(d, at[k], p, p.tgt_perm ? p.tgt_perm[i] : i);
     } else {
@@ -487,7 +508,8 @@ size_t f3d_workspace_bytes(const F3DJob& j, const LaunchCfg& c) {
 namespace {
 using F3Fn = void (*)(F3DKParams);
 template <int MASK, int ACC>
-F3Fn f3_T(int T) {
+F3Fn f3_T(int T, int q) {
+  if (q == 4) return T == 1 ? f3d_kernel<MASK, ACC, 1, 256, 4> : nullptr;
   switch (T) {
     case 1: return f3d_kernel<MASK, ACC, 1, 256>;
     case 4: return f3d_kernel<MASK, ACC, 4, 256>;
@@ -495,14 +517,14 @@ F3Fn f3_T(int T) {
   }
 }
 template <int MASK>
-F3Fn f3_acc(int acc, int T) {
-  return acc == ACC_PLAIN ? f3_T<MASK, ACC_PLAIN>(T) : f3_T<MASK, ACC_COMP>(T);
+F3Fn f3_acc(int acc, int T, int q) {
+  return acc == ACC_PLAIN ? f3_T<MASK, ACC_PLAIN>(T, q) : f3_T<MASK, ACC_COMP>(T, q);
 }
-F3Fn f3_pick(int mask, int acc, int T) {
+F3Fn f3_pick(int mask, int acc, int T, int q) {
   switch (mask) {
-    case OUT_VEL: return f3_acc<OUT_VEL>(acc, T);
-    case OUT_DVORT: return f3_acc<OUT_DVORT>(acc, T);
-    case OUT_VEL | OUT_DVORT: return f3_acc<OUT_VEL | OUT_DVORT>(acc, T);
+    case OUT_VEL: return f3_acc<OUT_VEL>(acc, T, q);
+    case OUT_DVORT: return f3_acc<OUT_DVORT>(acc, T, q);
+    case OUT_VEL | OUT_DVORT: return f3_acc<OUT_VEL | OUT_DVORT>(acc, T, q);
     default: return nullptr;
   }
 }
@@ -720,7 +742,7 @@ hipError_t launch_f3d(const F3DJob& j, const LaunchCfg& c, hipStream_t s) {
   if (((j.mask & OUT_VEL) && !j.out_vel) || ((j.mask & OUT_DVORT) && !j.out_dvort) || !j.tgt_pv ||
       (j.n_fil > 0 && (!j.fa || !j.fb)))
     return hipErrorInvalidValue;
-  F3Fn k = f3_pick(j.mask, j.acc, c.T);
+  F3Fn k = f3_pick(j.mask, j.acc, c.T, c.q);
   if (!k) return hipErrorInvalidValue;
   F3DKParams p{};
   p.fa = j.fa;
@@ -743,7 +765,7 @@ hipError_t launch_f3d(const F3DJob& j, const LaunchCfg& c, hipStream_t s) {
   }
   p.n_split = n_split;
   p.split_len = split_len;
-  const int per = c.wg * c.T;
+  const int per = c.wg * c.T / c.q;
   hipLaunchKernelGGL(k, dim3((j.n_tgt + per - 1) / per, n_split), dim3(c.wg), 0, s, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || n_split == 1) return e;

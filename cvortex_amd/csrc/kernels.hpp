@@ -22,6 +22,9 @@ struct LaunchCfg {
   int wg = 256;       // workgroup size (= source tile length); 256 only for now
   int n_split = 1;    // number of source partitions (each a grid row)
   int split_len = 0;  // sources per partition, a multiple of wg
+  // waves that share a group of 64 targets, each taking its part of every
+  // source tile (1: every wave has targets of its own; 4: T = 1 only)
+  int q = 1;
 };
 
 // FP64 epilogue scale factors.

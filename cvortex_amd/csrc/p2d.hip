@@ -151,8 +151,12 @@ struct P2DFar {
   }
 };
 
-template <int REG, int MASK, int ACC, int T, int WG>
+// Q > 1 (T = 1): 64 targets per workgroup, the same in all Q waves, each of
+// which takes 1/Q of every tile's sources; their FP64 sums are added at the
+// end (see narrow_cfg).
+template <int REG, int MASK, int ACC, int T, int WG, int Q = 1>
 __global__ __launch_bounds__(WG) void p2d_kernel(P2DKParams p) {
+  static_assert(Q == 1 || (T == 1 && WG == 64 * Q), "a group of shared targets is one wave wide");
   constexpr int NA = ((MASK & OUT_VEL) ? 2 : 0) + ((MASK & OUT_VISC) ? 1 : 0);
   constexpr int E = (MASK & OUT_VEL) ? 2 : 0;
   constexpr bool CULL = P2DFar<REG>::ENABLED && (MASK & OUT_VEL) != 0;
@@ -161,12 +165,15 @@ __global__ __launch_bounds__(WG) void p2d_kernel(P2DKParams p) {
   constexpr int WAVES = WG / 64;
   __shared__ float4 s_src[WG];
   __shared__ BoxPartials<2, WAVES> s_box;
+  __shared__ double s_share[Q > 1 ? Q - 1 : 1][Q > 1 ? NA : 1][64];
   const int tid = threadIdx.x;
-  const int base = blockIdx.x * (WG * T);
+  const int tl = Q == 1 ? tid : tid & 63;               // target within the group
+  const int part = Q == 1 ? 0 : (tid >> 6) * (WG / Q);  // first source of this wave's part
+  const int base = blockIdx.x * (WG * T / Q);
   float4 xt[T];
 #pragma unroll
   for (int k = 0; k < T; ++k) {
-    int i = base + k * WG + tid;
+    int i = base + k * WG + tl;
     i = i < p.n_tgt ? i : p.n_tgt - 1;
     xt[k] = p.tgt[i];
   }
@@ -220,7 +227,8 @@ __global__ __launch_bounds__(WG) void p2d_kernel(P2DKParams p) {
 #pragma unroll
         for (int a = 0; a < NA; ++a) acc[k][a] = 0.f;
     }
-    int jv = in_vgpr(0);  // LDS index in a VGPR (no SGPR operand per source)
+    int jv = in_vgpr(part);  // LDS index in a VGPR (no SGPR operand per source)
+    const int end = Q == 1 ? cnt : min(cnt, part + WG / Q);
     bool far = false;
     if constexpr (CULL) far = boxes_far<2>(tbox, box_combine<2, WAVES>(s_box), P2DFar<REG>::near2(p.rc));
     if (far) {
@@ -233,8 +241,8 @@ __global__ __launch_bounds__(WG) void p2d_kernel(P2DKParams p) {
           if constexpr (REG == REG_PLANETARY) return a;
           else return a * ks;
         };
-        int j = 0;
-        for (; j + U <= cnt; j += U, jv += U) {
+        int j = part;
+        for (; j + U <= end; j += U, jv += U) {
           float4 s[U];
 #pragma unroll
           for (int u = 0; u < U; ++u) s[u] = s_src[jv + u];
@@ -265,7 +273,7 @@ __global__ __launch_bounds__(WG) void p2d_kernel(P2DKParams p) {
             acc[k][1] = __builtin_fmaf(K[q], dx[q], acc[k][1]);
           }
         }
-        for (; j < cnt; ++j, ++jv) {
+        for (; j < end; ++j, ++jv) {
           const float4 s = s_src[jv];
           const float as = sk(s.z);
 #pragma unroll
@@ -282,7 +290,7 @@ __global__ __launch_bounds__(WG) void p2d_kernel(P2DKParams p) {
       // (the Gaussian's pinned branch cannot be unrolled around)
       constexpr int kUnroll = REG == REG_GAUSSIAN ? 1 : 4;
 #pragma unroll kUnroll
-      for (int j = 0; j < cnt; ++j, ++jv) {
+      for (int j = part; j < end; ++j, ++jv) {
         const float4 s = s_src[jv];
 #pragma unroll
         for (int k = 0; k < T; ++k) {
@@ -316,13 +324,26 @@ __global__ __launch_bounds__(WG) void p2d_kernel(P2DKParams p) {
 
 #pragma unroll
   for (int k = 0; k < T; ++k) {
-    const int i = base + k * WG + tid;
-    if (i >= p.n_tgt) continue;
+    const int i = base + k * WG + tl;
+    if (Q == 1 && i >= p.n_tgt) continue;
     double d[NA];
 #pragma unroll
     for (int a = 0; a < NA; ++a)
       d[a] = TS ? (double)hi[k][a] + (double)lo[k][a] : (double)acc[k][a];
     if constexpr (V64) d[E] = vacc[k];
+    if constexpr (Q > 1) {
+      const int w = tid >> 6;
+      if (w > 0) {
+#pragma unroll
+        for (int a = 0; a < NA; ++a) s_share[w - 1][a][tl] = d[a];
+      }
+      __syncthreads();
+      if (w > 0 || i >= p.n_tgt) return;
+#pragma unroll
+      for (int v = 0; v < Q - 1; ++v)
+#pragma unroll
+        for (int a = 0; a < NA; ++a) d[a] += s_share[v][a][tl];
+    }
     if (p.n_split == 1) {
       p2d_finish<MASK>(d, p, i);
     } else {
@@ -363,7 +384,8 @@ namespace {
 using K2Fn = void (*)(P2DKParams);
 
 template <int REG, int MASK, int ACC>
-K2Fn p2_T(int T) {
+K2Fn p2_T(int T, int q) {
+  if (q == 4) return T == 1 ? p2d_kernel<REG, MASK, ACC, 1, 256, 4> : nullptr;
   switch (T) {
     case 1: return p2d_kernel<REG, MASK, ACC, 1, 256>;
     case 4: return p2d_kernel<REG, MASK, ACC, 4, 256>;
@@ -372,31 +394,31 @@ K2Fn p2_T(int T) {
 }
 // ACC_TILES differs from ACC_COMP only in the viscous exchange's sum
 template <int REG, int MASK>
-K2Fn p2_acc(int acc, int T) {
-  if (acc == ACC_PLAIN) return p2_T<REG, MASK, ACC_PLAIN>(T);
+K2Fn p2_acc(int acc, int T, int q) {
+  if (acc == ACC_PLAIN) return p2_T<REG, MASK, ACC_PLAIN>(T, q);
   if constexpr ((MASK & OUT_VISC) != 0)
-    if (acc == ACC_TILES) return p2_T<REG, MASK, ACC_TILES>(T);
-  return p2_T<REG, MASK, ACC_COMP>(T);
+    if (acc == ACC_TILES) return p2_T<REG, MASK, ACC_TILES>(T, q);
+  return p2_T<REG, MASK, ACC_COMP>(T, q);
 }
 template <int REG>
-K2Fn p2_mask_inviscid(int mask, int acc, int T) {
-  return mask == OUT_VEL ? p2_acc<REG, OUT_VEL>(acc, T) : nullptr;
+K2Fn p2_mask_inviscid(int mask, int acc, int T, int q) {
+  return mask == OUT_VEL ? p2_acc<REG, OUT_VEL>(acc, T, q) : nullptr;
 }
 template <int REG>
-K2Fn p2_mask_viscous(int mask, int acc, int T) {
+K2Fn p2_mask_viscous(int mask, int acc, int T, int q) {
   switch (mask) {
-    case OUT_VEL: return p2_acc<REG, OUT_VEL>(acc, T);
-    case OUT_VISC: return p2_acc<REG, OUT_VISC>(acc, T);
-    case OUT_VEL | OUT_VISC: return p2_acc<REG, OUT_VEL | OUT_VISC>(acc, T);
+    case OUT_VEL: return p2_acc<REG, OUT_VEL>(acc, T, q);
+    case OUT_VISC: return p2_acc<REG, OUT_VISC>(acc, T, q);
+    case OUT_VEL | OUT_VISC: return p2_acc<REG, OUT_VEL | OUT_VISC>(acc, T, q);
     default: return nullptr;
   }
 }
-K2Fn p2_pick(int reg, int mask, int acc, int T) {
+K2Fn p2_pick(int reg, int mask, int acc, int T, int q) {
   switch (reg) {
-    case REG_SINGULAR: return p2_mask_inviscid<REG_SINGULAR>(mask, acc, T);
-    case REG_PLANETARY: return p2_mask_inviscid<REG_PLANETARY>(mask, acc, T);
-    case REG_WINCKELMANS: return p2_mask_viscous<REG_WINCKELMANS>(mask, acc, T);
-    case REG_GAUSSIAN: return p2_mask_viscous<REG_GAUSSIAN>(mask, acc, T);
+    case REG_SINGULAR: return p2_mask_inviscid<REG_SINGULAR>(mask, acc, T, q);
+    case REG_PLANETARY: return p2_mask_inviscid<REG_PLANETARY>(mask, acc, T, q);
+    case REG_WINCKELMANS: return p2_mask_viscous<REG_WINCKELMANS>(mask, acc, T, q);
+    case REG_GAUSSIAN: return p2_mask_viscous<REG_GAUSSIAN>(mask, acc, T, q);
     default: return nullptr;
   }
 }
@@ -417,7 +439,7 @@ hipError_t launch_p2d(const P2DJob& j, const LaunchCfg& c, hipStream_t s) {
   if (((j.mask & OUT_VEL) && !j.out_vel) || ((j.mask & OUT_VISC) && !j.out_visc) || !j.tgt ||
       (j.n_src > 0 && !j.src))
     return hipErrorInvalidValue;
-  K2Fn k = p2_pick(j.reg, j.mask, j.acc, c.T);
+  K2Fn k = p2_pick(j.reg, j.mask, j.acc, c.T, c.q);
   if (!k) return hipErrorInvalidValue;
   P2DKParams p{};
   p.src = j.src;
@@ -460,7 +482,7 @@ hipError_t launch_p2d(const P2DJob& j, const LaunchCfg& c, hipStream_t s) {
   }
   p.n_split = n_split;
   p.split_len = split_len;
-  const int per = c.wg * c.T;
+  const int per = c.wg * c.T / c.q;
   hipLaunchKernelGGL(k, dim3((j.n_tgt + per - 1) / per, n_split), dim3(c.wg), 0, s, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || n_split == 1) return e;

@@ -32,16 +32,17 @@ int p3d_nacc(int mask) {
   return ((mask & OUT_VEL) ? 3 : 0) + ((mask & OUT_DVORT) ? 6 : 0) + ((mask & OUT_VISC) ? 4 : 0);
 }
 
-template <int REG, int MASK, int ACC, int T, int WG>
+template <int REG, int MASK, int ACC, int T, int WG, int Q = 1>
 __global__ __launch_bounds__(WG) void p3d_kernel(P3DKParams p) {
   __shared__ P3DSmem<REG, MASK, ACC, WG> sm;
+  __shared__ P3DShare<MASK, Q> share;
   if constexpr (REG == REG_GAUSSIAN) {
     for (int i = threadIdx.x; i < 2 * GTAB_N; i += WG) sm.tab[i] = p.gtab[i];
   }
   const int s0 = blockIdx.y * p.split_len;
   const int s1 = min(s0 + p.split_len, p.n_src);
-  p3d_block<REG, MASK, ACC, T, WG>(p, p.rc, p.sc, blockIdx.x * (WG * T), p.n_tgt, s0, s1,
-                                   blockIdx.y, sm);
+  p3d_block<REG, MASK, ACC, T, WG, Q>(p, p.rc, p.sc, blockIdx.x * (WG * T / Q), p.n_tgt, s0, s1,
+                                      blockIdx.y, sm, &share);
 }
 
 template <int MASK>
@@ -173,7 +174,8 @@ namespace {
 using KernelFn = void (*)(P3DKParams);
 
 template <int REG, int MASK, int ACC>
-KernelFn pick_T(int T) {
+KernelFn pick_T(int T, int q) {
+  if (q == 4) return T == 1 ? p3d_kernel<REG, MASK, ACC, 1, 256, 4> : nullptr;
   switch (T) {
     case 1: return p3d_kernel<REG, MASK, ACC, 1, 256>;
     case 4: return p3d_kernel<REG, MASK, ACC, 4, 256>;
@@ -182,41 +184,41 @@ KernelFn pick_T(int T) {
 }
 
 template <int REG, int MASK>
-KernelFn pick_acc(int acc, int T) {
-  if (acc == ACC_PLAIN) return pick_T<REG, MASK, ACC_PLAIN>(T);
-  if (acc == ACC_TILES) return pick_T<REG, MASK, ACC_TILES>(T);
-  return pick_T<REG, MASK, ACC_COMP>(T);
+KernelFn pick_acc(int acc, int T, int q) {
+  if (acc == ACC_PLAIN) return pick_T<REG, MASK, ACC_PLAIN>(T, q);
+  if (acc == ACC_TILES) return pick_T<REG, MASK, ACC_TILES>(T, q);
+  return pick_T<REG, MASK, ACC_COMP>(T, q);
 }
 
 template <int REG>
-KernelFn pick_mask_inviscid(int mask, int acc, int T) {
+KernelFn pick_mask_inviscid(int mask, int acc, int T, int q) {
   switch (mask) {
-    case OUT_VEL: return pick_acc<REG, OUT_VEL>(acc, T);
-    case OUT_DVORT: return pick_acc<REG, OUT_DVORT>(acc, T);
-    case OUT_VEL | OUT_DVORT: return pick_acc<REG, OUT_VEL | OUT_DVORT>(acc, T);
+    case OUT_VEL: return pick_acc<REG, OUT_VEL>(acc, T, q);
+    case OUT_DVORT: return pick_acc<REG, OUT_DVORT>(acc, T, q);
+    case OUT_VEL | OUT_DVORT: return pick_acc<REG, OUT_VEL | OUT_DVORT>(acc, T, q);
     default: return nullptr;
   }
 }
 
 template <int REG>
-KernelFn pick_mask_viscous(int mask, int acc, int T) {
+KernelFn pick_mask_viscous(int mask, int acc, int T, int q) {
   switch (mask) {
-    case OUT_VEL: return pick_acc<REG, OUT_VEL>(acc, T);
-    case OUT_DVORT: return pick_acc<REG, OUT_DVORT>(acc, T);
-    case OUT_VISC: return pick_acc<REG, OUT_VISC>(acc, T);
-    case OUT_VEL | OUT_DVORT: return pick_acc<REG, OUT_VEL | OUT_DVORT>(acc, T);
-    case OUT_DVORT | OUT_VISC: return pick_acc<REG, OUT_DVORT | OUT_VISC>(acc, T);
-    case OUT_VEL | OUT_DVORT | OUT_VISC: return pick_acc<REG, OUT_VEL | OUT_DVORT | OUT_VISC>(acc, T);
+    case OUT_VEL: return pick_acc<REG, OUT_VEL>(acc, T, q);
+    case OUT_DVORT: return pick_acc<REG, OUT_DVORT>(acc, T, q);
+    case OUT_VISC: return pick_acc<REG, OUT_VISC>(acc, T, q);
+    case OUT_VEL | OUT_DVORT: return pick_acc<REG, OUT_VEL | OUT_DVORT>(acc, T, q);
+    case OUT_DVORT | OUT_VISC: return pick_acc<REG, OUT_DVORT | OUT_VISC>(acc, T, q);
+    case OUT_VEL | OUT_DVORT | OUT_VISC: return pick_acc<REG, OUT_VEL | OUT_DVORT | OUT_VISC>(acc, T, q);
     default: return nullptr;
   }
 }
 
-KernelFn pick_kernel(int reg, int mask, int acc, int T) {
+KernelFn pick_kernel(int reg, int mask, int acc, int T, int q) {
   switch (reg) {
-    case REG_SINGULAR: return pick_mask_inviscid<REG_SINGULAR>(mask, acc, T);
-    case REG_PLANETARY: return pick_mask_inviscid<REG_PLANETARY>(mask, acc, T);
-    case REG_WINCKELMANS: return pick_mask_viscous<REG_WINCKELMANS>(mask, acc, T);
-    case REG_GAUSSIAN: return pick_mask_viscous<REG_GAUSSIAN>(mask, acc, T);
+    case REG_SINGULAR: return pick_mask_inviscid<REG_SINGULAR>(mask, acc, T, q);
+    case REG_PLANETARY: return pick_mask_inviscid<REG_PLANETARY>(mask, acc, T, q);
+    case REG_WINCKELMANS: return pick_mask_viscous<REG_WINCKELMANS>(mask, acc, T, q);
+    case REG_GAUSSIAN: return pick_mask_viscous<REG_GAUSSIAN>(mask, acc, T, q);
     default: return nullptr;
   }
 }
@@ -244,7 +246,7 @@ hipError_t launch_p3d(const P3DJob& j, const LaunchCfg& c, hipStream_t s) {
   if (((j.mask & OUT_VEL) && !j.out_vel) || ((j.mask & OUT_DVORT) && !j.out_dvort) ||
       ((j.mask & OUT_VISC) && !j.out_visc) || !j.tgt_pv || (j.n_src > 0 && (!j.src_pv || !j.src_a)))
     return hipErrorInvalidValue;
-  KernelFn k = pick_kernel(j.reg, j.mask, j.acc, c.T);
+  KernelFn k = pick_kernel(j.reg, j.mask, j.acc, c.T, c.q);
   if (!k) return hipErrorInvalidValue;
 
   P3DKParams p{};
@@ -276,7 +278,7 @@ hipError_t launch_p3d(const P3DJob& j, const LaunchCfg& c, hipStream_t s) {
   p.n_split = n_split;
   p.split_len = split_len;
 
-  const int tgt_per_block = c.wg * c.T;
+  const int tgt_per_block = c.wg * c.T / c.q;
   dim3 grid((j.n_tgt + tgt_per_block - 1) / tgt_per_block, n_split);
   hipLaunchKernelGGL(k, grid, dim3(c.wg), 0, s, p);
   hipError_t e = hipGetLastError();

@@ -234,25 +234,38 @@ struct P3DSmem {
   float4 tab[REG == REG_GAUSSIAN ? 2 * GTAB_N : 1];
 };
 
+// FP64 sums of the waves that share targets (Q > 1), one set per wave but the
+// first.
+template <int MASK, int Q>
+struct P3DShare {
+  double d[Q > 1 ? Q - 1 : 1][Q > 1 ? P3DLayout<MASK>::N : 1][64];
+};
+
 // One workgroup: targets base + k*WG + lane (k < T) that are < tgt_end,
-// against sources [s0, s1).  Writes the outputs (n_split == 1) or the FP64
-// partials of partition `split`.  The caller has loaded sm.tab (Gaussian)
+// against sources [s0, s1).  Q > 1 (T = 1): targets base + lane of 64, the
+// same in all Q waves, each of which takes 1/Q of every tile's sources; their
+// sums are added in FP64 at the end (see narrow_cfg).  Writes the outputs
+// (n_split == 1) or the FP64 partials of partition `split`.  The caller has loaded sm.tab (Gaussian)
 // and issues no barrier-sensitive work on sm around the call.
-template <int REG, int MASK, int ACC, int T, int WG>
+template <int REG, int MASK, int ACC, int T, int WG, int Q = 1>
 __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& rc,
                                           const Scales& sc, int base, int tgt_end, int s0,
-                                          int s1, int split, P3DSmem<REG, MASK, ACC, WG>& sm) {
+                                          int s1, int split, P3DSmem<REG, MASK, ACC, WG>& sm,
+                                          P3DShare<MASK, Q>* share = nullptr) {
+  static_assert(Q == 1 || (T == 1 && WG == 64 * Q), "a group of shared targets is one wave wide");
   using L = P3DLayout<MASK>;
   using R = P3DRegs<REG, MASK, ACC>;
   constexpr int NF = R::NF;
   constexpr int ND = R::ND > 0 ? R::ND : 1;
   constexpr bool DBL_ = P3DSmem<REG, MASK, ACC, WG>::DBL;
   const int tid = threadIdx.x;
+  const int tl = Q == 1 ? tid : tid & 63;  // target within the group
+  const int part = Q == 1 ? 0 : (tid >> 6) * (WG / Q);  // first source of this wave's part
   float3 xt[T], at[T];
   float vt[T];
 #pragma unroll
   for (int k = 0; k < T; ++k) {
-    int i = base + k * WG + tid;
+    int i = base + k * WG + tl;
     i = i < tgt_end ? i : tgt_end - 1;
     if (p.tgt_perm) i = p.tgt_perm[i];
     const float4 q = p.tgt_pv[i];
@@ -320,9 +333,10 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
       }
       // the LDS index runs in a VGPR too: an SGPR index would cost an
       // SGPR-reading move per source to form the ds_read address
-      int jv = in_vgpr(0);
+      int jv = in_vgpr(part);
+      const int end = Q == 1 ? cnt : min(cnt, part + WG / Q);
 #pragma unroll kUnroll
-      for (int j = 0; j < cnt; ++j, ++jv) {
+      for (int j = part; j < end; ++j, ++jv) {
         const float4 xa = sm.xa[jv];
         const auto tl = sm.tl[jv];
         float vol = 0.f;
@@ -341,11 +355,13 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
     // are formed without a test and formed again with it only where some
     // pair's S was sigma^2 (r below 2^-12 sigma).  Both give the same value
     // for every other pair.  One FP32 running sum cannot be taken back.
+    // With Q > 1 the partitions are of a few tiles, and it tests each pair
+    // (4000 particles, vel + dvort, 31.0 -> 26.0 us).
     // With S formed from sigma^2 (RegKernel) 36 issue slots per pair instead
     // of 41, ms: 128 clouds, tile-compensated 51.1 -> 46.6; 64 clouds, FP64
     // stretching 32.1 -> 30.8; 400000 particles with the viscous term 147.4 ->
     // 141.0; velocity of 100000 (S alone) 4.38 -> 4.06.
-    constexpr bool WATCH = REG == REG_WINCKELMANS && ACC != ACC_PLAIN && (MASK & (OUT_DVORT | OUT_VISC)) != 0;
+    constexpr bool WATCH = Q == 1 && REG == REG_WINCKELMANS && ACC != ACC_PLAIN && (MASK & (OUT_DVORT | OUT_VISC)) != 0;
     if constexpr (WATCH) {
       double before[T][ND];
 #pragma unroll
@@ -373,8 +389,8 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
 
 #pragma unroll
   for (int k = 0; k < T; ++k) {
-    const int i = base + k * WG + tid;
-    if (i >= tgt_end) continue;
+    const int i = base + k * WG + tl;
+    if (Q == 1 && i >= tgt_end) continue;
     // gather the canonical layout
     double d[L::N];
     auto fval = [&](int a) -> double {
@@ -397,6 +413,19 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
     if constexpr ((MASK & OUT_VISC) != 0) {
 #pragma unroll
       for (int c = 0; c < 4; ++c) d[L::E + c] = R::DBL ? dacc[k][R::D_E + c] : fval(R::F_E + c);
+    }
+    if constexpr (Q > 1) {
+      const int w = tid >> 6;
+      if (w > 0) {
+#pragma unroll
+        for (int a = 0; a < L::N; ++a) share->d[w - 1][a][tl] = d[a];
+      }
+      __syncthreads();
+      if (w > 0 || i >= tgt_end) return;
+#pragma unroll
+      for (int v = 0; v < Q - 1; ++v)
+#pragma unroll
+        for (int a = 0; a < L::N; ++a) d[a] += share->d[v][a][tl];
     }
     if (p.n_split == 1) {
       p3d_finish<MASK>(d, at[k], vt[k], sc, p.out_vel, p.out_dvort, p.out_visc,

@@ -80,6 +80,46 @@ int ordered_kind(int kind, int reg, int n_src, int n_tgt) {
   return ordered ? kind + 16 : kind;
 }
 
+namespace {
+
+// Small problems: 64 targets per workgroup, shared by its four waves, each of
+// which takes a quarter of every source tile.  Bound by the waves in flight
+// and by the length of the longest one: with 256 targets per workgroup a
+// problem of a few tiles leaves most SIMDs idle, and one a little larger ends
+// in a wave of workgroups that is nearly empty.  The price is one staging of
+// a tile and its barriers per 64 pairs of a lane instead of 256, so the rule
+// ends at 24 target-block tiles of 256 x 256 per CU.  256 targets per
+// workgroup -> 64, us: Winckelmans vel + dvort of 2000 particles 32.4 -> 13.7,
+// 6000 60.6 -> 48.2, 9000 99.7 -> 82.3, 15000 215 -> 191, 18000 289 -> 275;
+// velocity of 1000 on the host's arrays 43.7 -> 34.8 a call; 2D Gaussian with
+// the viscous term, 3000 51.0 -> 20.5, 9000 103 -> 65, 18000 229 -> 196;
+// 3600 filaments on 20000 targets 242 -> 167, 10000 on 30000 467 -> 418 (on
+// 100000, 60 tiles per CU, 1054 -> 1190: a block of 64 targets has a smaller
+// box than one of 256, but its tiles are staged four times as often).
+// 2D velocities by the singular or the planetary kernel take so few
+// operations per pair that the staging counts from 4 tiles per CU on
+// (planetary 3000 14.3 -> 11.3, 7900 27.9 -> 29.6, 12000 47.6 -> 55.9).
+bool narrow(int kind, int reg, int mask, int n_src, int n_tgt, int cus) {
+  const long long nb = ((long long)n_tgt + 255) / 256, tiles = ((long long)n_src + 255) / 256;
+  const bool light = kind == KIND_P2D && !(mask & OUT_VISC) &&
+                     (reg == REG_PLANETARY || reg == REG_SINGULAR);
+  return n_tgt > 0 && tiles > 0 && nb * tiles < (light ? 4LL : 24LL) * cus;
+}
+
+// Partitions for 16 workgroups per CU of two tiles or more each, and for 4 per
+// CU down to one tile: 8192 particles (velocity, us) 40.9 with two tiles each,
+// 44.2 with four; 7000 (vel + dvort) 54.2 with three, 57.0 with two.
+LaunchCfg narrow_cfg(int n_src, int n_tgt, int cus) {
+  const long long groups = ((long long)n_tgt + 63) / 64, tiles = ((long long)n_src + 255) / 256;
+  auto fill = [&](long long per_cu) { return std::max(1LL, (per_cu * cus + groups - 1) / groups); };
+  const long long k = std::min(std::max(fill(4), std::min(fill(16), tiles / 2)), tiles);
+  LaunchCfg c = launch_shape(1, (int)k, n_src);
+  c.q = 4;
+  return c;
+}
+
+}  // namespace
+
 LaunchCfg choose_cfg(int kind, int reg, int mask, int acc, int n_src, int n_tgt, int n_cu) {
   auto it = cache().find(Key{ordered_kind(kind, reg, n_src, n_tgt), reg, mask, acc,
                              size_bucket(n_src), size_bucket(n_tgt)});
@@ -120,6 +160,7 @@ LaunchCfg choose_cfg(int kind, int reg, int mask, int acc, int n_src, int n_tgt,
     if (k > tiles / 2 && blocks * (tiles / 2) >= 32LL * cus) k = tiles / 2;
     return launch_shape(T, (int)std::min<long long>(k, 1 << 20), n_src);
   }
+  if (narrow(kind, reg, mask, n_src, n_tgt, cus)) return narrow_cfg(n_src, n_tgt, cus);
   LaunchCfg c = default_cfg(n_src, n_tgt, n_cu);
   const bool many_blocks = (long long)(n_tgt + 255) / 256 >= 4LL * cus;
   // Filaments: one target per lane.  It fits in fewer VGPRs (more waves per
