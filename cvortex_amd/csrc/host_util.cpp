@@ -105,17 +105,29 @@ LaunchCfg partitioned_cfg(int T, int n_src, int n_tgt, int n_cu) {
   const long long tiles = ((long long)n_src + 255) / 256;
   if (nb <= 0 || tiles <= 0) return c;  // nothing to split (no targets or sources)
   // Source partitions, for two reasons:
-  //   * to fill the chip (4 workgroups per CU) when there are few target
-  //     blocks, down to one tile per partition;
+  //   * to fill the chip when there are few target blocks: 4 workgroups per
+  //     CU down to one tile per partition, 8 down to two, 32 down to three;
   //   * for an even finish: with uniform work per pair, a launch of ~16
   //     workgroups per CU still ends unevenly across the CUs, and ~64 per CU
-  //     does better.  Measured: 16384 filaments x 2^20 targets, vel
-  //     16.54 -> 16.12 ms (T=1, 4 partitions), vel+dvort 24.43 -> 23.61 ms
-  //     (T=2, 4); 2^22 P2D sheet 3577 -> 3501 ms (T=4, 4).  These
-  //     partitions keep at least 16 tiles each.
-  const long long fill = nb >= 4 * cus ? 1 : (4 * cus + nb - 1) / nb;
+  //     does better, while a partition keeps at least 6 tiles (its FP64
+  //     partial sums, written and read once, are then 2 % of its work).
+  // Against at least 16 tiles per partition and one at a fill of 4, us:
+  // Winckelmans vel + dvort of 40000 particles 1272 -> 1204, with the viscous
+  // term 30000 particles 941 -> 868; 2D Gaussian with the viscous term, 30000
+  // 748 -> 491, 100003 3635 -> 3337; about 10000 filaments on 60000 targets 958
+  // -> 735, on 400000 4184 -> 3756; no change for the velocity of
+  // 60000 particles (1434, 1438).  Without the line for 32 per CU, 26000
+  // particles 550 -> 579 and the filaments' velocity at 60000 targets 537 ->
+  // 614; at least 8 tiles and 4: 26000 particles 578, the rest the same.
   const long long even = nb >= 64 * cus ? 1 : (64 * cus + nb - 1) / nb;
-  long long k = std::max(fill, std::min(even, std::max(1LL, tiles / 16)));
+  long long k = std::min(even, std::max(1LL, tiles / 6));
+  auto at_least = [&](long long per_cu, long long keep) {
+    if (nb * k < per_cu * cus)
+      k = std::max(k, std::min((per_cu * cus + nb - 1) / nb, std::max(1LL, tiles / keep)));
+  };
+  at_least(32, 3);
+  at_least(8, 2);
+  at_least(4, 1);
   k = std::min(k, std::max(1LL, tiles));
   if (k <= 1) {
     c.n_split = 1;
