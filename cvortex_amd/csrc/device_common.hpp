@@ -297,4 +297,60 @@ struct RegKernel<REG_GAUSSIAN> {
   }
 };
 
+// Waves that share their targets (Q > 1): the part [wave_part, wave_part_end)
+// of a tile of cnt sources that a wave takes, a multiple of four long except
+// for the last (the loops are unrolled by two and four).  The bounds are scalar,
+// and so is the loop (bounds in VGPRs, us: 3D velocity of 10000 particles 51.5
+// -> 48.4, 3600 filaments on 20000 targets 161 -> 154, 2D Gaussian with the
+// viscous term 12000 100.4 -> 93.4).
+template <int Q>
+__device__ __forceinline__ int wave_part(int cnt, int tid) {
+  if constexpr (Q == 1) return 0;
+  const int w = __builtin_amdgcn_readfirstlane(tid >> 6);
+  return min(cnt, w * (((cnt + 4 * Q - 1) / (4 * Q)) * 4));
+}
+template <int Q>
+__device__ __forceinline__ int wave_part_end(int cnt, int part) {
+  if constexpr (Q == 1) return cnt;
+  return min(cnt, part + ((cnt + 4 * Q - 1) / (4 * Q)) * 4);
+}
+
+// The target whose partials a thread of a 256-thread reduction sums, and their
+// sum over the partitions in d; true where this thread holds the total.
+// ROWS = 1: 256 targets per workgroup.  ROWS = 4, for few targets, where the
+// loads' latency bounds it: 64 targets, wave w adding partitions w, w + 4, ...,
+// then the first wave the others' sums.  1 -> 4, us a call: Gaussian vel +
+// dvort + visc of 2000 particles 25.2 -> 21.4, Winckelmans vel + dvort of 5000
+// 37.7 -> 33.6; but 65536 Gaussian 2629 -> 2639 (reduce_rows).
+template <int NA, int ROWS>
+__device__ __forceinline__ bool sum_partitions(const double* __restrict__ partial, int n_split,
+                                               int n_tgt, int& i, double (&d)[NA]) {
+  __shared__ double share[ROWS > 1 ? ROWS - 1 : 1][ROWS > 1 ? NA : 1][64];
+  const int lane = threadIdx.x & 63, w = ROWS > 1 ? threadIdx.x >> 6 : 0;
+  i = ROWS > 1 ? blockIdx.x * 64 + lane : blockIdx.x * 256 + threadIdx.x;
+#pragma unroll
+  for (int a = 0; a < NA; ++a) d[a] = 0.0;
+  if (i < n_tgt) {
+    // the loads of several partitions in flight at once
+#pragma unroll 4
+    for (int s = w; s < n_split; s += ROWS)
+#pragma unroll
+      for (int a = 0; a < NA; ++a) d[a] += partial[((size_t)s * NA + a) * n_tgt + i];
+  }
+  if constexpr (ROWS > 1) {
+    if (w > 0) {
+#pragma unroll
+      for (int a = 0; a < NA; ++a) share[w - 1][a][lane] = d[a];
+    }
+    __syncthreads();
+    if (w > 0) return false;
+#pragma unroll
+    for (int v = 0; v < ROWS - 1; ++v)
+#pragma unroll
+      for (int a = 0; a < NA; ++a) d[a] += share[v][a][lane];
+  }
+  return i < n_tgt;
+}
+inline int reduce_rows(int n_tgt) { return n_tgt <= 32768 ? 4 : 1; }
+
 }  // namespace cvtx

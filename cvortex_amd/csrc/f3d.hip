@@ -178,7 +178,6 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
   __shared__ double s_share[Q > 1 ? Q - 1 : 1][Q > 1 ? NA : 1][64];
   const int tid = threadIdx.x;
   const int tl = Q == 1 ? tid : tid & 63;               // target within the group
-  const int part = Q == 1 ? 0 : (tid >> 6) * (WG / Q);  // first filament of this wave's part
   const int base = blockIdx.x * (WG * T / Q);
   float3 xt[T], at[T];
 #pragma unroll
@@ -264,8 +263,8 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
 #pragma unroll
         for (int a = 0; a < NA; ++a) acc[k][a] = 0.f;
     }
+    const int part = wave_part<Q>(cnt, tid), end = wave_part_end<Q>(cnt, part);
     int jv = in_vgpr(part);  // LDS index in a VGPR (no SGPR operand per filament)
-    const int end = Q == 1 ? cnt : min(cnt, part + WG / Q);
     // velocity only: +inf in a VGPR, so |kk| < fin is a VGPR compare (against
     // the literal the compiler emits a class test whose mask operand is an
     // SGPR).  Measured on 16384 filaments x 2^20 targets: vel 16.79 -> 16.54
@@ -304,10 +303,11 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
       bool carry = false;
       unsigned long long links = 0;
       for (; j + U <= end; j += U, jv += U) {
-        if ((j & 63) == 0) {
+        if ((j & 63) == 0 || (Q > 1 && j == part)) {
           const unsigned long long m = s_link[j >> 6];
           links = ((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(m >> 32)) << 32) |
                   (unsigned)__builtin_amdgcn_readfirstlane((int)m);
+          if (Q > 1) links >>= j & 63;
         }
         float4 fa[U], fb[U], f0[U];
 #pragma unroll
@@ -479,18 +479,12 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
   }
 }
 
-template <int MASK>
+template <int MASK, int ROWS>
 __global__ __launch_bounds__(256) void f3d_reduce(F3DKParams p) {
   constexpr int NA = ((MASK & OUT_VEL) ? 3 : 0) + ((MASK & OUT_DVORT) ? 4 : 0);
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= p.n_tgt) return;
+  int i;
   double d[NA];
-#pragma unroll
-  for (int a = 0; a < NA; ++a) d[a] = 0.0;
-#pragma unroll 4
-  for (int s = 0; s < p.n_split; ++s)
-#pragma unroll
-    for (int a = 0; a < NA; ++a) d[a] += p.partial[((size_t)s * NA + a) * p.n_tgt + i];
+  if (!sum_partitions<NA, ROWS>(p.partial, p.n_split, p.n_tgt, i, d)) return;
   const int t = p.tgt_perm ? p.tgt_perm[i] : i;
   float3 at = make_float3(0.f, 0.f, 0.f);
   if constexpr ((MASK & OUT_DVORT) != 0) {
@@ -528,11 +522,12 @@ F3Fn f3_pick(int mask, int acc, int T, int q) {
     default: return nullptr;
   }
 }
+template <int ROWS>
 F3Fn f3_reduce(int mask) {
   switch (mask) {
-    case OUT_VEL: return f3d_reduce<OUT_VEL>;
-    case OUT_DVORT: return f3d_reduce<OUT_DVORT>;
-    case OUT_VEL | OUT_DVORT: return f3d_reduce<OUT_VEL | OUT_DVORT>;
+    case OUT_VEL: return f3d_reduce<OUT_VEL, ROWS>;
+    case OUT_DVORT: return f3d_reduce<OUT_DVORT, ROWS>;
+    case OUT_VEL | OUT_DVORT: return f3d_reduce<OUT_VEL | OUT_DVORT, ROWS>;
     default: return nullptr;
   }
 }
@@ -760,7 +755,7 @@ hipError_t launch_f3d(const F3DJob& j, const LaunchCfg& c, hipStream_t s) {
     n_split = 1;
     split_len = j.n_fil > 0 ? j.n_fil : 1;
   } else {
-    if (split_len <= 0 || split_len % c.wg != 0) return hipErrorInvalidValue;
+    if (split_len <= 0 || split_len % (c.wg / c.q) != 0) return hipErrorInvalidValue;
     if ((long long)split_len * n_split < j.n_fil || j.partial == nullptr) return hipErrorInvalidValue;
   }
   p.n_split = n_split;
@@ -769,7 +764,9 @@ hipError_t launch_f3d(const F3DJob& j, const LaunchCfg& c, hipStream_t s) {
   hipLaunchKernelGGL(k, dim3((j.n_tgt + per - 1) / per, n_split), dim3(c.wg), 0, s, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || n_split == 1) return e;
-  hipLaunchKernelGGL(f3_reduce(j.mask), dim3((j.n_tgt + 255) / 256), dim3(256), 0, s, p);
+  const int rows = reduce_rows(j.n_tgt), sums = 256 / rows;
+  hipLaunchKernelGGL(rows == 4 ? f3_reduce<4>(j.mask) : f3_reduce<1>(j.mask),
+                     dim3((j.n_tgt + sums - 1) / sums), dim3(256), 0, s, p);
   return hipGetLastError();
 }
 

@@ -21,7 +21,7 @@ struct LaunchCfg {
   int T = 2;          // targets per lane (1, 2 or 4)
   int wg = 256;       // workgroup size (= source tile length); 256 only for now
   int n_split = 1;    // number of source partitions (each a grid row)
-  int split_len = 0;  // sources per partition, a multiple of wg
+  int split_len = 0;  // sources per partition, a multiple of wg / q
   // waves that share a group of 64 targets, each taking its part of every
   // source tile (1: every wave has targets of its own; 4: T = 1 only)
   int q = 1;

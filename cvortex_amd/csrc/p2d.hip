@@ -168,7 +168,6 @@ __global__ __launch_bounds__(WG) void p2d_kernel(P2DKParams p) {
   __shared__ double s_share[Q > 1 ? Q - 1 : 1][Q > 1 ? NA : 1][64];
   const int tid = threadIdx.x;
   const int tl = Q == 1 ? tid : tid & 63;               // target within the group
-  const int part = Q == 1 ? 0 : (tid >> 6) * (WG / Q);  // first source of this wave's part
   const int base = blockIdx.x * (WG * T / Q);
   float4 xt[T];
 #pragma unroll
@@ -227,8 +226,8 @@ __global__ __launch_bounds__(WG) void p2d_kernel(P2DKParams p) {
 #pragma unroll
         for (int a = 0; a < NA; ++a) acc[k][a] = 0.f;
     }
+    const int part = wave_part<Q>(cnt, tid), end = wave_part_end<Q>(cnt, part);
     int jv = in_vgpr(part);  // LDS index in a VGPR (no SGPR operand per source)
-    const int end = Q == 1 ? cnt : min(cnt, part + WG / Q);
     bool far = false;
     if constexpr (CULL) far = boxes_far<2>(tbox, box_combine<2, WAVES>(s_box), P2DFar<REG>::near2(p.rc));
     if (far) {
@@ -353,18 +352,12 @@ __global__ __launch_bounds__(WG) void p2d_kernel(P2DKParams p) {
   }
 }
 
-template <int MASK>
+template <int MASK, int ROWS>
 __global__ __launch_bounds__(256) void p2d_reduce(P2DKParams p) {
   constexpr int NA = ((MASK & OUT_VEL) ? 2 : 0) + ((MASK & OUT_VISC) ? 1 : 0);
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= p.n_tgt) return;
+  int i;
   double d[NA];
-#pragma unroll
-  for (int a = 0; a < NA; ++a) d[a] = 0.0;
-#pragma unroll 4
-  for (int s = 0; s < p.n_split; ++s)
-#pragma unroll
-    for (int a = 0; a < NA; ++a) d[a] += p.partial[((size_t)s * NA + a) * p.n_tgt + i];
+  if (!sum_partitions<NA, ROWS>(p.partial, p.n_split, p.n_tgt, i, d)) return;
   p2d_finish<MASK>(d, p, i);
 }
 
@@ -422,11 +415,12 @@ K2Fn p2_pick(int reg, int mask, int acc, int T, int q) {
     default: return nullptr;
   }
 }
+template <int ROWS>
 K2Fn p2_reduce(int mask) {
   switch (mask) {
-    case OUT_VEL: return p2d_reduce<OUT_VEL>;
-    case OUT_VISC: return p2d_reduce<OUT_VISC>;
-    case OUT_VEL | OUT_VISC: return p2d_reduce<OUT_VEL | OUT_VISC>;
+    case OUT_VEL: return p2d_reduce<OUT_VEL, ROWS>;
+    case OUT_VISC: return p2d_reduce<OUT_VISC, ROWS>;
+    case OUT_VEL | OUT_VISC: return p2d_reduce<OUT_VEL | OUT_VISC, ROWS>;
     default: return nullptr;
   }
 }
@@ -477,7 +471,7 @@ hipError_t launch_p2d(const P2DJob& j, const LaunchCfg& c, hipStream_t s) {
     n_split = 1;
     split_len = j.n_src > 0 ? j.n_src : 1;
   } else {
-    if (split_len <= 0 || split_len % c.wg != 0) return hipErrorInvalidValue;
+    if (split_len <= 0 || split_len % (c.wg / c.q) != 0) return hipErrorInvalidValue;
     if ((long long)split_len * n_split < j.n_src || j.partial == nullptr) return hipErrorInvalidValue;
   }
   p.n_split = n_split;
@@ -486,7 +480,9 @@ hipError_t launch_p2d(const P2DJob& j, const LaunchCfg& c, hipStream_t s) {
   hipLaunchKernelGGL(k, dim3((j.n_tgt + per - 1) / per, n_split), dim3(c.wg), 0, s, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || n_split == 1) return e;
-  hipLaunchKernelGGL(p2_reduce(j.mask), dim3((j.n_tgt + 255) / 256), dim3(256), 0, s, p);
+  const int rows = reduce_rows(j.n_tgt), sums = 256 / rows;
+  hipLaunchKernelGGL(rows == 4 ? p2_reduce<4>(j.mask) : p2_reduce<1>(j.mask),
+                     dim3((j.n_tgt + sums - 1) / sums), dim3(256), 0, s, p);
   return hipGetLastError();
 }
 

@@ -45,21 +45,13 @@ __global__ __launch_bounds__(WG) void p3d_kernel(P3DKParams p) {
                                       blockIdx.y, sm, &share);
 }
 
-template <int MASK>
+template <int MASK, int ROWS>
 __global__ __launch_bounds__(256) void p3d_reduce(P3DKParams p) {
   using L = P3DLayout<MASK>;
   constexpr int NA = L::N;
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= p.n_tgt) return;
+  int i;
   double d[NA];
-#pragma unroll
-  for (int a = 0; a < NA; ++a) d[a] = 0.0;
-  // partitions added in order; unrolled so that the loads of several
-  // partitions are in flight at once
-#pragma unroll 4
-  for (int s = 0; s < p.n_split; ++s)
-#pragma unroll
-    for (int a = 0; a < NA; ++a) d[a] += p.partial[((size_t)s * NA + a) * p.n_tgt + i];
+  if (!sum_partitions<NA, ROWS>(p.partial, p.n_split, p.n_tgt, i, d)) return;
   const int t = p.tgt_perm ? p.tgt_perm[i] : i;
   const float4 q = p.tgt_pv[t];
   float3 at = make_float3(0.f, 0.f, 0.f);
@@ -68,22 +60,6 @@ __global__ __launch_bounds__(256) void p3d_reduce(P3DKParams p) {
     at = make_float3(w.x, w.y, w.z);
   }
   p3d_finish<MASK>(d, at, q.w, p.sc, p.out_vel, p.out_dvort, p.out_visc, t);
-}
-
-// Velocity alone: one thread per target and component, so three times the
-// threads of p3d_reduce (a small problem's reduction has few targets), each
-// with sixteen partitions' loads in flight; the partitions are added in
-// order, as p3d_reduce does.  Cube of 8192 (32 partitions): 44.0 -> 43.6 us
-// per evaluation.
-__global__ __launch_bounds__(64) void p3d_reduce_vel(P3DKParams p) {
-  const int i = blockIdx.x * 64 + threadIdx.x;
-  const int c = blockIdx.y;
-  if (i >= p.n_tgt) return;
-  double d = 0.0;
-#pragma unroll 16
-  for (int s = 0; s < p.n_split; ++s) d += p.partial[((size_t)s * 3 + c) * p.n_tgt + i];
-  const int t = p.tgt_perm ? p.tgt_perm[i] : i;
-  p.out_vel[3 * (size_t)t + c] = (float)(p.sc.vel * d);
 }
 
 // ---------------------------------------------------------------------------
@@ -223,13 +199,15 @@ KernelFn pick_kernel(int reg, int mask, int acc, int T, int q) {
   }
 }
 
+template <int ROWS>
 KernelFn pick_reduce(int mask) {
   switch (mask) {
-    case OUT_DVORT: return p3d_reduce<OUT_DVORT>;
-    case OUT_VISC: return p3d_reduce<OUT_VISC>;
-    case OUT_VEL | OUT_DVORT: return p3d_reduce<OUT_VEL | OUT_DVORT>;
-    case OUT_DVORT | OUT_VISC: return p3d_reduce<OUT_DVORT | OUT_VISC>;
-    case OUT_VEL | OUT_DVORT | OUT_VISC: return p3d_reduce<OUT_VEL | OUT_DVORT | OUT_VISC>;
+    case OUT_VEL: return p3d_reduce<OUT_VEL, ROWS>;
+    case OUT_DVORT: return p3d_reduce<OUT_DVORT, ROWS>;
+    case OUT_VISC: return p3d_reduce<OUT_VISC, ROWS>;
+    case OUT_VEL | OUT_DVORT: return p3d_reduce<OUT_VEL | OUT_DVORT, ROWS>;
+    case OUT_DVORT | OUT_VISC: return p3d_reduce<OUT_DVORT | OUT_VISC, ROWS>;
+    case OUT_VEL | OUT_DVORT | OUT_VISC: return p3d_reduce<OUT_VEL | OUT_DVORT | OUT_VISC, ROWS>;
     default: return nullptr;
   }
 }
@@ -271,7 +249,7 @@ hipError_t launch_p3d(const P3DJob& j, const LaunchCfg& c, hipStream_t s) {
     n_split = 1;
     split_len = j.n_src > 0 ? j.n_src : 1;
   } else {
-    if (split_len <= 0 || split_len % c.wg != 0) return hipErrorInvalidValue;
+    if (split_len <= 0 || split_len % (c.wg / c.q) != 0) return hipErrorInvalidValue;
     if ((long long)split_len * n_split < j.n_src) return hipErrorInvalidValue;
     if (j.partial == nullptr) return hipErrorInvalidValue;
   }
@@ -283,12 +261,9 @@ hipError_t launch_p3d(const P3DJob& j, const LaunchCfg& c, hipStream_t s) {
   hipLaunchKernelGGL(k, grid, dim3(c.wg), 0, s, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || n_split == 1) return e;
-  if (j.mask == OUT_VEL) {
-    hipLaunchKernelGGL(p3d_reduce_vel, dim3((j.n_tgt + 63) / 64, 3), dim3(64), 0, s, p);
-  } else {
-    KernelFn r = pick_reduce(j.mask);
-    hipLaunchKernelGGL(r, dim3((j.n_tgt + 255) / 256), dim3(256), 0, s, p);
-  }
+  const int rows = reduce_rows(j.n_tgt), sums = 256 / rows;
+  hipLaunchKernelGGL(rows == 4 ? pick_reduce<4>(j.mask) : pick_reduce<1>(j.mask),
+                     dim3((j.n_tgt + sums - 1) / sums), dim3(256), 0, s, p);
   return hipGetLastError();
 }
 

@@ -260,7 +260,6 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
   constexpr bool DBL_ = P3DSmem<REG, MASK, ACC, WG>::DBL;
   const int tid = threadIdx.x;
   const int tl = Q == 1 ? tid : tid & 63;  // target within the group
-  const int part = Q == 1 ? 0 : (tid >> 6) * (WG / Q);  // first source of this wave's part
   float3 xt[T], at[T];
   float vt[T];
 #pragma unroll
@@ -295,6 +294,7 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
   const RegConsts rv = loop_consts(rc);
   for (int ts = s0; ts < s1; ts += WG) {
     const int cnt = min(WG, s1 - ts);
+    const int part = wave_part<Q>(cnt, tid), end = wave_part_end<Q>(cnt, part);
     __syncthreads();
     if (tid < cnt) {
       float4 q = p.src_pv[ts + tid];
@@ -334,7 +334,6 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
       // the LDS index runs in a VGPR too: an SGPR index would cost an
       // SGPR-reading move per source to form the ds_read address
       int jv = in_vgpr(part);
-      const int end = Q == 1 ? cnt : min(cnt, part + WG / Q);
 #pragma unroll kUnroll
       for (int j = part; j < end; ++j, ++jv) {
         const float4 xa = sm.xa[jv];

@@ -109,12 +109,31 @@ bool narrow(int kind, int reg, int mask, int n_src, int n_tgt, int cus) {
 // Partitions for 16 workgroups per CU of two tiles or more each, and for 4 per
 // CU down to one tile: 8192 particles (velocity, us) 40.9 with two tiles each,
 // 44.2 with four; 7000 (vel + dvort) 54.2 with three, 57.0 with two.
-LaunchCfg narrow_cfg(int n_src, int n_tgt, int cus) {
+// Below 2 workgroups per CU a tile is split too, into quarters, so that each
+// wave's run of pairs, a chain it walks alone on its SIMD, is as short as 16:
+// Gaussian vel + dvort + visc of 500 particles 20.9 -> 10.4 us, 2000 21.4 ->
+// 15.4; Winckelmans vel + dvort of 1000 11.5 -> 8.4; 2D Gaussian with the
+// viscous term 1000 17.1 -> 8.9, 3D velocity of 1000 8.8 -> 7.0.  At most 64
+// partitions (20000 sources on 50 targets: 15.7 us with 79, 27.5 with 313, whose
+// sums are one group's reduction), and where one tile holds all sources, only
+// for pairs that cost more than the second launch: 256 particles by the Gaussian
+// 18.2 -> 10.4 and Winckelmans vel + dvort 8.5 -> 7.0, but velocity 5.7 -> 6.8
+// and 100 particles 5.2 -> 6.8.
+LaunchCfg narrow_cfg(int kind, int reg, int mask, int n_src, int n_tgt, int cus) {
   const long long groups = ((long long)n_tgt + 63) / 64, tiles = ((long long)n_src + 255) / 256;
   auto fill = [&](long long per_cu) { return std::max(1LL, (per_cu * cus + groups - 1) / groups); };
   const long long k = std::min(std::max(fill(4), std::min(fill(16), tiles / 2)), tiles);
   LaunchCfg c = launch_shape(1, (int)k, n_src);
   c.q = 4;
+  const bool heavy = reg == REG_GAUSSIAN || (kind == KIND_P3D && mask != OUT_VEL);
+  if (groups * tiles < 2LL * cus && (tiles > 1 || (heavy && n_src > 128))) {
+    const long long quarters = ((long long)n_src + 63) / 64;
+    const long long kq = std::min({quarters, fill(2), 64LL});
+    if (kq > k) {
+      c.split_len = (int)((quarters + kq - 1) / kq * 64);
+      c.n_split = (n_src + c.split_len - 1) / c.split_len;
+    }
+  }
   return c;
 }
 
@@ -160,7 +179,7 @@ LaunchCfg choose_cfg(int kind, int reg, int mask, int acc, int n_src, int n_tgt,
     if (k > tiles / 2 && blocks * (tiles / 2) >= 32LL * cus) k = tiles / 2;
     return launch_shape(T, (int)std::min<long long>(k, 1 << 20), n_src);
   }
-  if (narrow(kind, reg, mask, n_src, n_tgt, cus)) return narrow_cfg(n_src, n_tgt, cus);
+  if (narrow(kind, reg, mask, n_src, n_tgt, cus)) return narrow_cfg(kind, reg, mask, n_src, n_tgt, cus);
   LaunchCfg c = default_cfg(n_src, n_tgt, n_cu);
   const bool many_blocks = (long long)(n_tgt + 255) / 256 >= 4LL * cus;
   // Filaments: one target per lane.  It fits in fewer VGPRs (more waves per

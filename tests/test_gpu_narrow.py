@@ -13,7 +13,8 @@ from gpuutil import case, have_gpu
 
 pytestmark = pytest.mark.gpu
 SIZES = [(1, 1), (63, 64), (64, 65), (65, 63), (193, 129), (257, 255), (513, 1), (1, 700),
-         (1023, 257), (4097, 65), (130, 9001)]
+         (1023, 257), (4097, 65), (130, 9001),
+         (129, 40), (9000, 3), (16500, 70)]
 
 
 @pytest.fixture(scope="module", autouse=True)
