@@ -360,7 +360,7 @@ cvtx_hip_batch* cvtx_hip_batch_create(int n_clouds, const int* offsets, const fl
   std::vector<Scales> sc(n_clouds);
   for (int c = 0; c < n_clouds; ++c) {
     range[c] = make_int2(offsets[c], offsets[c + 1]);
-    rc[c] = p3d_consts(regularisation, sigmas[c]);
+    rc[c] = p3d_consts(regularisation, sigmas[c], outputs, accumulate);
     sc[c] = p3d_scales(regularisation, sigmas[c], nu);
   }
   bool ok = true;

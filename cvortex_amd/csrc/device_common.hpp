@@ -45,7 +45,8 @@ struct RegConsts {
   float inv_s2;    // 1/sigma^2
   float c1;        // gaussian: -log2(e)/2 | 2D winckelmans eta: 4 log2(e)
   float c2;        // gaussian: sqrt(2/pi)
-  float q_far = 208.f;  // gaussian: rho^2 beyond which exp(-rho^2/2) is 0 in FP32
+  float q_far = 208.f;  // gaussian: rho^2 from which the far form is taken (p3d_consts)
+  float q_exp = 46.f;   // 3D gaussian: rho^2 from which 1 - rho zeta and G - zeta/3 round to 1 and G
   float q_tab = (float)(GTAB_RHO_MAX * GTAB_RHO_MAX);  // gaussian: table range in rho^2
   float xs = 1.f;  // 3D winckelmans: power of two that positions are multiplied by
 };
@@ -74,6 +75,7 @@ __device__ __forceinline__ RegConsts loop_consts(const RegConsts& k) {
   v.c1 = in_vgpr(k.c1);
   v.c2 = in_vgpr(k.c2);
   v.q_far = in_vgpr(k.q_far);
+  v.q_exp = in_vgpr(k.q_exp);
   v.q_tab = in_vgpr(k.q_tab);
   return v;
 }
@@ -272,14 +274,20 @@ struct RegKernel<REG_GAUSSIAN> {
   // branch, far_cb(G): the caller needs no copy of G that the near branch
   // would zero (a register copy per pair otherwise).  Ring of 2^20, fused
   // vel + dvort: 694.5 -> 679.1 ms (three A/B pairs on one box).
-  template <class Near, class FarCb>
+  // NEST: for callers that use neither zeta nor, below rho^2 = 208, anything
+  // but FP64 sums of G: beyond q_exp (there 1 - rho zeta and 1 - zeta/(3 G) round
+  // to 1) G and H are the far form's, bit for bit, and the exp is skipped.  Of
+  // the ring's rounds (a wave and a source) 9.4 % have a pair below 208 and 3.6 %
+  // one below 46: 65536 2685 -> 2652 us, cube of 50000 1681 -> 1636 (targets not
+  // ordered, where nearly every such round has both: 6000 59.8 -> 61.1 with it).
+  template <bool NEST, class Near, class FarCb>
   static __device__ __forceinline__ void eval_split(float r2, const RegConsts& k,
                                                     const float4* tab, float& Kv, float& Kh,
                                                     float& eta, Near&& near_cb, FarCb&& far_cb) {
     const Far f = far(r2, k);
     float g = f.g, h = f.h, z = 0.f;
     if (f.q < k.q_far) {
-      near(f, r2, k, tab, g, h, z);
+      if (!NEST || f.q < k.q_exp) near(f, r2, k, tab, g, h, z);
       near_cb(g, z);
     } else {
       far_cb(f.g);

@@ -150,7 +150,7 @@ hipError_t launch_relax(float4* a, const float* omega, int n, float fdt, hipStre
 
 // Host-side helpers.
 Scales p3d_scales(int reg, float sigma, float nu);
-RegConsts p3d_consts(int reg, float sigma);
+RegConsts p3d_consts(int reg, float sigma, int mask, int acc);
 bool p3d_supported(int reg, int mask);
 bool p2d_supported(int reg, int mask);
 

@@ -159,7 +159,13 @@ __global__ __launch_bounds__(WG) void p2d_kernel(P2DKParams p) {
   static_assert(Q == 1 || (T == 1 && WG == 64 * Q), "a group of shared targets is one wave wide");
   constexpr int NA = ((MASK & OUT_VEL) ? 2 : 0) + ((MASK & OUT_VISC) ? 1 : 0);
   constexpr int E = (MASK & OUT_VEL) ? 2 : 0;
-  constexpr bool CULL = P2DFar<REG>::ENABLED && (MASK & OUT_VEL) != 0;
+  constexpr bool VEL = (MASK & OUT_VEL) != 0;
+  constexpr bool CULL = P2DFar<REG>::ENABLED;
+  // whether a far tile leaves a target as it is: eta is 0 there, but not its
+  // product with a strength or an area that is not finite
+  auto passive = [](const float4& q) {
+    return VEL || (__builtin_isfinite(q.z) && __builtin_isfinite(q.w));
+  };
   constexpr bool TS = ACC != ACC_PLAIN;                           // tile sums folded by TwoSum
   constexpr bool V64 = ACC == ACC_COMP && (MASK & OUT_VISC) != 0;  // exchange summed in FP64
   constexpr int WAVES = WG / 64;
@@ -200,13 +206,14 @@ __global__ __launch_bounds__(WG) void p2d_kernel(P2DKParams p) {
     }
     bool fin = true;
 #pragma unroll
-    for (int k = 0; k < T; ++k) fin = fin && __builtin_isfinite(xt[k].x) && __builtin_isfinite(xt[k].y);
+    for (int k = 0; k < T; ++k) fin = fin && __builtin_isfinite(xt[k].x) && __builtin_isfinite(xt[k].y) && passive(xt[k]);
     tbox = block_box<2, WAVES>(lo2, hi2, fin, s_box);
   }
 
   const int s0 = blockIdx.y * p.split_len;
   const int s1 = min(s0 + p.split_len, p.n_src);
   const RegConsts rv = loop_consts(p.rc);
+  const float cexp = in_vgpr(p.rc.inv_s2 * p.rc.c1);
   for (int ts = s0; ts < s1; ts += WG) {
     const int cnt = min(WG, s1 - ts);
     __syncthreads();
@@ -217,7 +224,9 @@ __global__ __launch_bounds__(WG) void p2d_kernel(P2DKParams p) {
     }
     if constexpr (CULL) {
       const float x2[2] = {src.x, src.y};
-      box_partial<2, WAVES>(x2, tid < cnt, s_box);
+      box_partial<2, WAVES>(x2, x2, 0.f,
+                            __builtin_isfinite(src.x) && __builtin_isfinite(src.y) && passive(src),
+                            tid < cnt, s_box);
     }
     __syncthreads();
     if constexpr (TS) {
@@ -228,10 +237,14 @@ __global__ __launch_bounds__(WG) void p2d_kernel(P2DKParams p) {
     }
     const int part = wave_part<Q>(cnt, tid), end = wave_part_end<Q>(cnt, part);
     int jv = in_vgpr(part);  // LDS index in a VGPR (no SGPR operand per source)
-    bool far = false;
-    if constexpr (CULL) far = boxes_far<2>(tbox, box_combine<2, WAVES>(s_box), P2DFar<REG>::near2(p.rc));
+    bool far = false, mid = false;
+    if constexpr (CULL) {
+      const Box<2> sbox = box_combine<2, WAVES>(s_box);
+      far = boxes_far<2>(tbox, sbox, P2DFar<REG>::near2(p.rc));
+      if constexpr (REG == REG_GAUSSIAN) mid = !far && boxes_far<2>(tbox, sbox, 1.001f * p.rc.s2);
+    }
     if (far) {
-      if constexpr (CULL) {
+      if constexpr (CULL && VEL) {
         // U sources x T targets = 4 pairs per shared reciprocal; eta = 0
         constexpr int U = 4 / T;
         const float ks = in_vgpr(P2DFar<REG>::kscale(p.rc));
@@ -282,6 +295,36 @@ __global__ __launch_bounds__(WG) void p2d_kernel(P2DKParams p) {
             const float ka = __builtin_amdgcn_rcpf(__builtin_fmaf(dx, dx, dy * dy)) * as;
             acc[k][0] = __builtin_fmaf(ka, dy, acc[k][0]);
             acc[k][1] = __builtin_fmaf(ka, dx, acc[k][1]);
+          }
+        }
+      }
+    } else if (REG == REG_GAUSSIAN && mid) {
+      // Gaussian, every pair at q >= 1: (1 - e)/q and e without the range tests
+      // and the series, unrolled.  Bound by issue: 23 slots per pair with the
+      // FP64 exchange, where the general loop takes 40 and more.  100003
+      // particles of a sheet (36 % of the pairs below 208, most of them here),
+      // velocity and exchange: 3314 -> 3080 us; unrolled by one or four 3093, 3154.
+#pragma unroll 2
+      for (int j = part; j < end; ++j, ++jv) {
+        const float4 s = s_src[jv];
+        const float as = s.z * rv.s2;
+#pragma unroll
+        for (int k = 0; k < T; ++k) {
+          const float dx = xt[k].x - s.x;
+          const float dy = xt[k].y - s.y;
+          const float r2 = __builtin_fmaf(dx, dx, dy * dy);
+          const float e = __builtin_amdgcn_exp2f(r2 * cexp);
+          if constexpr (VEL) {
+            const float ka = (1.f - e) * (__builtin_amdgcn_rcpf(r2) * as);
+            acc[k][0] = __builtin_fmaf(ka, dy, acc[k][0]);
+            acc[k][1] = __builtin_fmaf(ka, dx, acc[k][1]);
+          }
+          if constexpr (V64) {
+            const double d = __builtin_fma(tA[k], (double)s.z, -(ta[k] * (double)s.w));
+            vacc[k] = __builtin_fma(d, (double)e, vacc[k]);
+          } else if constexpr ((MASK & OUT_VISC) != 0) {
+            const float d = __builtin_fmaf(xt[k].w, s.z, -(xt[k].z * s.w));
+            acc[k][E] = __builtin_fmaf(d, e, acc[k][E]);
           }
         }
       }
@@ -462,6 +505,9 @@ hipError_t launch_p2d(const P2DJob& j, const LaunchCfg& c, hipStream_t s) {
       break;
     default:
       p.rc.c1 = (float)(-0.5 / std::log(2.0));
+      // 1 - exp(-q/2) rounds to 1 from q = 34.7 on, so without eta the far form
+      // holds from there (100003 particles 2800 -> 2620 us with the middle loop)
+      if (j.mask == OUT_VEL) p.rc.q_far = 36.f;
       p.sc_vel = k2pi / (sa * sa);
       p.sc_visc = 2.0 * (double)j.nu / (sa * sa);
       break;

@@ -76,7 +76,7 @@ struct P3DKParams {
 // repeats the tile with SELF_TEST (see p3d_block).
 enum SelfMode : int { SELF_NONE, SELF_TEST, SELF_WATCH };
 
-template <int REG, int MASK, int ACC, int SELF>
+template <int REG, int MASK, int ACC, int SELF, bool NEST>
 __device__ __forceinline__ void p3d_pair(const float4 sp, const float4 sa, const double2* pxy,
                                          const double2* pzv, const float3 xt, const float3 at,
                                          const RegConsts& rc, const float4* tab, float* acc,
@@ -97,8 +97,8 @@ __device__ __forceinline__ void p3d_pair(const float4 sp, const float4 sa, const
       eta = same ? 0.f : eta;
     }
   } else if constexpr (R::SPLIT && (MASK & OUT_DVORT) != 0) {
-    RegKernel<REG_GAUSSIAN>::eval_split(r2, rc, tab, Kv, Kh, eta,
-                                        [&](float kn, float en) {
+    RegKernel<REG_GAUSSIAN>::template eval_split<NEST && (MASK & OUT_VISC) == 0>(
+        r2, rc, tab, Kv, Kh, eta, [&](float kn, float en) {
       const double2 sxy = *pxy, szv = *pzv;
       const double k = (double)kn;
       dacc[R::D_A + 0] = __builtin_fma(k, sxy.x, dacc[R::D_A + 0]);
@@ -344,7 +344,7 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
         const float4 sa = make_float4(xa.w, tl.x, tl.y, 0.f);
 #pragma unroll
         for (int k = 0; k < T; ++k)
-          p3d_pair<REG, MASK, ACC, decltype(mode)::value>(sp, sa, &sm.xy[DBL_ ? jv : 0],
+          p3d_pair<REG, MASK, ACC, decltype(mode)::value, Q == 1>(sp, sa, &sm.xy[DBL_ ? jv : 0],
                                                           &sm.zv[DBL_ ? jv : 0], xt[k], at[k], rv,
                                                           sm.tab, acc[k], dacc[k], smin);
       }
