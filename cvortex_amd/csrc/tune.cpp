@@ -137,6 +137,36 @@ LaunchCfg narrow_cfg(int kind, int reg, int mask, int n_src, int n_tgt, int cus)
   return c;
 }
 
+// 2D problems that are not narrow.  One target per lane is bound by the LDS: a
+// source's 16 bytes take its port 8 cycles per wave, 32 for the four SIMDs of a
+// CU, as long as 16 issue slots, where a far pair needs 11.  So two targets per
+// lane as soon as there is enough work, in tiles of 256 x 256 per CU, and four
+// from 1024 on for the velocity without the Gaussian's ranges (their wider blocks
+// have fewer far tiles), with partitions of two tiles or more for 64 workgroups
+// per CU, or of one for 32.  One target -> two, us: planetary 21000 particles
+// 125 -> 98, 100003 2349 -> 1600 (four: 1588), 200000 9209 -> 6108 with four;
+// Gaussian velocity 50000 697 -> 618 (30000: 292 with one, 302 with two),
+// exchange 100003 3063 -> 2925; Winckelmans with the exchange 35000 817 -> 733,
+// 200000 25185 -> 22259; its velocity at 262144 14976 -> 14846 with four, 15537
+// with two; singular, 50000, 561 with one, 587 with two.  More partitions alone:
+// Gaussian velocity and exchange 21000 particles 307 -> 208, singular 9000 34.3
+// -> 29.7.
+LaunchCfg p2d_cfg(int reg, int mask, int n_src, int n_tgt, int cus) {
+  const long long tiles = ((long long)n_src + 255) / 256;
+  auto blocks = [&](int T) { return ((long long)n_tgt + 256LL * T - 1) / (256LL * T); };
+  const bool visc = (mask & OUT_VISC) != 0;
+  const long long work = blocks(1) * tiles / cus;
+  int T = 1;
+  if (reg == REG_GAUSSIAN) T = work >= 100 ? 2 : 1;
+  else if (visc) T = work >= 24 ? 2 : 1;
+  else if (reg == REG_PLANETARY) T = work >= 1024 ? 4 : (work >= 16 ? 2 : 1);
+  else T = work >= 1024 ? 4 : 1;
+  const long long nb = blocks(T);
+  long long k = std::min((64LL * cus + nb - 1) / std::max(1LL, nb), std::max(1LL, tiles / 2));
+  if (nb * k < 32LL * cus) k = std::min((32LL * cus + nb - 1) / std::max(1LL, nb), tiles);
+  return launch_shape(T, (int)std::max(1LL, k), n_src);
+}
+
 }  // namespace
 
 LaunchCfg choose_cfg(int kind, int reg, int mask, int acc, int n_src, int n_tgt, int n_cu) {
@@ -180,6 +210,7 @@ LaunchCfg choose_cfg(int kind, int reg, int mask, int acc, int n_src, int n_tgt,
     return launch_shape(T, (int)std::min<long long>(k, 1 << 20), n_src);
   }
   if (narrow(kind, reg, mask, n_src, n_tgt, cus)) return narrow_cfg(kind, reg, mask, n_src, n_tgt, cus);
+  if (kind == KIND_P2D) return p2d_cfg(reg, mask, n_src, n_tgt, cus);
   LaunchCfg c = default_cfg(n_src, n_tgt, n_cu);
   const bool many_blocks = (long long)(n_tgt + 255) / 256 >= 4LL * cus;
   // Filaments: one target per lane.  It fits in fewer VGPRs (more waves per
@@ -189,11 +220,6 @@ LaunchCfg choose_cfg(int kind, int reg, int mask, int acc, int n_src, int n_tgt,
   // per lane -> one): vel 13.7 -> 13.1, dvort 21.1 -> 19.2, fused 21.4 ->
   // 20.4.
   if (kind == KIND_F3D && c.T > 1 && many_blocks) c = partitioned_cfg(1, n_src, n_tgt, n_cu);
-  // 2D Gaussian with the viscous term: two targets per lane (2^22 sheet,
-  // 4 partitions: 3331 ms with four, 3226 with two); planetary and the
-  // velocity alone keep four (2720 ms against 3042 with two).
-  if (kind == KIND_P2D && reg == REG_GAUSSIAN && (mask & OUT_VISC) && c.T == 4)
-    c = partitioned_cfg(2, n_src, n_tgt, n_cu);
   return c;
 }
 
