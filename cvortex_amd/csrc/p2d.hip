@@ -133,21 +133,25 @@ __device__ __forceinline__ void p2d_finish(const double* a, const P2DKParams& p,
   }
 }
 
-// Far tiles (tile_cull.hpp): for planetary and Gaussian, a pair at
-// r^2 >= near2 has K = 1/r^2 in the kernel's units (planetary: r^2 >=
-// sigma^2, outside the core; Gaussian: rho^2 >= 208, where exp(-rho^2/2) is
-// 0 in FP32 and K = 1/rho^2 = sigma^2/r^2, eta = 0), so a tile whose box is
+// Far tiles (tile_cull.hpp): a pair at r^2 >= near2 has K = 1/r^2 in the
+// kernel's units (planetary: r^2 >= sigma^2, outside the core; singular: every
+// pair that does not coincide; Gaussian: rho^2 >= 208, where exp(-rho^2/2) is 0
+// in FP32 and K = 1/rho^2 = sigma^2/r^2, eta = 0), so a tile whose box is
 // at least that far from the block's targets needs no range test: its
-// pairs take K from one shared reciprocal per four pairs.
+// pairs take K from one shared reciprocal per four pairs.  Singular and planetary
+// only with two targets per lane or more: with one the LDS bounds the loop (see
+// p2d_cfg), and the boxes cost more than the test (us, far loop -> without:
+// planetary 6000 20.4 -> 15.6, 12000 44.9 -> 38.8).  Singular with the far loop,
+// two and four targets per lane: 25000 156 -> 124, 120000 3116 -> 2298, 600000
+// 74228 -> 55657.
 template <int REG>
 struct P2DFar {
-  static constexpr bool ENABLED = REG == REG_PLANETARY || REG == REG_GAUSSIAN;
   static __device__ __forceinline__ float near2(const RegConsts& k) {
-    return REG == REG_PLANETARY ? k.s2 : k.q_far * k.s2;
+    return REG == REG_SINGULAR ? 0.f : (REG == REG_PLANETARY ? k.s2 : k.q_far * k.s2);
   }
   // factor of 1/r^2 in K
   static __device__ __forceinline__ float kscale(const RegConsts& k) {
-    return REG == REG_PLANETARY ? 1.f : k.s2;
+    return REG == REG_GAUSSIAN ? k.s2 : 1.f;
   }
 };
 
@@ -160,7 +164,7 @@ __global__ __launch_bounds__(WG) void p2d_kernel(P2DKParams p) {
   constexpr int NA = ((MASK & OUT_VEL) ? 2 : 0) + ((MASK & OUT_VISC) ? 1 : 0);
   constexpr int E = (MASK & OUT_VEL) ? 2 : 0;
   constexpr bool VEL = (MASK & OUT_VEL) != 0;
-  constexpr bool CULL = P2DFar<REG>::ENABLED;
+  constexpr bool CULL = REG == REG_GAUSSIAN || ((REG == REG_PLANETARY || REG == REG_SINGULAR) && T > 1);
   // whether a far tile leaves a target as it is: eta is 0 there, but not its
   // product with a strength or an area that is not finite
   auto passive = [](const float4& q) {
@@ -250,7 +254,7 @@ __global__ __launch_bounds__(WG) void p2d_kernel(P2DKParams p) {
         const float ks = in_vgpr(P2DFar<REG>::kscale(p.rc));
         // a_s times the factor of 1/r^2 in K (planetary: 1, so no multiply)
         auto sk = [=](float a) {
-          if constexpr (REG == REG_PLANETARY) return a;
+          if constexpr (REG != REG_GAUSSIAN) return a;
           else return a * ks;
         };
         int j = part;

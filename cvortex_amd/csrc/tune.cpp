@@ -96,14 +96,13 @@ namespace {
 // 3600 filaments on 20000 targets 242 -> 167, 10000 on 30000 467 -> 418 (on
 // 100000, 60 tiles per CU, 1054 -> 1190: a block of 64 targets has a smaller
 // box than one of 256, but its tiles are staged four times as often).
-// 2D velocities by the singular or the planetary kernel take so few
-// operations per pair that the staging counts from 4 tiles per CU on
-// (planetary 3000 14.3 -> 11.3, 7900 27.9 -> 29.6, 12000 47.6 -> 55.9).
+// 2D velocities by the singular or the planetary kernel end at 16, where two
+// targets per lane win (planetary 15000 62.6 -> 56.2, 17000 68.4 -> 71.9).
 bool narrow(int kind, int reg, int mask, int n_src, int n_tgt, int cus) {
   const long long nb = ((long long)n_tgt + 255) / 256, tiles = ((long long)n_src + 255) / 256;
   const bool light = kind == KIND_P2D && !(mask & OUT_VISC) &&
                      (reg == REG_PLANETARY || reg == REG_SINGULAR);
-  return n_tgt > 0 && tiles > 0 && nb * tiles < (light ? 4LL : 24LL) * cus;
+  return n_tgt > 0 && tiles > 0 && nb * tiles < (light ? 16LL : 24LL) * cus;
 }
 
 // Partitions for 16 workgroups per CU of two tiles or more each, and for 4 per
@@ -148,7 +147,7 @@ LaunchCfg narrow_cfg(int kind, int reg, int mask, int n_src, int n_tgt, int cus)
 // Gaussian velocity 50000 697 -> 618 (30000: 292 with one, 302 with two),
 // exchange 100003 3063 -> 2925; Winckelmans with the exchange 35000 817 -> 733,
 // 200000 25185 -> 22259; its velocity at 262144 14976 -> 14846 with four, 15537
-// with two; singular, 50000, 561 with one, 587 with two.  More partitions alone:
+// with two.  More partitions alone:
 // Gaussian velocity and exchange 21000 particles 307 -> 208, singular 9000 34.3
 // -> 29.7.
 LaunchCfg p2d_cfg(int reg, int mask, int n_src, int n_tgt, int cus) {
@@ -159,7 +158,7 @@ LaunchCfg p2d_cfg(int reg, int mask, int n_src, int n_tgt, int cus) {
   int T = 1;
   if (reg == REG_GAUSSIAN) T = work >= 100 ? 2 : 1;
   else if (visc) T = work >= 24 ? 2 : 1;
-  else if (reg == REG_PLANETARY) T = work >= 1024 ? 4 : (work >= 16 ? 2 : 1);
+  else if (reg == REG_PLANETARY || reg == REG_SINGULAR) T = work >= 1024 ? 4 : (work >= 16 ? 2 : 1);
   else T = work >= 1024 ? 4 : 1;
   const long long nb = blocks(T);
   long long k = std::min((64LL * cus + nb - 1) / std::max(1LL, nb), std::max(1LL, tiles / 2));
