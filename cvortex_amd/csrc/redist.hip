@@ -389,19 +389,24 @@ __global__ __launch_bounds__(256) void rd_nodes(const unsigned long long* __rest
 // cells, 36 in 2D), stages 64 particles at a time as the weights of the
 // block's nodes along each axis (separable: 12 or 16 evaluations per particle
 // and block instead of one per particle, node and axis), and every lane sums
-// its node in FP64 in sorted order.  Regions of many particles are split into
-// items of kItem, whose partial sums a second kernel adds in order, so that
-// the work of a wave is bounded.
+// its node in FP64 in sorted order.  Particles with no weight in the block on
+// some axis, a third of a region's for a radius of 2 and three quarters for 1,
+// are left out of the staging.  Regions of many particles are split into items
+// of kItem, whose partial sums a second kernel adds in order: a wave walks its
+// item alone, so the longest item bounds a launch on a coarse grid, where there
+// are few blocks.  Items of 2048 without that culling -> 512 with it: 308618
+// particles on 0.0177, lambda1 1260 -> 1107 us a call, on 0.03, m4' 1155 ->
+// 1010; 10^6 on 0.0177, m4' 2017 -> 1848.
 //
 // Ring of 2^20 particles, m4', h = 0.01 (131 million candidate contributions):
 // by_entries writes, sorts three times and reads 1.6 GB of entries, 4.5 ms of
-// kernels; here rd_block_sums takes 0.50 ms (8 blocks of 64 nodes per
-// particle, 24 % of whose products are nonzero: vector and LDS issue), the
-// rest 0.3 ms.  A call on host arrays 6.24 -> 2.69 ms; 800000 particles on
+// kernels; here rd_block_sums took 0.50 ms before the culling (8 blocks of 64
+// nodes per particle, 24 % of whose products are nonzero: vector and LDS
+// issue), the rest 0.3 ms.  A call on host arrays 6.24 -> 2.42 ms; 800000 particles on
 // 0.03 (lambda3) 4.31 -> 1.66; 300000 in 2D 0.96 -> 0.89.
 // ---------------------------------------------------------------------------
 constexpr int kBlockKeyBits = 30;
-constexpr int kItem = 2048;
+constexpr int kItem = 512;
 
 template <int DIM>
 struct Blk {
@@ -639,7 +644,10 @@ __global__ __launch_bounds__(256) void rd_block_sums(
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
     const int e = base + lane;
-    if (e < i1) {
+    float wt[DIM * SIDE];
+    float4 al = make_float4(0.f, 0.f, 0.f, 0.f);
+    bool live = e < i1;
+    if (live) {
       int s = 0;  // the last cell that starts at or before e
 #pragma unroll
       for (int h = 32; h > 0; h >>= 1)
@@ -647,26 +655,36 @@ __global__ __launch_bounds__(256) void rd_block_sums(
       const int i = s_start[w][s] + e - s_pref[w][s];
       const float4 p = spv[i];
       const float x[3] = {p.x, p.y, p.z};
-      float4 al;
       if constexpr (DIM == 3) al = sa[i];
       else al = make_float4(p.z, 0.f, 0.f, 0.f);
 #pragma unroll
       for (int c = 0; c < DIM; ++c) {
         const unsigned q = nearest<DIM>(x[c], g, c);
+        bool reaches = false;
 #pragma unroll
         for (int m = 0; m < SIDE; ++m) {
           const unsigned nd = q0[c] + m;
           const bool in = nd - q + (unsigned)g.R <= 2u * (unsigned)g.R;
           const float pos = rn_add(g.mn[c], rn_mul(g.h, (float)nd));
           const float U = fabsf(rn_mul(rn_sub(x[c], pos), g.rh));
-          s_w[w][lane][c * SIDE + m] = in ? rd_f<RID>(U) : 0.f;
+          wt[c * SIDE + m] = in ? rd_f<RID>(U) : 0.f;
+          reaches = reaches || wt[c * SIDE + m] != 0.f;
         }
+        live = live && reaches;
       }
-      s_a[w][lane] = al;
+    }
+    // only the particles with a weight on every axis are staged, in order
+    const unsigned long long lives = __ballot(live);
+    if (live) {
+      const int at = __popcll(lives & ((1ull << lane) - 1));
+#pragma unroll
+      for (int m = 0; m < DIM * SIDE; ++m) s_w[w][at][m] = wt[m];
+      s_a[w][at] = al;
     }
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
     __builtin_amdgcn_wave_barrier();
-    const int cnt = min(64, i1 - base);
+    const int cnt = __popcll(lives);
+#pragma unroll 4
     for (int j = 0; j < cnt; ++j) {
       float frac = s_w[w][j][node[0]];
       frac = rn_mul(frac, s_w[w][j][SIDE + node[1]]);
