@@ -402,7 +402,7 @@ __global__ __launch_bounds__(256) void rd_nodes(const unsigned long long* __rest
 // by_entries writes, sorts three times and reads 1.6 GB of entries, 4.5 ms of
 // kernels; here rd_block_sums took 0.50 ms before the culling (8 blocks of 64
 // nodes per particle, 24 % of whose products are nonzero: vector and LDS
-// issue), the rest 0.3 ms.  A call on host arrays 6.24 -> 2.42 ms; 800000 particles on
+// issue), the rest 0.3 ms.  A call on host arrays 6.24 -> 2.29 ms; 800000 particles on
 // 0.03 (lambda3) 4.31 -> 1.66; 300000 in 2D 0.96 -> 0.89.
 // ---------------------------------------------------------------------------
 constexpr int kBlockKeyBits = 30;
@@ -793,30 +793,34 @@ __global__ __launch_bounds__(256) void rd_str_stats(const float* __restrict__ st
 
 // The removal threshold, negligible x the mean strength, from the blocks' sums
 // (added in block order, in the reference's types: src/P3D.cpp:600-605).
-__global__ __launch_bounds__(64) void rd_threshold(const double* __restrict__ psum, int n,
+__global__ __launch_bounds__(kPartBlocks) void rd_threshold(const double* __restrict__ psum, int n,
                                                    float negligible, float* __restrict__ thr) {
   __shared__ double s[kPartBlocks];
-  for (int i = threadIdx.x; i < kPartBlocks; i += 64) s[i] = psum[i];
+  s[threadIdx.x] = psum[threadIdx.x];
   __syncthreads();
   if (threadIdx.x != 0) return;
   double a = 0.0;
+#pragma unroll 16
   for (int b = 0; b < kPartBlocks; ++b) a += s[b];
   const float mean = __fdiv_rn((float)a, (float)n);
   *thr = rn_mul(mean, negligible);
 }
 
 // Each kept particle's share of the removed strength.
-__global__ __launch_bounds__(64) void rd_share(const double* __restrict__ pdef,
+__global__ __launch_bounds__(kPartBlocks) void rd_share(const double* __restrict__ pdef,
                                                const int* __restrict__ n_kept,
                                                float4* __restrict__ share) {
   __shared__ double s[kPartBlocks * 3];
-  for (int i = threadIdx.x; i < kPartBlocks * 3; i += 64) s[i] = pdef[i];
+#pragma unroll
+  for (int k = 0; k < 3; ++k) s[k * kPartBlocks + threadIdx.x] = pdef[k * kPartBlocks + threadIdx.x];
   __syncthreads();
   const int c = threadIdx.x;
   if (c >= 4) return;
   double d = 0.0;
-  if (c < 3)
+  if (c < 3) {
+#pragma unroll 16
     for (int b = 0; b < kPartBlocks; ++b) d += s[b * 3 + c];
+  }
   // the reference divides the removed strength by the kept count in FP32
   reinterpret_cast<float*>(share)[c] = c < 3 ? __fdiv_rn((float)d, (float)*n_kept) : 0.f;
 }
@@ -994,7 +998,7 @@ bool alloc_nodes(Runtime& rt, Device& d, int nn, Nodes* n, hipStream_t s) {
   if (e != hipSuccess) return rd_fail(rt, "select size", e), false;
   const size_t need = al256(n->sel_bytes) + al256(nn) + al256(sizeof(float4) * nn) * 4 +
                       al256(sizeof(float) * nn) * 2 + al256(sizeof(int) * nn) + al256(sizeof(int)) +
-                      al256(sizeof(double) * kPartBlocks * 3) + al256(sizeof(float) * kPartBlocks) * 2 +
+                      al256(sizeof(double) * kPartBlocks * 3) + al256(sizeof(float) * kPartBlocks * 2) +
                       al256(sizeof(int) * 1024) + al256(sizeof(float4)) * 2 +
                       al256(sizeof(float) * 7 * (size_t)nn);
   Arena na;
@@ -1012,8 +1016,8 @@ bool alloc_nodes(Runtime& rt, Device& d, int nn, Nodes* n, hipStream_t s) {
   n->kidx = na.take<int>(nn);
   n->nkept = na.take<int>(1);
   n->pdef = na.take<double>(kPartBlocks * 3);
-  n->psmin = na.take<float>(kPartBlocks);
-  n->psmax = na.take<float>(kPartBlocks);
+  n->psmin = na.take<float>(2 * kPartBlocks);
+  n->psmax = n->psmin + kPartBlocks;
   n->counts = na.take<int>(1024);
   n->thr = na.take<float>(1);
   n->share = na.take<float4>(1);
@@ -1022,13 +1026,32 @@ bool alloc_nodes(Runtime& rt, Device& d, int nn, Nodes* n, hipStream_t s) {
   return true;
 }
 
-// Running counts (in place of `counts`, into `incl`) and their total on the host.
+// What comes back to the host, in pinned memory: a copy to pageable memory goes
+// through a staging buffer and waits for it on its own.  A call makes four to ten
+// such copies; with the three of the bounds in one, and rd_threshold's and
+// rd_share's loads in flight at once, us a call: 8000 particles on 0.008
+// 548 -> 405, on 0.03 393 -> 300, 308618 on 0.0177 1107 -> 1006, 8000 in 2D
+// 350 -> 282.
+struct Bounds {
+  float mn[kPartBlocks * 3], mx[kPartBlocks * 3];
+  double sum[kPartBlocks * 3];
+};
+struct Landing {
+  Bounds bounds;
+  float smin[kPartBlocks], smax[kPartBlocks];  // adjacent on the device too
+  int bins[1024];
+  int total;
+  float threshold;
+};
+
+// Running counts (in place of `counts`, into `incl`); with `land`, their total
+// in land->total.
 bool running_counts(Runtime& rt, int* counts, int* incl, size_t n, void* tmp, size_t tmp_bytes,
-                    int* total, hipStream_t s) {
+                    Landing* land, hipStream_t s) {
   hipError_t e = rocprim::inclusive_scan(tmp, tmp_bytes, counts, incl, n, rocprim::plus<int>(), s);
-  if (e == hipSuccess && total)
-    e = hipMemcpyAsync(total, incl + (n - 1), sizeof(int), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess && total) e = hipStreamSynchronize(s);
+  if (e == hipSuccess && land)
+    e = hipMemcpyAsync(&land->total, incl + (n - 1), sizeof(int), hipMemcpyDeviceToHost, s);
+  if (e == hipSuccess && land) e = hipStreamSynchronize(s);
   if (e != hipSuccess) return rd_fail(rt, "redistribution scan", e), false;
   return true;
 }
@@ -1045,7 +1068,7 @@ constexpr size_t kBlockBytes = (size_t)4 << 30;
 
 template <int DIM>
 int by_blocks(Runtime& rt, Device& d, const RedistJob& j, const Grid& g, int key_bits, Nodes* out,
-              hipStream_t s) {
+              Landing* land, hipStream_t s) {
   using B = Blk<DIM>;
   if (key_bits > kBlockKeyBits || key_bits < 6) return kNotByBlocks;
   const int n = j.n;
@@ -1097,8 +1120,8 @@ int by_blocks(Runtime& rt, Device& d, const RedistJob& j, const Grid& g, int key
   if (!running_counts(rt, pop, cincl, cw, tmp, scan_tmp, nullptr, s)) return -1;
   hipLaunchKernelGGL(rd_starts<DIM>, pg, blk, 0, s, keys, n, cells, cincl, starts);
   hipLaunchKernelGGL(rd_popcounts, dim3((bw + 255) / 256), blk, 0, s, blocks, bw, pop);
-  int nb = 0;
-  if (!running_counts(rt, pop, bincl, bw, tmp, scan_tmp, &nb, s)) return -1;
+  if (!running_counts(rt, pop, bincl, bw, tmp, scan_tmp, land, s)) return -1;
+  const int nb = land->total;
   if (nb == 0) return kNotByBlocks;
   // ---- items of each block's region, their sums ----
   const size_t most = (size_t)nb + (size_t)kRegionsOfACell * n / kItem + 1;
@@ -1136,8 +1159,8 @@ int by_blocks(Runtime& rt, Device& d, const RedistJob& j, const Grid& g, int key
   hipLaunchKernelGGL(sum, dim3((unsigned)((most + 3) / 4)), blk, 0, s, spv, sa, g, list, n_cells,
                      cells, cincl, starts, ilist, iincl + (nb - 1), sums, nonzero);
   hipLaunchKernelGGL(rd_block_nodes, bg, blk, 0, s, items, iincl, nb, nonzero, mask, ncount);
-  int nn = 0;
-  if (!running_counts(rt, ncount, nincl, nb, tmp2, scan_tmp, &nn, s)) return -1;
+  if (!running_counts(rt, ncount, nincl, nb, tmp2, scan_tmp, land, s)) return -1;
+  const int nn = land->total;
   if (nn == 0) return 0;
   if (!alloc_nodes(rt, d, nn, out, s)) return -1;
   hipLaunchKernelGGL(rd_emit<DIM>, wg, blk, 0, s, list, items, iincl, nb, mask, nincl, sums, g,
@@ -1150,7 +1173,7 @@ int by_blocks(Runtime& rt, Device& d, const RedistJob& j, const Grid& g, int key
 // Nodes by sorting every nonzero (node, contribution) entry: any grid.
 template <int DIM>
 int by_entries(Runtime& rt, Device& d, const RedistJob& j, const Grid& g, int key_bits, Nodes* out,
-               hipStream_t s) {
+               Landing* land, hipStream_t s) {
   auto fail = [&](const char* what, hipError_t e) { return rd_fail(rt, what, e); };
   const int n = j.n;
   const int W = 2 * g.R + 1;
@@ -1172,7 +1195,9 @@ int by_entries(Runtime& rt, Device& d, const RedistJob& j, const Grid& g, int ke
   void* ct = ca.take<char>(scan_tmp);
   // the count of the chunks' items (in cincl's last element) on the host
   auto scan_total = [&](long chunks, int* total) {
-    return running_counts(rt, ccount, cincl, (size_t)chunks, ct, scan_tmp, total, s);
+    if (!running_counts(rt, ccount, cincl, (size_t)chunks, ct, scan_tmp, land, s)) return false;
+    *total = land->total;
+    return true;
   };
   e = launch_contrib_count<DIM>(j.rid, j.pv, j.a, ne, g, ccount, s);
   if (e != hipSuccess) return fail("redistribution contributions", e);
@@ -1234,29 +1259,16 @@ static int redistribute_dim(Runtime& rt, Device& d, const RedistJob& j, float** 
   *out_dev = nullptr;
   if (n == 0) return 0;
   // ---- grid origin (reference src/P3D.cpp:538-548) ----
-  float* pmin = nullptr;
-  float* pmax = nullptr;
-  double* psum = nullptr;
-  {
-    Arena small;
-    const size_t bytes = 2 * al256(sizeof(float) * kPartBlocks * 3) + al256(sizeof(double) * kPartBlocks * 3);
-    small.base = (char*)device_buffer(rt, d, SLOT_RD_SMALL, bytes);
-    small.cap = bytes;
-    if (!small.base) return -1;
-    pmin = small.take<float>(kPartBlocks * 3);
-    pmax = small.take<float>(kPartBlocks * 3);
-    psum = small.take<double>(kPartBlocks * 3);
-  }
-  hipLaunchKernelGGL((rd_bounds<DIM>), dim3(kPartBlocks), dim3(256), 0, s, j.pv, n, pmin, pmax, psum);
-  std::vector<float> hmin(kPartBlocks * DIM), hmax(kPartBlocks * DIM);
-  std::vector<double> hsum(kPartBlocks * DIM);
-  hipError_t e = hipMemcpyAsync(hmin.data(), pmin, sizeof(float) * hmin.size(), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(hmax.data(), pmax, sizeof(float) * hmax.size(), hipMemcpyDeviceToHost, s);
-  if (e == hipSuccess)
-    e = hipMemcpyAsync(hsum.data(), psum, sizeof(double) * hsum.size(), hipMemcpyDeviceToHost, s);
+  Bounds* db = (Bounds*)device_buffer(rt, d, SLOT_RD_SMALL, sizeof(Bounds));
+  Landing* land = (Landing*)host_buffer(rt, d, SLOT_RD_SMALL, sizeof(Landing));
+  if (!db || !land) return -1;
+  hipLaunchKernelGGL((rd_bounds<DIM>), dim3(kPartBlocks), dim3(256), 0, s, j.pv, n, db->mn, db->mx,
+                     db->sum);
+  hipError_t e = hipMemcpyAsync(&land->bounds, db, sizeof(Bounds), hipMemcpyDeviceToHost, s);
   if (e == hipSuccess) e = hipStreamSynchronize(s);
   if (e != hipSuccess) return fail("redistribution bounds", e);
+  const float *hmin = land->bounds.mn, *hmax = land->bounds.mx;
+  const double* hsum = land->bounds.sum;
   Grid g{};
   g.h = j.h;
   g.rh = 1.f / j.h;
@@ -1287,8 +1299,8 @@ static int redistribute_dim(Runtime& rt, Device& d, const RedistJob& j, float** 
   if ((long)n * (DIM == 3 ? W * W * W : W * W) >= 2147483647L)
     return fail("too many grid contributions for one call", hipSuccess);
   Nodes nd;
-  int nn = by_blocks<DIM>(rt, d, j, g, key_bits, &nd, s);
-  if (nn == kNotByBlocks) nn = by_entries<DIM>(rt, d, j, g, key_bits, &nd, s);
+  int nn = by_blocks<DIM>(rt, d, j, g, key_bits, &nd, land, s);
+  if (nn == kNotByBlocks) nn = by_entries<DIM>(rt, d, j, g, key_bits, &nd, land, s);
   if (nn <= 0) return nn;
   // ---- removal: strength <= threshold (in nd.thr) or index >= max_keep ----
   auto remove = [&](int max_keep) -> int {
@@ -1298,42 +1310,40 @@ static int redistribute_dim(Runtime& rt, Device& d, const RedistJob& j, float** 
     hipError_t ee = rocprim::select(nd.sel, tb2, rocprim::counting_iterator<int>(0), nd.head,
                                     nd.kidx, nd.nkept, (size_t)nn, s);
     if (ee != hipSuccess) return fail("redistribution compaction", ee);
-    hipLaunchKernelGGL(rd_share, dim3(1), dim3(64), 0, s, nd.pdef, nd.nkept, nd.share);
+    hipLaunchKernelGGL(rd_share, dim3(1), dim3(kPartBlocks), 0, s, nd.pdef, nd.nkept, nd.share);
     hipLaunchKernelGGL((rd_keep<DIM>), dim3((nn + 255) / 256), dim3(256), 0, s, nd.kidx, nd.nkept,
                        nd.pos0, nd.w0, nd.share, nd.pos1, nd.w1, nd.str1);
-    int hk = 0;
-    ee = hipMemcpyAsync(&hk, nd.nkept, sizeof(int), hipMemcpyDeviceToHost, s);
+    ee = hipMemcpyAsync(&land->total, nd.nkept, sizeof(int), hipMemcpyDeviceToHost, s);
     if (ee == hipSuccess) ee = hipStreamSynchronize(s);
     if (ee != hipSuccess) return fail("redistribution compaction", ee);
     std::swap(nd.pos0, nd.pos1);
     std::swap(nd.w0, nd.w1);
     std::swap(nd.str0, nd.str1);
-    nn = hk;
+    nn = land->total;
     return 0;
   };
   hipLaunchKernelGGL(rd_str_stats, dim3(kPartBlocks), dim3(256), 0, s, nd.str0, nn, nd.pdef,
                      nd.psmin, nd.psmax);
-  hipLaunchKernelGGL(rd_threshold, dim3(1), dim3(64), 0, s, nd.pdef, nn, j.negligible, nd.thr);
+  hipLaunchKernelGGL(rd_threshold, dim3(1), dim3(kPartBlocks), 0, s, nd.pdef, nn, j.negligible, nd.thr);
   if (remove(nn) != 0) return -1;
   if (j.max_out >= 0 && nn > j.max_out) {
     // strength threshold, reference src/redistribution_helper_funcs.cpp:33-80
     hipLaunchKernelGGL(rd_str_stats, dim3(kPartBlocks), dim3(256), 0, s, nd.str0, nn, nd.pdef,
                        nd.psmin, nd.psmax);
-    std::vector<float> hl(kPartBlocks), hh(kPartBlocks);
-    e = hipMemcpyAsync(hl.data(), nd.psmin, sizeof(float) * kPartBlocks, hipMemcpyDeviceToHost, s);
-    if (e == hipSuccess)
-      e = hipMemcpyAsync(hh.data(), nd.psmax, sizeof(float) * kPartBlocks, hipMemcpyDeviceToHost, s);
+    static_assert(offsetof(Landing, smax) - offsetof(Landing, smin) == sizeof(float) * kPartBlocks,
+                  "adjacent");
+    e = hipMemcpyAsync(land->smin, nd.psmin, sizeof(float) * kPartBlocks * 2, hipMemcpyDeviceToHost, s);
     if (e == hipSuccess) e = hipStreamSynchronize(s);
     if (e != hipSuccess) return fail("redistribution strengths", e);
     float smin = __builtin_inff(), smax = -__builtin_inff();
     for (int b = 0; b < kPartBlocks; ++b) {
-      smin = hl[b] < smin ? hl[b] : smin;
-      smax = hh[b] > smax ? hh[b] : smax;
+      smin = land->smin[b] < smin ? land->smin[b] : smin;
+      smax = land->smax[b] > smax ? land->smax[b] : smax;
     }
     double minv = smin, maxv = smax, range;
     const int n_guesses = 1024;
     std::vector<float> guesses(n_guesses);
-    std::vector<int> gc(n_guesses);
+    int* gc = land->bins;
     int k = 0;
     const float tol = 0.01f;
     for (int iter = 0; iter < 4096; ++iter) {
@@ -1344,7 +1354,7 @@ static int redistribute_dim(Runtime& rt, Device& d, const RedistJob& j, float** 
       if (e != hipSuccess) return fail("redistribution histogram", e);
       hipLaunchKernelGGL(rd_hist, dim3(kPartBlocks), dim3(256), 0, s, nd.str0, nn, minv, range,
                          nd.counts);
-      e = hipMemcpyAsync(gc.data(), nd.counts, sizeof(int) * 1024, hipMemcpyDeviceToHost, s);
+      e = hipMemcpyAsync(gc, nd.counts, sizeof(int) * 1024, hipMemcpyDeviceToHost, s);
       if (e == hipSuccess) e = hipStreamSynchronize(s);
       if (e != hipSuccess) return fail("redistribution histogram", e);
       int interp = gc[n_guesses - 1];
@@ -1362,7 +1372,8 @@ static int redistribute_dim(Runtime& rt, Device& d, const RedistJob& j, float** 
           std::fabs((float)(j.max_out - gc[k]) / ((float)j.max_out)) < tol * 0.6)
         break;
     }
-    e = hipMemcpyAsync(nd.thr, &guesses[k], sizeof(float), hipMemcpyHostToDevice, s);
+    land->threshold = guesses[k];
+    e = hipMemcpyAsync(nd.thr, &land->threshold, sizeof(float), hipMemcpyHostToDevice, s);
     if (e != hipSuccess) return fail("redistribution threshold", e);
     if (remove(j.max_out) != 0) return -1;
   }
