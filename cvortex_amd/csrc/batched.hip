@@ -66,7 +66,7 @@ __global__ __launch_bounds__(WG) void p3d_batched_kernel(BatchParams bp) {
     if (u >= bp.n_units) break;  // uniform over the workgroup
     const int2 un = bp.units[u];
     const int2 r = bp.range[un.x];
-    p3d_block<REG, MASK, ACC, T, WG>(bp.base, bp.rc[un.x], bp.sc[un.x], un.y, r.y, r.x, r.y, 0, sm);
+    p3d_block<REG, MASK, ACC, T, WG, false>(bp.base, bp.rc[un.x], bp.sc[un.x], un.y, r.y, r.x, r.y, 0, sm);
   }
 }
 
@@ -360,8 +360,8 @@ cvtx_hip_batch* cvtx_hip_batch_create(int n_clouds, const int* offsets, const fl
   std::vector<Scales> sc(n_clouds);
   for (int c = 0; c < n_clouds; ++c) {
     range[c] = make_int2(offsets[c], offsets[c + 1]);
-    rc[c] = p3d_consts(regularisation, sigmas[c], outputs, accumulate);
-    sc[c] = p3d_scales(regularisation, sigmas[c], nu);
+    rc[c] = p3d_consts(regularisation, sigmas[c], outputs, accumulate, false);
+    sc[c] = p3d_scales(regularisation, sigmas[c], nu, false);
   }
   bool ok = true;
   const size_t nc = std::max(1, n_clouds);

@@ -48,7 +48,10 @@ struct RegConsts {
   float q_far = 208.f;  // gaussian: rho^2 from which the far form is taken (p3d_consts)
   float q_exp = 46.f;   // 3D gaussian: rho^2 from which 1 - rho zeta and G - zeta/3 round to 1 and G
   float q_tab = (float)(GTAB_RHO_MAX * GTAB_RHO_MAX);  // gaussian: table range in rho^2
-  float xs = 1.f;  // 3D winckelmans: power of two that positions are multiplied by
+  float xs = 1.f;  // 3D winckelmans, gaussian: power of two that positions are multiplied by
+  // 3D gaussian, with t from GaussianKernel: 1/t^3, 1/t^5, t^3, -1/t,
+  // -1/(3 t^3), GTAB_PER_UNIT/t (used by the near ranges only)
+  float g3 = 1.f, h5 = 1.f, t3 = 1.f, nt1 = -1.f, nt3 = -1.f / 3.f, tp = GTAB_PER_UNIT;
 };
 
 // A uniform value that a pair loop reads on every pair, held in a VGPR.  On
@@ -69,7 +72,7 @@ __device__ __forceinline__ int in_vgpr(int x) {
 
 // The constants of `k` as VGPR values (see in_vgpr), for use inside pair loops.
 __device__ __forceinline__ RegConsts loop_consts(const RegConsts& k) {
-  RegConsts v;
+  RegConsts v = k;
   v.s2 = in_vgpr(k.s2);
   v.inv_s2 = in_vgpr(k.inv_s2);
   v.c1 = in_vgpr(k.c1);
@@ -185,62 +188,86 @@ struct RegKernel<REG_PLANETARY> {
   }
 };
 
-template <>
-struct RegKernel<REG_GAUSSIAN> {
-  // Works in reduced units: Kv = G(rho), Kh = H(rho)/3 (the epilogue scales
-  // by |sigma|^-3 and 3 |sigma|^-5), eta = zeta = sqrt(2/pi) exp(-rho^2/2).
-  // Three ranges of rho^2, nested so that a wave runs only the ranges its
+// DIRECT: see below; the other regularisations have one form.
+template <bool DIRECT>
+struct GaussianKernel {
+  // Positions come multiplied by a power of two (RegConsts::xs, exact) that puts
+  // sigma in [1, 2).  In those units, with t = sigma (DIRECT), Kv = G(rho)/t^3, Kh
+  // = H(rho)/(3 t^5), eta = zeta = sqrt(2/pi) exp(-rho^2/2): beyond the core Kv =
+  // r^-3 and Kh = r^-5, so the usual pair does without rho^2 = r^2/sigma^2, one
+  // issue slot of about 33 for velocity and stretching, and one rounding.  The
+  // near ranges, which need rho, pay two multiplications and a rounding instead.
+  // So !DIRECT (r^2 taken in units of sigma^2, t = 1) where most rounds (a wave
+  // and a source) have a near pair: targets that are not ordered, that is clouds
+  // and small problems (q = 4).  Reduced -> DIRECT: ring of 2^20 661.8 -> 635 ms,
+  // velocity of a ring of 100000 4005 -> 3953 us, its error against 64 bits
+  // 7.2e-8 -> 5.3e-8, of the ring of 65536 1.2e-7 -> 8.1e-8; but 48 clouds 16.3
+  // -> 17.0 ms and 3.3e-7 -> 3.4e-7.
+  // Three ranges of rho^2 (limits in r^2), nested so that a wave runs only the ranges its
   // lanes need (for spatially ordered targets, order.hip, a wave's lanes
   // are close together and most sources fall in the first range for all):
   //   rho^2 >= 208: exp(-rho^2/2) < 2^-149 is zero in FP32, so
-  //                 G = rho^-3, H/3 = rho^-5, zeta = 0;
+  //                 G = rho^-3, H/3 = rho^-5, zeta = 0: Kv = r^-3, Kh = r^-5;
   //   rho^2 >= 36:  erf(rho/sqrt2) = 1 to below 2e-9, so
   //                 G = rho^-3 (1 - rho zeta), H/3 = (G - zeta/3) rho^-2;
   //   rho^2 < 36:   cubic pieces of G and H/3 from the LDS table, built on the host from
   //                 exact FP64 values (series below rho = 0.5), so the
   //                 small-rho behaviour has no cancellation.
-  // r2 == 0 (self or coincident pair) falls in the last range, where G and
-  // zeta are zeroed; H stays finite and only ever multiplies d = 0.
+  // A self or coincident pair falls in the last range, where same() is asked and
+  // G and zeta are zeroed; H stays finite and only ever multiplies d = 0.  1e-30
+  // added to r2 (by the caller if DIRECT) keeps 1/r finite.
   //
-  // eval_ranges also reports the split between the ranges: near(Kv, eta) is
+  // eval_ranges also reports the split between the ranges: near(G, eta) is
   // called inside the rho^2 < 208 branch (only there is eta nonzero), and
   // Kfar is Kv for the pairs beyond it and 0 for the others.  A caller can so
   // accumulate the near pairs in a wider type at the cost of the branch only.
   // The evaluation in two steps, for callers that interleave pairs:
   // far() is the rho^2 >= 208 form every pair starts from, near() replaces
   // g and h and sets zeta for a pair with rho^2 < 208 (the caller tests
-  // q < k.q_far).  eval_ranges is the two combined.
+  // r2 < k.q_far).  eval_ranges is the two combined.
   struct Far {
-    float q, pinv, pinv2, g, h;
+    float pinv, pinv2, g, h;
   };
-  static __device__ __forceinline__ Far far(float r2, const RegConsts& k) {
+  static __device__ __forceinline__ Far far(float& r2, const RegConsts& k) {
+    if constexpr (!DIRECT) r2 = __builtin_fmaf(r2, k.inv_s2, 1e-30f);
     Far f;
-    f.q = __builtin_fmaf(r2, k.inv_s2, 1e-30f);  // rho^2; the 1e-30 keeps rho finite at r2 = 0
-    f.pinv = __builtin_amdgcn_rsqf(f.q);         // 1/rho
+    f.pinv = __builtin_amdgcn_rsqf(r2);  // 1/r
     f.pinv2 = f.pinv * f.pinv;
     f.g = f.pinv2 * f.pinv;
     f.h = f.g * f.pinv2;
     return f;
   }
+  // (G itself in gr where the caller sums it in FP64: its product with 1/t^3
+  // would be rounded to FP32, so the epilogue multiplies the sum.)
+  template <class Same>
   static __device__ __forceinline__ void near(const Far& f, float r2, const RegConsts& k,
-                                              const float4* tab, float& g, float& h,
-                                              float& z) {
-    z = k.c2 * __builtin_amdgcn_exp2f(f.q * k.c1);
-    g = f.pinv2 * (f.pinv - z);
-    h = __builtin_fmaf(z, -1.f / 3.f, g) * f.pinv2;
-    if (f.q < k.q_tab) {
-      float t = f.q * f.pinv * (float)GTAB_PER_UNIT;  // rho * 16
+                                              const float4* tab, Same&& same, float& g, float& h,
+                                              float& z, float& gr) {
+    z = k.c2 * __builtin_amdgcn_exp2f(r2 * k.c1);
+    if constexpr (DIRECT) {
+      g = f.pinv2 * __builtin_fmaf(z, k.nt1, f.pinv);
+      h = __builtin_fmaf(z, k.nt3, g) * f.pinv2;
+      gr = g * k.t3;
+    } else {
+      g = f.pinv2 * (f.pinv - z);
+      h = __builtin_fmaf(z, -1.f / 3.f, g) * f.pinv2;
+      gr = g;
+    }
+    if (r2 < k.q_tab) {
+      float t = r2 * f.pinv * (DIRECT ? k.tp : (float)GTAB_PER_UNIT);  // rho * 16
       int i = (int)t;
       i = i < (GTAB_N - 1) ? i : (GTAB_N - 1);
       i = i > 0 ? i : 0;
       float u = t - (float)i;
       float4 cg = tab[2 * i];
       float4 ch = tab[2 * i + 1];
-      g = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(cg.w, u, cg.z), u, cg.y), u, cg.x);
+      gr = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(cg.w, u, cg.z), u, cg.y), u, cg.x);
       h = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(ch.w, u, ch.z), u, ch.y), u, ch.x);
-      bool zr = (r2 == 0.f);
-      g = zr ? 0.f : g;
+      if constexpr (DIRECT) h *= k.h5;
+      const bool zr = same();
+      gr = zr ? 0.f : gr;
       z = zr ? 0.f : z;
+      g = DIRECT ? gr * k.g3 : gr;
     }
   }
 
@@ -252,16 +279,18 @@ struct RegKernel<REG_GAUSSIAN> {
   // compensated vel-only kernel 593 -> 515 ms with the pin; the plain FP32
   // vel+dvort kernel (two targets per lane) 680 -> 700 ms, so eval() does
   // not pin.
-  template <bool PIN = false, class Near>
+  template <bool PIN = false, class Same, class Near>
   static __device__ __forceinline__ void eval_ranges(float r2, const RegConsts& k,
-                                                     const float4* tab, float& Kv, float& Kh,
-                                                     float& eta, float& Kfar, Near&& near_cb) {
+                                                     const float4* tab, Same&& same, float& Kv,
+                                                     float& Kh, float& eta, float& Kfar,
+                                                     Near&& near_cb) {
     const Far f = far(r2, k);
     float g = f.g, h = f.h, z = 0.f, kf = f.g;
-    if (f.q < k.q_far) {
+    if (r2 < k.q_far) {
       if constexpr (PIN) asm volatile("");
-      near(f, r2, k, tab, g, h, z);
-      near_cb(g, z);
+      float gr;
+      near(f, r2, k, tab, same, g, h, z, gr);
+      near_cb(gr, z);
       kf = 0.f;
     }
     Kv = g;
@@ -280,15 +309,17 @@ struct RegKernel<REG_GAUSSIAN> {
   // the ring's rounds (a wave and a source) 9.4 % have a pair below 208 and 3.6 %
   // one below 46: 65536 2685 -> 2652 us, cube of 50000 1681 -> 1636 (targets not
   // ordered, where nearly every such round has both: 6000 59.8 -> 61.1 with it).
-  template <bool NEST, class Near, class FarCb>
+  template <bool NEST, class Same, class Near, class FarCb>
   static __device__ __forceinline__ void eval_split(float r2, const RegConsts& k,
-                                                    const float4* tab, float& Kv, float& Kh,
-                                                    float& eta, Near&& near_cb, FarCb&& far_cb) {
+                                                    const float4* tab, Same&& same, float& Kv,
+                                                    float& Kh, float& eta, Near&& near_cb,
+                                                    FarCb&& far_cb) {
     const Far f = far(r2, k);
     float g = f.g, h = f.h, z = 0.f;
-    if (f.q < k.q_far) {
-      if (!NEST || f.q < k.q_exp) near(f, r2, k, tab, g, h, z);
-      near_cb(g, z);
+    if (r2 < k.q_far) {
+      float gr = DIRECT ? f.g * k.t3 : f.g;
+      if (!NEST || r2 < k.q_exp) near(f, r2, k, tab, same, g, h, z, gr);
+      near_cb(gr, z);
     } else {
       far_cb(f.g);
     }
@@ -297,11 +328,11 @@ struct RegKernel<REG_GAUSSIAN> {
     eta = z;
   }
 
-  template <bool SELF = true>
+  template <class Same>
   static __device__ __forceinline__ void eval(float r2, const RegConsts& k, const float4* tab,
-                                              float& Kv, float& Kh, float& eta) {
+                                              Same&& same, float& Kv, float& Kh, float& eta) {
     float kf;
-    eval_ranges(r2, k, tab, Kv, Kh, eta, kf, [](float, float) {});
+    eval_ranges(r2, k, tab, same, Kv, Kh, eta, kf, [](float, float) {});
   }
 };
 

@@ -30,6 +30,7 @@ struct LaunchCfg {
 // FP64 epilogue scale factors.
 struct Scales {
   double vel = 0, dG = 0, dH = 0, visc = 0;
+  double near = 1;  // 3D gaussian: Kv / G, applied to the FP64 near sums of G
 };
 
 struct P3DJob {
@@ -149,8 +150,9 @@ LaunchCfg vort_default_cfg(int n_src, int n_tgt, int n_cu, bool sorted);
 hipError_t launch_relax(float4* a, const float* omega, int n, float fdt, hipStream_t s);
 
 // Host-side helpers.
-Scales p3d_scales(int reg, float sigma, float nu);
-RegConsts p3d_consts(int reg, float sigma, int mask, int acc);
+// direct: which form of the Gaussian pair (GaussianKernel).
+Scales p3d_scales(int reg, float sigma, float nu, bool direct);
+RegConsts p3d_consts(int reg, float sigma, int mask, int acc, bool direct);
 bool p3d_supported(int reg, int mask);
 bool p2d_supported(int reg, int mask);
 

@@ -41,7 +41,7 @@ __global__ __launch_bounds__(WG) void p3d_kernel(P3DKParams p) {
   }
   const int s0 = blockIdx.y * p.split_len;
   const int s1 = min(s0 + p.split_len, p.n_src);
-  p3d_block<REG, MASK, ACC, T, WG, Q>(p, p.rc, p.sc, blockIdx.x * (WG * T / Q), p.n_tgt, s0, s1,
+  p3d_block<REG, MASK, ACC, T, WG, Q == 1, Q>(p, p.rc, p.sc, blockIdx.x * (WG * T / Q), p.n_tgt, s0, s1,
                                       blockIdx.y, sm, &share);
 }
 
@@ -73,31 +73,46 @@ bool p3d_supported(int reg, int mask) {
   return true;
 }
 
-// Winckelmans: the exponent e for which sigma 2^e is in [1, 2) (0 for a radius
+// The exponent e for which sigma 2^e is in [1, 2) (0 for a radius
 // that is zero, infinite or NaN).
-static int winckelmans_exponent(float sigma) {
+static int radius_exponent(float sigma) {
   const double s = std::fabs((double)sigma);
   if (!(s > 0.0) || !std::isfinite(s)) return 0;
   return std::min(126, std::max(-126, -std::ilogb(s)));
 }
 
-RegConsts p3d_consts(int reg, float sigma, int mask, int acc) {
+RegConsts p3d_consts(int reg, float sigma, int mask, int acc, bool direct) {
   RegConsts k{};
   const double s = std::fabs((double)sigma);
   k.s2 = (float)(s * s);
   k.inv_s2 = (float)(1.0 / (s * s));
   if (reg == REG_GAUSSIAN) {
-    k.c1 = (float)(-0.5 / std::log(2.0));
+    k.xs = (float)std::ldexp(1.0, radius_exponent(sigma));
+    // (an infinite radius is scaled by 0 below, 0 and NaN give NaN there)
+    const double sx = std::isinf(s) || s == 0.0 ? 1.0 : s * (double)k.xs;
+    k.inv_s2 = (float)(1.0 / (sx * sx));
+    const double t = direct ? sx : 1.0, t2 = t * t;
+    k.c1 = (float)(-0.5 / (std::log(2.0) * t2));
     k.c2 = (float)std::sqrt(2.0 / M_PI);
+    k.g3 = (float)(1.0 / (t2 * t));
+    k.h5 = (float)(1.0 / (t2 * t2 * t));
+    k.t3 = (float)(t2 * t);
+    k.nt1 = (float)(-1.0 / t);
+    k.nt3 = (float)(-1.0 / (3.0 * t2 * t));
+    k.tp = (float)(GTAB_PER_UNIT / t);
     // Where no pair's FP64 sum and no zeta depends on it, the far form is taken
     // from where the near one rounds to it: 1 - rho zeta = 1 from rho^2 = 38 on,
     // and G - zeta/3 = G from 44 on.  Bit for bit the same results; velocity, us:
     // ring of 100000 4113 -> 4005, box of 50000 1401 -> 1193.
     if (mask == OUT_VEL) k.q_far = 40.f;
     else if (!(mask & OUT_VISC) && acc != ACC_COMP) k.q_far = k.q_exp;
+    // as limits of r^2 (in units of sigma^2 where not direct)
+    k.q_far = (float)(k.q_far * t2);
+    k.q_exp = (float)(k.q_exp * t2);
+    k.q_tab = (float)(k.q_tab * t2);
   }
   if (reg == REG_WINCKELMANS) {
-    k.xs = (float)std::ldexp(1.0, winckelmans_exponent(sigma));
+    k.xs = (float)std::ldexp(1.0, radius_exponent(sigma));
     const double t = s * (double)k.xs;
     // no field of a radius that is no length: 0 and NaN give NaN; an infinite
     // one is scaled by 0 below
@@ -108,23 +123,29 @@ RegConsts p3d_consts(int reg, float sigma, int mask, int acc) {
   return k;
 }
 
-Scales p3d_scales(int reg, float sigma, float nu) {
+Scales p3d_scales(int reg, float sigma, float nu, bool direct) {
   Scales sc;
   const double s = std::fabs((double)sigma);
   const double sgn = sigma < 0 ? -1.0 : 1.0;
   const double k4pi = 1.0 / (4.0 * M_PI);
   const double s3 = s * s * s, s5 = s3 * s * s;
   switch (reg) {
-    case REG_GAUSSIAN:
-      sc.vel = -k4pi / s3;
-      sc.dG = sgn * k4pi / s3;
-      sc.dH = 3.0 * sgn * k4pi / s5;
-      sc.visc = 2.0 * (double)nu / (s * s);
+    case REG_GAUSSIAN: {
+      // as for Winckelmans below
+      const double x = std::ldexp(1.0, radius_exponent(sigma)), t = std::isinf(s) ? 1.0 : s * x;
+      const double on = std::isinf(s) ? 0.0 : (s == 0.0 ? std::nan("") : 1.0);
+      const double f = direct ? 1.0 : 1.0 / (t * t * t);
+      sc.vel = -k4pi * x * x * on * f;
+      sc.dG = sgn * k4pi * x * x * x * on * f;
+      sc.dH = 3.0 * sc.dG * (direct ? 1.0 : 1.0 / (t * t));
+      sc.near = direct ? 1.0 / (t * t * t) : 1.0;
+      sc.visc = on * (2.0 * (double)nu / (s * s));
       break;
+    }
     case REG_WINCKELMANS: {
       // in positions multiplied by x: Kv is x^-3 of the dimensional one, each
       // position factor x
-      const double x = std::ldexp(1.0, winckelmans_exponent(sigma)), t = s * x;
+      const double x = std::ldexp(1.0, radius_exponent(sigma)), t = s * x;
       const double on = std::isinf(s) ? 0.0 : 1.0;
       sc.vel = -k4pi * x * x * on;
       sc.dG = sgn * k4pi * x * x * x * on;
@@ -246,8 +267,8 @@ hipError_t launch_p3d(const P3DJob& j, const LaunchCfg& c, hipStream_t s) {
   p.tgt_perm = j.tgt_perm;
   p.n_src = j.n_src;
   p.n_tgt = j.n_tgt;
-  p.rc = p3d_consts(j.reg, j.sigma, j.mask, j.acc);
-  p.sc = p3d_scales(j.reg, j.sigma, j.nu);
+  p.rc = p3d_consts(j.reg, j.sigma, j.mask, j.acc, c.q == 1);
+  p.sc = p3d_scales(j.reg, j.sigma, j.nu, c.q == 1);
 
   int n_split = c.n_split;
   int split_len = c.split_len;

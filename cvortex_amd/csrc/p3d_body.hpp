@@ -37,7 +37,8 @@ struct P3DLayout {
 // inside the regularisation's near branch; the stretching terms of the
 // pairs beyond (Kv < 208^-3/2 in reduced units, and eta = 0 there) are
 // summed in FP32 tiles combined by TwoSum, in the F_A slots, on the far
-// branch (RegKernel<REG_GAUSSIAN>::eval_split).
+// branch (GaussianKernel::eval_split).  The near sum is of G itself,
+// the far one of Kv: Scales::near is the factor between them.
 template <int REG, int MASK, int ACC>
 struct P3DRegs {
   static constexpr bool DBL = (ACC == ACC_COMP);
@@ -76,7 +77,7 @@ struct P3DKParams {
 // repeats the tile with SELF_TEST (see p3d_block).
 enum SelfMode : int { SELF_NONE, SELF_TEST, SELF_WATCH };
 
-template <int REG, int MASK, int ACC, int SELF, bool NEST>
+template <int REG, int MASK, int ACC, int SELF, bool DIRECT>
 __device__ __forceinline__ void p3d_pair(const float4 sp, const float4 sa, const double2* pxy,
                                          const double2* pzv, const float3 xt, const float3 at,
                                          const RegConsts& rc, const float4* tab, float* acc,
@@ -85,20 +86,26 @@ __device__ __forceinline__ void p3d_pair(const float4 sp, const float4 sa, const
   const float dx = xt.x - sp.x;
   const float dy = xt.y - sp.y;
   const float dz = xt.z - sp.z;
-  const float r2 = __builtin_fmaf(
-      dx, dx, __builtin_fmaf(dy, dy, REG == REG_WINCKELMANS ? __builtin_fmaf(dz, dz, rc.s2) : dz * dz));
+  const float z2 = REG == REG_WINCKELMANS ? __builtin_fmaf(dz, dz, rc.s2)
+                   : REG == REG_GAUSSIAN && DIRECT ? __builtin_fmaf(dz, dz, 1e-30f)
+                                                   : dz * dz;
+  const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, z2));
+  auto same_place = [&] {
+    if constexpr (REG == REG_GAUSSIAN && !DIRECT) return r2 == 0.f;
+    return (__float_as_uint(dx) | __float_as_uint(dy) | __float_as_uint(dz)) == 0u;
+  };
   float Kv, Kh, eta, Kfar = 0.f;
   if constexpr (REG == REG_WINCKELMANS) {
     RegKernel<REG_WINCKELMANS>::eval(r2, rc, Kv, Kh, eta);
     if constexpr (SELF == SELF_WATCH) smin = fminf(smin, r2);
     if constexpr (SELF == SELF_TEST) {
-      const bool same = (__float_as_uint(dx) | __float_as_uint(dy) | __float_as_uint(dz)) == 0u;
+      const bool same = same_place();
       Kv = same ? 0.f : Kv;
       eta = same ? 0.f : eta;
     }
   } else if constexpr (R::SPLIT && (MASK & OUT_DVORT) != 0) {
-    RegKernel<REG_GAUSSIAN>::template eval_split<NEST && (MASK & OUT_VISC) == 0>(
-        r2, rc, tab, Kv, Kh, eta, [&](float kn, float en) {
+    GaussianKernel<DIRECT>::template eval_split<DIRECT && (MASK & OUT_VISC) == 0>(
+        r2, rc, tab, same_place, Kv, Kh, eta, [&](float kn, float en) {
       const double2 sxy = *pxy, szv = *pzv;
       const double k = (double)kn;
       dacc[R::D_A + 0] = __builtin_fma(k, sxy.x, dacc[R::D_A + 0]);
@@ -118,7 +125,7 @@ __device__ __forceinline__ void p3d_pair(const float4 sp, const float4 sa, const
     });
   } else if constexpr (R::SPLIT) {
     constexpr bool PIN = (MASK & (OUT_DVORT | OUT_VISC)) == 0;  // no FP64 near sums
-    RegKernel<REG_GAUSSIAN>::template eval_ranges<PIN>(r2, rc, tab, Kv, Kh, eta, Kfar,
+    GaussianKernel<DIRECT>::template eval_ranges<PIN>(r2, rc, tab, same_place, Kv, Kh, eta, Kfar,
                                                        [&](float kn, float en) {
       // FP64 source strengths are read from LDS here, on the rare path (a
       // conversion of sa would be speculated out of the branch)
@@ -137,6 +144,8 @@ __device__ __forceinline__ void p3d_pair(const float4 sp, const float4 sa, const
         dacc[R::D_E + 3] = __builtin_fma(e, szv.y, dacc[R::D_E + 3]);
       }
     });
+  } else if constexpr (REG == REG_GAUSSIAN) {
+    GaussianKernel<DIRECT>::eval(r2, rc, tab, same_place, Kv, Kh, eta);
   } else {
     RegKernel<REG>::template eval<(MASK & (OUT_DVORT | OUT_VISC)) != 0>(r2, rc, tab, Kv, Kh, eta);
   }
@@ -247,7 +256,8 @@ struct P3DShare {
 // sums are added in FP64 at the end (see narrow_cfg).  Writes the outputs
 // (n_split == 1) or the FP64 partials of partition `split`.  The caller has loaded sm.tab (Gaussian)
 // and issues no barrier-sensitive work on sm around the call.
-template <int REG, int MASK, int ACC, int T, int WG, int Q = 1>
+// DIRECT: which form of the Gaussian pair (GaussianKernel).
+template <int REG, int MASK, int ACC, int T, int WG, bool DIRECT, int Q = 1>
 __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& rc,
                                           const Scales& sc, int base, int tgt_end, int s0,
                                           int s1, int split, P3DSmem<REG, MASK, ACC, WG>& sm,
@@ -257,6 +267,7 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
   using R = P3DRegs<REG, MASK, ACC>;
   constexpr int NF = R::NF;
   constexpr int ND = R::ND > 0 ? R::ND : 1;
+  constexpr bool SCALED = REG == REG_WINCKELMANS || REG == REG_GAUSSIAN;  // RegConsts::xs
   constexpr bool DBL_ = P3DSmem<REG, MASK, ACC, WG>::DBL;
   const int tid = threadIdx.x;
   const int tl = Q == 1 ? tid : tid & 63;  // target within the group
@@ -268,8 +279,7 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
     i = i < tgt_end ? i : tgt_end - 1;
     if (p.tgt_perm) i = p.tgt_perm[i];
     const float4 q = p.tgt_pv[i];
-    xt[k] = REG == REG_WINCKELMANS ? make_float3(q.x * rc.xs, q.y * rc.xs, q.z * rc.xs)
-                                   : make_float3(q.x, q.y, q.z);
+    xt[k] = SCALED ? make_float3(q.x * rc.xs, q.y * rc.xs, q.z * rc.xs) : make_float3(q.x, q.y, q.z);
     vt[k] = q.w;
     if constexpr (L::NEED_TA) {
       const float4 w = p.tgt_a[i];
@@ -299,7 +309,7 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
     if (tid < cnt) {
       float4 q = p.src_pv[ts + tid];
       const float4 w = p.src_a[ts + tid];
-      if constexpr (REG == REG_WINCKELMANS) {
+      if constexpr (SCALED) {
         q.x *= rc.xs;
         q.y *= rc.xs;
         q.z *= rc.xs;
@@ -344,7 +354,7 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
         const float4 sa = make_float4(xa.w, tl.x, tl.y, 0.f);
 #pragma unroll
         for (int k = 0; k < T; ++k)
-          p3d_pair<REG, MASK, ACC, decltype(mode)::value, Q == 1>(sp, sa, &sm.xy[DBL_ ? jv : 0],
+          p3d_pair<REG, MASK, ACC, decltype(mode)::value, DIRECT>(sp, sa, &sm.xy[DBL_ ? jv : 0],
                                                           &sm.zv[DBL_ ? jv : 0], xt[k], at[k], rv,
                                                           sm.tab, acc[k], dacc[k], smin);
       }
@@ -403,7 +413,7 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         if constexpr (R::SPLIT)
-          d[L::A + c] = dacc[k][R::D_A + c] + fval(R::F_A + c);
+          d[L::A + c] = sc.near * dacc[k][R::D_A + c] + fval(R::F_A + c);
         else
           d[L::A + c] = R::DBL ? dacc[k][R::D_A + c] : fval(R::F_A + c);
         d[L::H + c] = fval(R::F_H + c);
