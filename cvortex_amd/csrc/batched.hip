@@ -5,7 +5,8 @@
 // cloud c owns particles [begin_c, end_c) and its own regularisation radius.
 // Each cloud interacts only with itself (sources = targets = the cloud).
 //
-// Work units are (cloud, block of WG*T targets), sorted by cost (cloud size)
+// Work units are (cloud, block of WG*T targets, or of 64 that the four waves
+// of a workgroup share: see batch_default_shape), sorted by cost (cloud size)
 // in decreasing order -- the longest-processing-time-first rule -- so that
 // the 64x spread of cloud sizes (1024 .. 65536 particles) leaves no long
 // tail.  A persistent grid of a few workgroups per CU pulls units from a
@@ -51,9 +52,10 @@ __global__ void batch_reset_counter(unsigned int* counter) {
   if (threadIdx.x == 0 && blockIdx.x == 0) counter[0] = 0u;
 }
 
-template <int REG, int MASK, int ACC, int T, int WG>
+template <int REG, int MASK, int ACC, int T, int WG, int Q = 1>
 __global__ __launch_bounds__(WG) void p3d_batched_kernel(BatchParams bp) {
   __shared__ P3DSmem<REG, MASK, ACC, WG> sm;
+  __shared__ P3DShare<MASK, Q> share;
   __shared__ int s_unit;
   if constexpr (REG == REG_GAUSSIAN) {
     for (int i = threadIdx.x; i < 2 * GTAB_N; i += WG) sm.tab[i] = bp.base.gtab[i];
@@ -66,7 +68,8 @@ __global__ __launch_bounds__(WG) void p3d_batched_kernel(BatchParams bp) {
     if (u >= bp.n_units) break;  // uniform over the workgroup
     const int2 un = bp.units[u];
     const int2 r = bp.range[un.x];
-    p3d_block<REG, MASK, ACC, T, WG, false>(bp.base, bp.rc[un.x], bp.sc[un.x], un.y, r.y, r.x, r.y, 0, sm);
+    p3d_block<REG, MASK, ACC, T, WG, false, Q>(bp.base, bp.rc[un.x], bp.sc[un.x], un.y, r.y, r.x,
+                                               r.y, 0, sm, &share);
   }
 }
 
@@ -128,26 +131,28 @@ BFn b_T(int T) {
   }
 }
 template <int REG, int MASK, int ACC>
-BFn b_wg(int wg, int T) {
+BFn b_wg(int wg, int T, int q) {
+  if (q == 4) return p3d_batched_kernel<REG, MASK, ACC, 1, 256, 4>;
   return wg == 128 ? b_T<REG, MASK, ACC, 128>(T) : b_T<REG, MASK, ACC, 256>(T);
 }
 template <int REG, int MASK>
-BFn b_acc(int acc, int wg, int T) {
-  if (acc == ACC_PLAIN) return b_wg<REG, MASK, ACC_PLAIN>(wg, T);
-  if (acc == ACC_TILES) return b_wg<REG, MASK, ACC_TILES>(wg, T);
-  return b_wg<REG, MASK, ACC_COMP>(wg, T);
+BFn b_acc(int acc, int wg, int T, int q) {
+  if (acc == ACC_PLAIN) return b_wg<REG, MASK, ACC_PLAIN>(wg, T, q);
+  if (acc == ACC_TILES) return b_wg<REG, MASK, ACC_TILES>(wg, T, q);
+  return b_wg<REG, MASK, ACC_COMP>(wg, T, q);
 }
 template <int REG>
-BFn b_mask(int mask, int wg, int T, int acc) {
-  if (mask == (OUT_VEL | OUT_DVORT)) return b_acc<REG, OUT_VEL | OUT_DVORT>(acc, wg, T);
+BFn b_mask(int mask, int wg, int T, int q, int acc) {
+  if (mask == (OUT_VEL | OUT_DVORT)) return b_acc<REG, OUT_VEL | OUT_DVORT>(acc, wg, T, q);
   if (mask == (OUT_VEL | OUT_DVORT | OUT_VISC))
-    return b_acc<REG, OUT_VEL | OUT_DVORT | OUT_VISC>(acc, wg, T);
+    return b_acc<REG, OUT_VEL | OUT_DVORT | OUT_VISC>(acc, wg, T, q);
   return nullptr;
 }
-BFn b_pick(int reg, int mask, int acc, int wg, int T) {
+BFn b_pick(int reg, int mask, int acc, int wg, int T, int q) {
   if (wg != 128 && wg != 256) return nullptr;
-  if (reg == REG_WINCKELMANS) return b_mask<REG_WINCKELMANS>(mask, wg, T, acc);
-  if (reg == REG_GAUSSIAN) return b_mask<REG_GAUSSIAN>(mask, wg, T, acc);
+  if (q != 1 && (q != 4 || wg != 256 || T != 1)) return nullptr;
+  if (reg == REG_WINCKELMANS) return b_mask<REG_WINCKELMANS>(mask, wg, T, q, acc);
+  if (reg == REG_GAUSSIAN) return b_mask<REG_GAUSSIAN>(mask, wg, T, q, acc);
   return nullptr;
 }
 
@@ -168,6 +173,7 @@ struct cvtx_hip_batch {
   float nu = 0.f;
   int T = 2;
   int wg = 256;  // workgroup size = source tile length
+  int q = 1;     // waves that share a group of 64 targets (4: T = 1, wg = 256)
   int wpc = 4;   // resident workgroups per CU of the persistent grid
   int n_units = 0;
   int grid = 0;
@@ -235,8 +241,8 @@ bool batch_live(Runtime& rt, const cvtx_hip_batch* b) {
   return true;
 }
 
-bool build_units(cvtx_hip_batch* b, int T, int wg) {
-  const int per = wg * T;
+bool build_units(cvtx_hip_batch* b, int T, int wg, int q = 1) {
+  const int per = wg * T / q;
   std::vector<int> order(b->n_clouds);
   std::iota(order.begin(), order.end(), 0);
   std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
@@ -248,6 +254,7 @@ bool build_units(cvtx_hip_batch* b, int T, int wg) {
   b->n_units = (int)units.size();
   b->T = T;
   b->wg = wg;
+  b->q = q;
   if (b->d_units) (void)hipFree(b->d_units);
   b->d_units = nullptr;
   if (units.empty()) return true;
@@ -277,7 +284,7 @@ P3DKParams base_params(cvtx_hip_batch* b, const float* pv, const float* a, float
 hipError_t enqueue_eval(cvtx_hip_batch* b, const float* pv, const float* a, float* vel,
                         float* dvort, float* visc, hipStream_t s) {
   if (b->n_units == 0) return hipSuccess;
-  BFn k = b_pick(b->reg, b->mask, b->acc, b->wg, b->T);
+  BFn k = b_pick(b->reg, b->mask, b->acc, b->wg, b->T, b->q);
   if (!k) return hipErrorInvalidValue;
   BatchParams bp{};
   bp.base = base_params(b, pv, a, vel, dvort, visc);
@@ -310,6 +317,32 @@ BatchSignature batch_signature(const cvtx_hip_batch* b) {
   g.pairs = pairs;
   g.n_clouds = b->n_clouds;
   return g;
+}
+
+// The shape of a batch that was not tuned: one target per lane, and below a
+// number of groups of 64 targets per CU 64 targets per workgroup, shared by its
+// four waves.  A unit's targets meet its whole cloud, so the longest unit bounds
+// a batch of few targets, whose units do not fill the chip: with two targets per
+// lane a cloud of 9000 is 18 workgroups that each walk 18000 pairs per lane, here
+// 141 that walk 2250.  With many units the staging of a tile per 64 targets costs
+// more than the last units' unevenness.  ms, two targets per lane -> one -> 64
+// targets per workgroup, by groups per CU: Winckelmans (FP32 tiles) 0.6: 0.47 ->
+// 0.28 -> 0.09, 5: 1.09 -> 0.75 -> 0.42, 25: 10.9 -> 6.2 -> 4.7, 52: 13.2 -> 9.9 ->
+// 9.6, 61: 29.6 -> 23.8 -> 23.6, 105: 33.4 -> 29.0 -> 31.2, 121 (2 10^6 particles)
+// 49.4 -> 43.5 -> 47.5, 486: 182.3 -> 172.7 -> 190.0; Gaussian (5 and 6 resident
+// workgroups per CU) 0.6: 1.30 -> 0.73 -> 0.20, 25: 16.3 -> 10.0 -> 6.7, 61: 46.3 ->
+// 36.8 -> 35.1, 105: 48.1 -> 45.8 -> 46.1, 121: 72.3 -> 70.2 -> 70.6, 486: 277.9 ->
+// 273.3 -> 279.8.
+BatchShape batch_default_shape(const cvtx_hip_batch* b) {
+  long long groups = 0;
+  for (int c = 0; c < b->n_clouds; ++c) groups += (b->end[c] - b->begin[c] + 63) / 64;
+  const bool gauss = b->reg == REG_GAUSSIAN;
+  BatchShape s{1, 256, gauss ? 5 : 4, 0.f};
+  if (groups < (gauss ? 100LL : 60LL) * std::max(1, b->dev->n_cu)) {
+    s.q = 4;
+    s.wpc = gauss ? 6 : 4;
+  }
+  return s;
 }
 
 }  // namespace
@@ -374,12 +407,11 @@ cvtx_hip_batch* cvtx_hip_batch_create(int n_clouds, const int* offsets, const fl
     ok = ok && hipMemcpy(b->d_rc, rc.data(), sizeof(RegConsts) * n_clouds, hipMemcpyHostToDevice) == hipSuccess;
     ok = ok && hipMemcpy(b->d_sc, sc.data(), sizeof(Scales) * n_clouds, hipMemcpyHostToDevice) == hipSuccess;
   }
-  // the autotuner's shape for this batch's signature, if one is cached;
-  // else two targets per lane, 256-wide workgroups, 4 resident per CU
-  BatchShape shp{2, 256, 4, 0.f};
+  // the autotuner's shape for this batch's signature, if one is cached
+  BatchShape shp = batch_default_shape(b);
   (void)batch_shape_lookup(batch_signature(b), &shp);
   b->wpc = shp.wpc;
-  ok = ok && build_units(b, shp.T, shp.wg);
+  ok = ok && build_units(b, shp.T, shp.wg, shp.q);
   // a few resident workgroups per CU; the loop exits when the units run out
   b->grid = std::max(1, std::min(b->n_units, b->wpc * std::max(1, d->n_cu)));
   if (!ok) {
@@ -565,7 +597,8 @@ int cvtx_hip_batch_rk4_step(cvtx_hip_batch* b, int n_steps, void* stream) {
 
 // Times the persistent launch of this batch (its outputs are overwritten)
 // for every candidate shape -- targets per lane {1, 2, 4} x workgroup size
-// {128, 256} x resident workgroups per CU {2, 4, 8} -- with HIP events on
+// {128, 256}, or 64 targets per workgroup of 256, x resident workgroups per CU
+// {2, 4, 8} -- with HIP events on
 // the library's stream, keeps the fastest, and records it in the shape cache
 // under the batch's signature, so later batches of the same signature start
 // with it.  Returns 0 and the winner, or -1.
@@ -586,37 +619,36 @@ int cvtx_hip_batch_autotune(cvtx_hip_batch* b, const float* pv, const float* a, 
     if (e0) (void)hipEventDestroy(e0);
     return -1;
   }
-  BatchShape best{b->T, b->wg, b->wpc, -1.f};
+  BatchShape best{b->T, b->wg, b->wpc, -1.f, b->q};
   bool ok = true;
-  for (int wg : {128, 256}) {
-    for (int T : {1, 2, 4}) {
-      if (!build_units(b, T, wg)) {
-        ok = false;
-        break;
-      }
-      for (int wpc : {2, 4, 8}) {
-        b->grid = std::max(1, std::min(b->n_units, wpc * std::max(1, b->dev->n_cu)));
-        float ms = -1.f;
-        if (enqueue_eval(b, pv, a, vel, dvort, visc, s) == hipSuccess &&  // warm-up
-            hipEventRecord(e0, s) == hipSuccess) {
-          bool run = true;
-          for (int r = 0; r < reps && run; ++r)
-            run = enqueue_eval(b, pv, a, vel, dvort, visc, s) == hipSuccess;
-          if (run && hipEventRecord(e1, s) == hipSuccess && hipEventSynchronize(e1) == hipSuccess &&
-              hipEventElapsedTime(&ms, e0, e1) == hipSuccess)
-            ms /= (float)reps;
-          else
-            ms = -1.f;
-        }
-        if (ms > 0.f && (best.ms < 0.f || ms < best.ms)) best = BatchShape{T, wg, wpc, ms};
-      }
+  const BatchShape tried[] = {{1, 128, 0, 0.f}, {2, 128, 0, 0.f}, {4, 128, 0, 0.f}, {1, 256, 0, 0.f},
+                              {2, 256, 0, 0.f}, {4, 256, 0, 0.f}, {1, 256, 0, 0.f, 4}};
+  for (const BatchShape& c : tried) {
+    if (!build_units(b, c.T, c.wg, c.q)) {
+      ok = false;
+      break;
     }
-    if (!ok) break;
+    for (int wpc : {2, 4, 8}) {
+      b->grid = std::max(1, std::min(b->n_units, wpc * std::max(1, b->dev->n_cu)));
+      float ms = -1.f;
+      if (enqueue_eval(b, pv, a, vel, dvort, visc, s) == hipSuccess &&  // warm-up
+          hipEventRecord(e0, s) == hipSuccess) {
+        bool run = true;
+        for (int r = 0; r < reps && run; ++r)
+          run = enqueue_eval(b, pv, a, vel, dvort, visc, s) == hipSuccess;
+        if (run && hipEventRecord(e1, s) == hipSuccess && hipEventSynchronize(e1) == hipSuccess &&
+            hipEventElapsedTime(&ms, e0, e1) == hipSuccess)
+          ms /= (float)reps;
+        else
+          ms = -1.f;
+      }
+      if (ms > 0.f && (best.ms < 0.f || ms < best.ms)) best = BatchShape{c.T, c.wg, wpc, ms, c.q};
+    }
   }
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
   // leave the batch in the winning shape (or its previous one)
-  if (!build_units(b, best.T, best.wg)) {
+  if (!build_units(b, best.T, best.wg, best.q)) {
     set_error(rt, "batch autotune: allocation failed");
     return -1;
   }

@@ -302,6 +302,7 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
   }
 
   const RegConsts rv = loop_consts(rc);
+  const bool one_array = p.src_pv == p.tgt_pv && p.tgt_perm == nullptr;
   for (int ts = s0; ts < s1; ts += WG) {
     const int cnt = min(WG, s1 - ts);
     const int part = wave_part<Q>(cnt, tid), end = wave_part_end<Q>(cnt, part);
@@ -372,19 +373,24 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
     // 141.0; velocity of 100000 (S alone) 4.38 -> 4.06.
     constexpr bool WATCH = Q == 1 && REG == REG_WINCKELMANS && ACC != ACC_PLAIN && (MASK & (OUT_DVORT | OUT_VISC)) != 0;
     if constexpr (WATCH) {
-      double before[T][ND];
-#pragma unroll
-      for (int k = 0; k < T; ++k)
-#pragma unroll
-        for (int a = 0; a < ND; ++a) before[k][a] = dacc[k][a];
-      tile(std::integral_constant<int, SELF_WATCH>());
-      if (__any(smin <= rc.s2)) {
+      // (a block's own tiles, where sources and targets are one array, are known)
+      bool test = one_array && ts < base + T * WG && ts + cnt > base;
+      if (!test) {
+        double before[T][ND];
 #pragma unroll
         for (int k = 0; k < T; ++k)
 #pragma unroll
-          for (int a = 0; a < ND; ++a) dacc[k][a] = before[k][a];
-        tile(std::integral_constant<int, SELF_TEST>());
+          for (int a = 0; a < ND; ++a) before[k][a] = dacc[k][a];
+        tile(std::integral_constant<int, SELF_WATCH>());
+        if (__any(smin <= rc.s2)) {
+          test = true;
+#pragma unroll
+          for (int k = 0; k < T; ++k)
+#pragma unroll
+            for (int a = 0; a < ND; ++a) dacc[k][a] = before[k][a];
+        }
       }
+      if (test) tile(std::integral_constant<int, SELF_TEST>());
     } else {
       tile(std::integral_constant<int, MASK == OUT_VEL ? SELF_NONE : SELF_TEST>());
     }

@@ -8,7 +8,8 @@
 // The cache can be saved to and loaded from a small text file, one entry
 // per line: "kind reg mask acc bucket_src bucket_tgt T n_split ms wg" (kind 3:
 // a multi-cloud batch, keyed by its pair count and cloud count; n_split is
-// then the resident workgroups per CU).
+// then the resident workgroups per CU), and a last column 4 for the variant
+// with 64 targets per workgroup (LaunchCfg::q).
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
@@ -36,6 +37,7 @@ struct Entry {
   int n_split;
   float ms;
   int wg = 256;
+  int q = 1;
 };
 
 std::map<Key, Entry>& cache() {
@@ -171,8 +173,10 @@ LaunchCfg p2d_cfg(int reg, int mask, int n_src, int n_tgt, int cus) {
 LaunchCfg choose_cfg(int kind, int reg, int mask, int acc, int n_src, int n_tgt, int n_cu) {
   auto it = cache().find(Key{ordered_kind(kind, reg, n_src, n_tgt), reg, mask, acc,
                              size_bucket(n_src), size_bucket(n_tgt)});
-  if (it != cache().end()) return launch_shape(it->second.T, it->second.n_split, n_src);
   const int cus = n_cu > 0 ? n_cu : 256;
+  if (it != cache().end())
+    return it->second.q == 4 ? narrow_cfg(kind, reg, mask, n_src, n_tgt, cus)
+                             : launch_shape(it->second.T, it->second.n_split, n_src);
   // Spatially ordered targets (Gaussian P3D, compensated sums).  One target
   // per lane: a 64-target wave of Morton-ordered targets is more compact
   // than a 128-target one, so fewer of its source rounds take the FP64
@@ -244,12 +248,12 @@ Key batch_key(const BatchSignature& g) {
 bool batch_shape_lookup(const BatchSignature& g, BatchShape* out) {
   auto it = cache().find(batch_key(g));
   if (it == cache().end()) return false;
-  *out = BatchShape{it->second.T, it->second.wg, it->second.n_split, it->second.ms};
+  *out = BatchShape{it->second.T, it->second.wg, it->second.n_split, it->second.ms, it->second.q};
   return true;
 }
 
 void batch_shape_record(const BatchSignature& g, const BatchShape& s) {
-  cache()[batch_key(g)] = Entry{s.T, s.wpc, s.ms, s.wg};
+  cache()[batch_key(g)] = Entry{s.T, s.wpc, s.ms, s.wg, s.q};
 }
 
 }  // namespace cvtx
@@ -335,7 +339,10 @@ int cvtx_hip_autotune_p3d(const cvtx_hip_p3d_problem* p, int reps, int* best_T, 
   }
   float best = -1.f;
   LaunchCfg win;
-  for (const LaunchCfg& c : candidates(j.n_src, j.n_tgt, d->n_cu)) {
+  std::vector<LaunchCfg> shapes = candidates(j.n_src, j.n_tgt, d->n_cu);
+  if (!j.tgt_perm && narrow(KIND_P3D, j.reg, j.mask, j.n_src, j.n_tgt, d->n_cu))
+    shapes.push_back(narrow_cfg(KIND_P3D, j.reg, j.mask, j.n_src, j.n_tgt, d->n_cu));
+  for (const LaunchCfg& c : shapes) {
     P3DJob jj = j;
     const size_t wb = p3d_workspace_bytes(jj, c);
     if (wb) {
@@ -350,7 +357,7 @@ int cvtx_hip_autotune_p3d(const cvtx_hip_p3d_problem* p, int reps, int* best_T, 
   }
   if (best < 0.f) return -1;
   cache()[Key{ordered_kind(KIND_P3D, j.reg, j.n_src, j.n_tgt), j.reg, j.mask, j.acc,
-              size_bucket(j.n_src), size_bucket(j.n_tgt)}] = Entry{win.T, win.n_split, best};
+              size_bucket(j.n_src), size_bucket(j.n_tgt)}] = Entry{win.T, win.n_split, best, 256, win.q};
   if (best_T) *best_T = win.T;
   if (best_split) *best_split = win.n_split;
   if (best_ms) *best_ms = best;
@@ -362,9 +369,9 @@ int cvtx_hip_tune_save(const char* path) {
   if (!f) return -1;
   for (auto& kv : cache()) {
     const Key& k = kv.first;
-    std::fprintf(f, "%d %d %d %d %d %d %d %d %.6f %d\n", std::get<0>(k), std::get<1>(k),
+    std::fprintf(f, "%d %d %d %d %d %d %d %d %.6f %d%s\n", std::get<0>(k), std::get<1>(k),
                  std::get<2>(k), std::get<3>(k), std::get<4>(k), std::get<5>(k), kv.second.T,
-                 kv.second.n_split, kv.second.ms, kv.second.wg);
+                 kv.second.n_split, kv.second.ms, kv.second.wg, kv.second.q == 4 ? " 4" : "");
   }
   std::fclose(f);
   return 0;
@@ -373,17 +380,19 @@ int cvtx_hip_tune_save(const char* path) {
 int cvtx_hip_tune_load(const char* path) {
   FILE* f = std::fopen(path, "r");
   if (!f) return -1;
-  int kind, reg, mask, acc, bs, bt, T, ns, wg;
+  int kind, reg, mask, acc, bs, bt, T, ns, wg, q;
   float ms;
   int n = 0;
   char line[256];
-  // one entry per line; the workgroup size column may be absent (256)
+  // one entry per line; the last two columns may be absent (256, 1)
   while (std::fgets(line, sizeof(line), f)) {
     wg = 256;
-    const int got = std::sscanf(line, "%d %d %d %d %d %d %d %d %f %d", &kind, &reg, &mask, &acc,
-                                &bs, &bt, &T, &ns, &ms, &wg);
+    q = 1;
+    const int got = std::sscanf(line, "%d %d %d %d %d %d %d %d %f %d %d", &kind, &reg, &mask, &acc,
+                                &bs, &bt, &T, &ns, &ms, &wg, &q);
     if (got >= 9 && (T == 1 || T == 2 || T == 4) && ns >= 1 && (wg == 128 || wg == 256)) {
-      cache()[Key{kind, reg, mask, acc, bs, bt}] = Entry{T, ns, ms, wg};
+      if (q != 4 || T != 1 || wg != 256) q = 1;
+      cache()[Key{kind, reg, mask, acc, bs, bt}] = Entry{T, ns, ms, wg, q};
       ++n;
     }
   }

@@ -33,6 +33,7 @@ struct BatchShape {
   int wg;   // workgroup size
   int wpc;  // resident workgroups per CU
   float ms;
+  int q = 1;  // LaunchCfg::q
 };
 bool batch_shape_lookup(const BatchSignature& g, BatchShape* out);
 void batch_shape_record(const BatchSignature& g, const BatchShape& s);

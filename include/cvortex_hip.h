@@ -320,7 +320,8 @@ int cvtx_hip_batch_info(const cvtx_hip_batch* batch, int* n_units, int* grid, in
 int cvtx_hip_batch_shape(const cvtx_hip_batch* batch, int* targets_per_lane, int* workgroup_size,
                          int* workgroups_per_cu);
 /* Autotuner of the persistent launch: times every candidate shape
- * (targets per lane {1, 2, 4} x workgroup size {128, 256} x resident
+ * (targets per lane {1, 2, 4} x workgroup size {128, 256}, or one target per
+ * lane shared by the four waves of a workgroup, x resident
  * workgroups per CU {2, 4, 8}; one warm-up and `reps` timed evaluations
  * each, on the library's stream; the outputs are overwritten), keeps the
  * fastest for this batch and records it in the shape cache under the
