@@ -109,6 +109,13 @@ bool d2h(Runtime& rt, Device& d, void* dst, const void* src, size_t bytes) {
   return check_hip(rt, hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, d.stream), "D2H copy");
 }
 
+bool stage(Runtime& rt, Device& d, void* dst, const void* src, size_t bytes, hipMemcpyKind kind) {
+  if (bytes == 0) return true;
+  const hipError_t e = bytes <= kStageMax ? launch_stage(dst, src, bytes, d.stream)
+                                          : hipMemcpyAsync(dst, src, bytes, kind, d.stream);
+  return check_hip(rt, e, kind == hipMemcpyHostToDevice ? "H2D copy" : "D2H copy");
+}
+
 void report_failure(const char* fn, float* out, long n) {
   std::fprintf(stderr, "cvortex: %s failed: %s (result set to NaN)\n", fn,
                runtime().last_error.c_str());
@@ -189,7 +196,8 @@ int p3d_host(const cvtx_P3D** src, int ns, const bsv_V3f* mes, const cvtx_P3D** 
   // the selected outputs side by side, so that one copy brings them back
   const int n_out = ((mask & OUT_VEL) ? 1 : 0) + ((mask & OUT_DVORT) ? 1 : 0) + ((mask & OUT_VISC) ? 1 : 0);
   float* h_outs = (float*)host_buffer(rt, *d, SLOT_OUT0, ob * n_out);
-  float* d_outs = (float*)device_buffer(rt, *d, SLOT_OUT0, ob * n_out);
+  const bool straight = ob * n_out <= kStraightMax;
+  float* d_outs = straight ? h_outs : (float*)device_buffer(rt, *d, SLOT_OUT0, ob * n_out);
   if (!h_outs || !d_outs) return -1;
   float* h_out[3] = {nullptr, nullptr, nullptr};
   float* d_out[3] = {nullptr, nullptr, nullptr};
@@ -207,7 +215,7 @@ int p3d_host(const cvtx_P3D** src, int ns, const bsv_V3f* mes, const cvtx_P3D** 
   } else {
     gather_p3d(ind, nt, h_tpv, h_ta);
   }
-  if (!h2d(rt, *d, d_in, h_in, sizeof(float4) * n4)) return -1;
+  if (!stage(rt, *d, d_in, h_in, sizeof(float4) * n4, hipMemcpyHostToDevice)) return -1;
 
   P3DJob j;
   j.src_pv = d_spv;
@@ -233,7 +241,7 @@ int p3d_host(const cvtx_P3D** src, int ns, const bsv_V3f* mes, const cvtx_P3D** 
   }
   if (!maybe_order(rt, *d, j, d->stream)) return -1;
   if (!check_hip(rt, launch_p3d(j, c, d->stream), "P3D kernel launch")) return -1;
-  if (!d2h(rt, *d, h_outs, d_outs, ob * n_out)) return -1;
+  if (!straight && !stage(rt, *d, h_outs, d_outs, ob * n_out, hipMemcpyDeviceToHost)) return -1;
   if (!check_hip(rt, hipStreamSynchronize(d->stream), "P3D kernels")) return -1;
   for (int o = 0; o < 3; ++o)
     if (d_out[o]) std::memcpy(user_out[o], h_out[o], ob);
@@ -262,7 +270,8 @@ int f3d_host(const cvtx_F3D** src, int nf, const bsv_V3f* mes, const cvtx_P3D** 
   float4* h_in = (float4*)host_buffer(rt, *d, SLOT_SRC0, sizeof(float4) * n4);
   float4* d_in = (float4*)device_buffer(rt, *d, SLOT_SRC0, sizeof(float4) * n4);
   float* h_outs = (float*)host_buffer(rt, *d, SLOT_OUT0, ob * n_out);
-  float* d_outs = (float*)device_buffer(rt, *d, SLOT_OUT0, ob * n_out);
+  const bool straight = ob * n_out <= kStraightMax;
+  float* d_outs = straight ? h_outs : (float*)device_buffer(rt, *d, SLOT_OUT0, ob * n_out);
   if (!h_in || !d_in || !h_outs || !d_outs) return -1;
   float4* h_fa = h_in;
   float4* h_fb = h_in + nf1;
@@ -287,7 +296,7 @@ int f3d_host(const cvtx_F3D** src, int nf, const bsv_V3f* mes, const cvtx_P3D** 
   } else {
     gather_p3d(ind, nt, h_tpv, h_ta);
   }
-  if (!h2d(rt, *d, d_in, h_in, sizeof(float4) * n4)) return -1;
+  if (!stage(rt, *d, d_in, h_in, sizeof(float4) * n4, hipMemcpyHostToDevice)) return -1;
   F3DJob j;
   j.fa = d_fa;
   j.fb = d_fb;
@@ -310,7 +319,7 @@ int f3d_host(const cvtx_F3D** src, int nf, const bsv_V3f* mes, const cvtx_P3D** 
     if (!j.tgt_perm) return -1;
   }
   if (!check_hip(rt, launch_f3d(j, c, d->stream), "F3D kernel launch")) return -1;
-  if (!d2h(rt, *d, h_outs, d_outs, ob * n_out)) return -1;
+  if (!straight && !stage(rt, *d, h_outs, d_outs, ob * n_out, hipMemcpyDeviceToHost)) return -1;
   if (!check_hip(rt, hipStreamSynchronize(d->stream), "F3D kernels")) return -1;
   for (int o = 0; o < 2; ++o)
     if (d_out[o]) std::memcpy(user_out[o], h_out[o], ob);
@@ -352,7 +361,8 @@ int p2d_host(const cvtx_P2D** src, int ns, const bsv_V2f* mes, const cvtx_P2D** 
   float4* h_in = (float4*)host_buffer(rt, *d, SLOT_SRC0, sizeof(float4) * n4);
   float4* d_in = (float4*)device_buffer(rt, *d, SLOT_SRC0, sizeof(float4) * n4);
   float* h_outs = (float*)host_buffer(rt, *d, SLOT_OUT0, vb + eb);
-  float* d_outs = (float*)device_buffer(rt, *d, SLOT_OUT0, vb + eb);
+  const bool straight = vb + eb <= kStraightMax;
+  float* d_outs = straight ? h_outs : (float*)device_buffer(rt, *d, SLOT_OUT0, vb + eb);
   if (!h_in || !d_in || !h_outs || !d_outs) return -1;
   float4* h_s = h_in;
   float4* h_t = h_in + ns1;
@@ -368,7 +378,7 @@ int p2d_host(const cvtx_P2D** src, int ns, const bsv_V2f* mes, const cvtx_P2D** 
   } else {
     gather_p2d(ind, nt, h_t);
   }
-  if (!h2d(rt, *d, d_in, h_in, sizeof(float4) * n4)) return -1;
+  if (!stage(rt, *d, d_in, h_in, sizeof(float4) * n4, hipMemcpyHostToDevice)) return -1;
   P2DJob j;
   j.src = d_s;
   j.n_src = ns;
@@ -388,7 +398,7 @@ int p2d_host(const cvtx_P2D** src, int ns, const bsv_V2f* mes, const cvtx_P2D** 
     if (!j.partial) return -1;
   }
   if (!check_hip(rt, launch_p2d(j, c, d->stream), "P2D kernel launch")) return -1;
-  if (!d2h(rt, *d, h_outs, d_outs, vb + eb)) return -1;
+  if (!straight && !stage(rt, *d, h_outs, d_outs, vb + eb, hipMemcpyDeviceToHost)) return -1;
   if (!check_hip(rt, hipStreamSynchronize(d->stream), "P2D kernels")) return -1;
   if (d_v) std::memcpy(vel, h_v, vb);
   if (d_e) std::memcpy(visc, h_e, eb);

@@ -160,6 +160,11 @@ bool p2d_supported(int reg, int mask);
 // computed in FP64 on the host.
 void build_gaussian_table(float* out /* 8*GTAB_N floats */);
 
+// Copy of at most kStageMax bytes, a multiple of 4, between pinned host memory and
+// the device (stage.hip); both 16-byte aligned.  Larger ones go through HIP.
+constexpr size_t kStageMax = (size_t)1 << 20;
+hipError_t launch_stage(void* dst, const void* src, size_t bytes, hipStream_t s);
+
 // Spatial (Morton) order of n points: perm[i] = index of the i-th point.
 // Workspace: target_order_workspace(n) bytes (device).
 size_t target_order_workspace(int n);

@@ -93,13 +93,13 @@ int cvtx::vort_host(const cvtx_P3D** src, int ns, const bsv_V3f* mes, int nt, fl
   if (!h_spv || !h_sa || !h_t || !h_out || !d_spv || !d_sa || !d_t || !d_out) return -1;
   gather_p3d(src, ns, h_spv, h_sa);
   gather_pts3(mes, nt, h_t);
-  if (!h2d(rt, *d, d_spv, h_spv, sizeof(float4) * (size_t)ns)) return -1;
-  if (!h2d(rt, *d, d_sa, h_sa, sizeof(float4) * (size_t)ns)) return -1;
-  if (!h2d(rt, *d, d_t, h_t, tb)) return -1;
+  if (!stage(rt, *d, d_spv, h_spv, sizeof(float4) * (size_t)ns, hipMemcpyHostToDevice)) return -1;
+  if (!stage(rt, *d, d_sa, h_sa, sizeof(float4) * (size_t)ns, hipMemcpyHostToDevice)) return -1;
+  if (!stage(rt, *d, d_t, h_t, tb, hipMemcpyHostToDevice)) return -1;
   if (!vort_core(rt, *d, d_spv, d_sa, ns, d_t, nt, d_out, reg, rt.acc_mode, sigma, false,
                  d->stream, nullptr, cutoff))
     return -1;
-  if (!d2h(rt, *d, h_out, d_out, ob)) return -1;
+  if (!stage(rt, *d, h_out, d_out, ob, hipMemcpyDeviceToHost)) return -1;
   if (!check_hip(rt, hipStreamSynchronize(d->stream), "vorticity kernels")) return -1;
   std::memcpy(out, h_out, ob);
   return 0;
@@ -126,11 +126,12 @@ int relax_host(cvtx_P3D** p, int n, float fdt, const cvtx_VortFunc* vf, float si
   float* d_om = (float*)device_buffer(rt, *d, SLOT_OUT0, ob);
   if (!h_pv || !h_a || !d_pv || !d_a || !d_om) return -1;
   gather_p3d(p, n, h_pv, h_a);
-  if (!h2d(rt, *d, d_pv, h_pv, pb) || !h2d(rt, *d, d_a, h_a, pb)) return -1;
+  if (!stage(rt, *d, d_pv, h_pv, pb, hipMemcpyHostToDevice) ||
+      !stage(rt, *d, d_a, h_a, pb, hipMemcpyHostToDevice)) return -1;
   if (!vort_core(rt, *d, d_pv, d_a, n, d_pv, n, d_om, reg, rt.acc_mode, sigma, true, d->stream))
     return -1;
   if (!check_hip(rt, launch_relax(d_a, d_om, n, fdt, d->stream), "relaxation kernel")) return -1;
-  if (!d2h(rt, *d, h_a, d_a, pb)) return -1;
+  if (!stage(rt, *d, h_a, d_a, pb, hipMemcpyDeviceToHost)) return -1;
   if (!check_hip(rt, hipStreamSynchronize(d->stream), "relaxation")) return -1;
   parallel_for(n, [&](long b, long e) {
     for (long i = b; i < e; ++i) {
