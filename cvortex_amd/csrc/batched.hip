@@ -42,7 +42,7 @@ struct BatchParams {
   P3DKParams base;  // concatenated particle arrays and outputs; n_split = 1
   const int2* __restrict__ units;          // (cloud, first target)
   const int2* __restrict__ range;          // cloud -> (begin, end)
-  const RegConsts* __restrict__ rc;        // per cloud
+  const P3DConsts* __restrict__ rc;        // per cloud
   const Scales* __restrict__ sc;           // per cloud
   unsigned int* __restrict__ counter;
   int n_units;
@@ -182,7 +182,7 @@ struct cvtx_hip_batch {
   // device
   int2* d_units = nullptr;
   int2* d_range = nullptr;
-  RegConsts* d_rc = nullptr;
+  P3DConsts* d_rc = nullptr;
   Scales* d_sc = nullptr;
   unsigned int* d_counter = nullptr;
   double* d_work = nullptr;
@@ -389,7 +389,7 @@ cvtx_hip_batch* cvtx_hip_batch_create(int n_clouds, const int* offsets, const fl
   b->end.assign(offsets + 1, offsets + n_clouds + 1);
   b->sigma.assign(sigmas, sigmas + n_clouds);
   std::vector<int2> range(n_clouds);
-  std::vector<RegConsts> rc(n_clouds);
+  std::vector<P3DConsts> rc(n_clouds);
   std::vector<Scales> sc(n_clouds);
   for (int c = 0; c < n_clouds; ++c) {
     range[c] = make_int2(offsets[c], offsets[c + 1]);
@@ -399,12 +399,12 @@ cvtx_hip_batch* cvtx_hip_batch_create(int n_clouds, const int* offsets, const fl
   bool ok = true;
   const size_t nc = std::max(1, n_clouds);
   ok = ok && hipMalloc(&b->d_range, sizeof(int2) * nc) == hipSuccess;
-  ok = ok && hipMalloc(&b->d_rc, sizeof(RegConsts) * nc) == hipSuccess;
+  ok = ok && hipMalloc(&b->d_rc, sizeof(P3DConsts) * nc) == hipSuccess;
   ok = ok && hipMalloc(&b->d_sc, sizeof(Scales) * nc) == hipSuccess;
   ok = ok && hipMalloc(&b->d_counter, 256) == hipSuccess;
   if (ok && n_clouds > 0) {
     ok = ok && hipMemcpy(b->d_range, range.data(), sizeof(int2) * n_clouds, hipMemcpyHostToDevice) == hipSuccess;
-    ok = ok && hipMemcpy(b->d_rc, rc.data(), sizeof(RegConsts) * n_clouds, hipMemcpyHostToDevice) == hipSuccess;
+    ok = ok && hipMemcpy(b->d_rc, rc.data(), sizeof(P3DConsts) * n_clouds, hipMemcpyHostToDevice) == hipSuccess;
     ok = ok && hipMemcpy(b->d_sc, sc.data(), sizeof(Scales) * n_clouds, hipMemcpyHostToDevice) == hipSuccess;
   }
   // the autotuner's shape for this batch's signature, if one is cached

@@ -49,6 +49,12 @@ struct RegConsts {
   float q_exp = 46.f;   // 3D gaussian: rho^2 from which 1 - rho zeta and G - zeta/3 round to 1 and G
   float q_tab = (float)(GTAB_RHO_MAX * GTAB_RHO_MAX);  // gaussian: table range in rho^2
   float xs = 1.f;  // 3D winckelmans, gaussian: power of two that positions are multiplied by
+};
+
+// The 3D kernels' constants.  (A struct of their own: the other kernels' schedules
+// suffer from a larger argument; the 2D planetary velocity with four targets per
+// lane takes 12.5 ms instead of 11.3 for 262144 particles.)
+struct P3DConsts : RegConsts {
   // 3D gaussian, with t from GaussianKernel: 1/t^3, 1/t^5, t^3, -1/t,
   // -1/(3 t^3), GTAB_PER_UNIT/t (used by the near ranges only)
   float g3 = 1.f, h5 = 1.f, t3 = 1.f, nt1 = -1.f, nt3 = -1.f / 3.f, tp = GTAB_PER_UNIT;
@@ -72,7 +78,7 @@ __device__ __forceinline__ int in_vgpr(int x) {
 
 // The constants of `k` as VGPR values (see in_vgpr), for use inside pair loops.
 __device__ __forceinline__ RegConsts loop_consts(const RegConsts& k) {
-  RegConsts v = k;
+  RegConsts v;
   v.s2 = in_vgpr(k.s2);
   v.inv_s2 = in_vgpr(k.inv_s2);
   v.c1 = in_vgpr(k.c1);
@@ -80,6 +86,11 @@ __device__ __forceinline__ RegConsts loop_consts(const RegConsts& k) {
   v.q_far = in_vgpr(k.q_far);
   v.q_exp = in_vgpr(k.q_exp);
   v.q_tab = in_vgpr(k.q_tab);
+  return v;
+}
+__device__ __forceinline__ P3DConsts loop_consts(const P3DConsts& k) {
+  P3DConsts v = k;
+  static_cast<RegConsts&>(v) = loop_consts(static_cast<const RegConsts&>(k));
   return v;
 }
 
@@ -228,7 +239,7 @@ struct GaussianKernel {
   struct Far {
     float pinv, pinv2, g, h;
   };
-  static __device__ __forceinline__ Far far(float& r2, const RegConsts& k) {
+  static __device__ __forceinline__ Far far(float& r2, const P3DConsts& k) {
     if constexpr (!DIRECT) r2 = __builtin_fmaf(r2, k.inv_s2, 1e-30f);
     Far f;
     f.pinv = __builtin_amdgcn_rsqf(r2);  // 1/r
@@ -240,7 +251,7 @@ struct GaussianKernel {
   // (G itself in gr where the caller sums it in FP64: its product with 1/t^3
   // would be rounded to FP32, so the epilogue multiplies the sum.)
   template <class Same>
-  static __device__ __forceinline__ void near(const Far& f, float r2, const RegConsts& k,
+  static __device__ __forceinline__ void near(const Far& f, float r2, const P3DConsts& k,
                                               const float4* tab, Same&& same, float& g, float& h,
                                               float& z, float& gr) {
     z = k.c2 * __builtin_amdgcn_exp2f(r2 * k.c1);
@@ -280,7 +291,7 @@ struct GaussianKernel {
   // vel+dvort kernel (two targets per lane) 680 -> 700 ms, so eval() does
   // not pin.
   template <bool PIN = false, class Same, class Near>
-  static __device__ __forceinline__ void eval_ranges(float r2, const RegConsts& k,
+  static __device__ __forceinline__ void eval_ranges(float r2, const P3DConsts& k,
                                                      const float4* tab, Same&& same, float& Kv,
                                                      float& Kh, float& eta, float& Kfar,
                                                      Near&& near_cb) {
@@ -310,7 +321,7 @@ struct GaussianKernel {
   // one below 46: 65536 2685 -> 2652 us, cube of 50000 1681 -> 1636 (targets not
   // ordered, where nearly every such round has both: 6000 59.8 -> 61.1 with it).
   template <bool NEST, class Same, class Near, class FarCb>
-  static __device__ __forceinline__ void eval_split(float r2, const RegConsts& k,
+  static __device__ __forceinline__ void eval_split(float r2, const P3DConsts& k,
                                                     const float4* tab, Same&& same, float& Kv,
                                                     float& Kh, float& eta, Near&& near_cb,
                                                     FarCb&& far_cb) {
@@ -329,7 +340,7 @@ struct GaussianKernel {
   }
 
   template <class Same>
-  static __device__ __forceinline__ void eval(float r2, const RegConsts& k, const float4* tab,
+  static __device__ __forceinline__ void eval(float r2, const P3DConsts& k, const float4* tab,
                                               Same&& same, float& Kv, float& Kh, float& eta) {
     float kf;
     eval_ranges(r2, k, tab, same, Kv, Kh, eta, kf, [](float, float) {});

@@ -152,7 +152,7 @@ hipError_t launch_relax(float4* a, const float* omega, int n, float fdt, hipStre
 // Host-side helpers.
 // direct: which form of the Gaussian pair (GaussianKernel).
 Scales p3d_scales(int reg, float sigma, float nu, bool direct);
-RegConsts p3d_consts(int reg, float sigma, int mask, int acc, bool direct);
+P3DConsts p3d_consts(int reg, float sigma, int mask, int acc, bool direct);
 bool p3d_supported(int reg, int mask);
 bool p2d_supported(int reg, int mask);
 

@@ -81,8 +81,8 @@ static int radius_exponent(float sigma) {
   return std::min(126, std::max(-126, -std::ilogb(s)));
 }
 
-RegConsts p3d_consts(int reg, float sigma, int mask, int acc, bool direct) {
-  RegConsts k{};
+P3DConsts p3d_consts(int reg, float sigma, int mask, int acc, bool direct) {
+  P3DConsts k{};
   const double s = std::fabs((double)sigma);
   k.s2 = (float)(s * s);
   k.inv_s2 = (float)(1.0 / (s * s));

@@ -65,7 +65,7 @@ struct P3DKParams {
   double* __restrict__ partial;          // indexed by target slot
   const int* __restrict__ tgt_perm;      // slot -> target (nullptr: identity)
   int n_src, n_tgt, split_len, n_split;
-  RegConsts rc;
+  P3DConsts rc;
   Scales sc;
 };
 
@@ -80,7 +80,7 @@ enum SelfMode : int { SELF_NONE, SELF_TEST, SELF_WATCH };
 template <int REG, int MASK, int ACC, int SELF, bool DIRECT>
 __device__ __forceinline__ void p3d_pair(const float4 sp, const float4 sa, const double2* pxy,
                                          const double2* pzv, const float3 xt, const float3 at,
-                                         const RegConsts& rc, const float4* tab, float* acc,
+                                         const P3DConsts& rc, const float4* tab, float* acc,
                                          double* dacc, float& smin) {
   using R = P3DRegs<REG, MASK, ACC>;
   const float dx = xt.x - sp.x;
@@ -258,7 +258,7 @@ struct P3DShare {
 // and issues no barrier-sensitive work on sm around the call.
 // DIRECT: which form of the Gaussian pair (GaussianKernel).
 template <int REG, int MASK, int ACC, int T, int WG, bool DIRECT, int Q = 1>
-__device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& rc,
+__device__ __forceinline__ void p3d_block(const P3DKParams& p, const P3DConsts& rc,
                                           const Scales& sc, int base, int tgt_end, int s0,
                                           int s1, int split, P3DSmem<REG, MASK, ACC, WG>& sm,
                                           P3DShare<MASK, Q>* share = nullptr) {
@@ -267,7 +267,7 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
   using R = P3DRegs<REG, MASK, ACC>;
   constexpr int NF = R::NF;
   constexpr int ND = R::ND > 0 ? R::ND : 1;
-  constexpr bool SCALED = REG == REG_WINCKELMANS || REG == REG_GAUSSIAN;  // RegConsts::xs
+  constexpr bool SCALED = REG == REG_WINCKELMANS || REG == REG_GAUSSIAN;  // P3DConsts::xs
   constexpr bool DBL_ = P3DSmem<REG, MASK, ACC, WG>::DBL;
   const int tid = threadIdx.x;
   const int tl = Q == 1 ? tid : tid & 63;  // target within the group
@@ -301,7 +301,7 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const RegConsts& 
     for (int a = 0; a < ND; ++a) dacc[k][a] = 0.0;
   }
 
-  const RegConsts rv = loop_consts(rc);
+  const P3DConsts rv = loop_consts(rc);
   const bool one_array = p.src_pv == p.tgt_pv && p.tgt_perm == nullptr;
   for (int ts = s0; ts < s1; ts += WG) {
     const int cnt = min(WG, s1 - ts);
