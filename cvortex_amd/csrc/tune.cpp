@@ -214,6 +214,17 @@ LaunchCfg choose_cfg(int kind, int reg, int mask, int acc, int n_src, int n_tgt,
   }
   if (narrow(kind, reg, mask, n_src, n_tgt, cus)) return narrow_cfg(kind, reg, mask, n_src, n_tgt, cus);
   if (kind == KIND_P2D) return p2d_cfg(reg, mask, n_src, n_tgt, cus);
+  // Filaments: a block's tiles near it take several times the far ones' time, so
+  // partitions go down to one tile for 64 workgroups per CU, which spread them
+  // (a kernel of one or two tiles' worth of filaments gains nothing from it).
+  // Partitions of six, three and two tiles -> this, us: 14000 filaments on 40000
+  // targets velocity 509 -> 418, both 737 -> 622, 4293 on 156344 558 -> 491, 801 ->
+  // 759, 11475 on 312258 2186 -> 2087, 16384 on 2^20 9368 -> 9195; but 459 on 394673
+  // 341 -> 351.
+  if (kind == KIND_F3D && n_src >= 12 * 256) {
+    const long long nb = ((long long)n_tgt + 255) / 256, tiles = ((long long)n_src + 255) / 256;
+    return launch_shape(1, (int)std::min(tiles, (64LL * cus + nb - 1) / std::max(1LL, nb)), n_src);
+  }
   LaunchCfg c = default_cfg(n_src, n_tgt, n_cu);
   const bool many_blocks = (long long)(n_tgt + 255) / 256 >= 4LL * cus;
   // Filaments: one target per lane.  It fits in fewer VGPRs (more waves per
