@@ -138,8 +138,8 @@ struct RegKernel;
 
 template <>
 struct RegKernel<REG_SINGULAR> {
-  // Kv = r^-3, Kh = r^-5 (x3 in the epilogue); infinite at r2 = 0, so the
-  // test stays for every SELF
+  // Kv = r^-3, Kh = r^-5 (x3 in the epilogue); infinite at r2 = 0: SELF = false
+  // only where the caller finds such pairs itself (SELF_WATCH)
   template <bool SELF = true>
   static __device__ __forceinline__ void eval(float r2, const RegConsts&, const float4*,
                                               float& Kv, float& Kh, float& eta) {
@@ -147,7 +147,7 @@ struct RegKernel<REG_SINGULAR> {
     float y2 = y * y;
     float kv = y * y2;
     float kh = kv * y2;
-    bool z = (r2 == 0.f);
+    bool z = SELF && (r2 == 0.f);
     Kv = z ? 0.f : kv;
     Kh = z ? 0.f : kh;
     eta = 0.f;

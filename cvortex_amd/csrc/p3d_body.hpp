@@ -69,12 +69,12 @@ struct P3DKParams {
   Scales sc;
 };
 
-// How a Winckelmans pair with equal coordinates is dropped (the other
-// regularisations test r^2 == 0 in their own kernels).  SELF_NONE: it need
-// not be, the velocity term being Kv (d x a_s) with d = 0.  SELF_TEST: a
-// compare per pair.  SELF_WATCH: only the smallest S = r^2 + sigma^2 of the
-// tile is kept, a third as many instructions; where it is sigma^2 the caller
-// repeats the tile with SELF_TEST (see p3d_block).
+// How a Winckelmans pair with equal coordinates, or a singular one with r^2 = 0,
+// is dropped (the others test r^2 == 0 in their own kernels).  SELF_NONE: it need
+// not be, the velocity term being Kv (d x a_s) with d = 0 and Kv finite.
+// SELF_TEST: a compare per pair.  SELF_WATCH: only the smallest r^2 (+ sigma^2)
+// of the tile is kept, a third as many instructions; where it is that of such a
+// pair the caller repeats the tile with SELF_TEST (see p3d_block).
 enum SelfMode : int { SELF_NONE, SELF_TEST, SELF_WATCH };
 
 template <int REG, int MASK, int ACC, int SELF, bool DIRECT>
@@ -146,6 +146,9 @@ __device__ __forceinline__ void p3d_pair(const float4 sp, const float4 sa, const
     });
   } else if constexpr (REG == REG_GAUSSIAN) {
     GaussianKernel<DIRECT>::eval(r2, rc, tab, same_place, Kv, Kh, eta);
+  } else if constexpr (REG == REG_SINGULAR) {
+    RegKernel<REG_SINGULAR>::template eval<SELF != SELF_WATCH>(r2, rc, tab, Kv, Kh, eta);
+    if constexpr (SELF == SELF_WATCH) smin = fminf(smin, r2);
   } else {
     RegKernel<REG>::template eval<(MASK & (OUT_DVORT | OUT_VISC)) != 0>(r2, rc, tab, Kv, Kh, eta);
   }
@@ -371,7 +374,12 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const P3DConsts& 
     // of 41, ms: 128 clouds, tile-compensated 51.1 -> 46.6; 64 clouds, FP64
     // stretching 32.1 -> 30.8; 400000 particles with the viscous term 147.4 ->
     // 141.0; velocity of 100000 (S alone) 4.38 -> 4.06.
-    constexpr bool WATCH = Q == 1 && REG == REG_WINCKELMANS && ACC != ACC_PLAIN && (MASK & (OUT_DVORT | OUT_VISC)) != 0;
+    // Singular, whose Kv is infinite there, likewise (r^2 = 0) for every output:
+    // a compare and one or two selects less.  100000 particles on 300000, velocity
+    // 11.95 -> 11.16 ms, with the stretching 20.50 -> 19.23.
+    constexpr bool WATCH = Q == 1 && ACC != ACC_PLAIN &&
+                           (REG == REG_SINGULAR ||
+                            (REG == REG_WINCKELMANS && (MASK & (OUT_DVORT | OUT_VISC)) != 0));
     if constexpr (WATCH) {
       // (a block's own tiles, where sources and targets are one array, are known)
       bool test = one_array && ts < base + T * WG && ts + cnt > base;
@@ -382,7 +390,7 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const P3DConsts& 
 #pragma unroll
           for (int a = 0; a < ND; ++a) before[k][a] = dacc[k][a];
         tile(std::integral_constant<int, SELF_WATCH>());
-        if (__any(smin <= rc.s2)) {
+        if (__any(smin <= (REG == REG_SINGULAR ? 0.f : rc.s2))) {
           test = true;
 #pragma unroll
           for (int k = 0; k < T; ++k)
