@@ -92,7 +92,8 @@ __device__ __forceinline__ void p3d_pair(const float4 sp, const float4 sa, const
   const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, z2));
   auto same_place = [&] {
     if constexpr (REG == REG_GAUSSIAN && !DIRECT) return r2 == 0.f;
-    return (__float_as_uint(dx) | __float_as_uint(dy) | __float_as_uint(dz)) == 0u;
+    // zeros of either sign: -0.0 - (+0.0) is -0.0
+    return __uint_as_float(__float_as_uint(dx) | __float_as_uint(dy) | __float_as_uint(dz)) == 0.f;
   };
   float Kv, Kh, eta, Kfar = 0.f;
   if constexpr (REG == REG_WINCKELMANS) {
