@@ -133,7 +133,7 @@ Scales p3d_scales(int reg, float sigma, float nu, bool direct) {
     case REG_GAUSSIAN: {
       // as for Winckelmans below
       const double x = std::ldexp(1.0, radius_exponent(sigma)), t = std::isinf(s) ? 1.0 : s * x;
-      const double on = std::isinf(s) ? 0.0 : (s == 0.0 ? std::nan("") : 1.0);
+      const double on = std::isinf(s) ? 0.0 : (s > 0.0 ? 1.0 : std::nan(""));
       const double f = direct ? 1.0 : 1.0 / (t * t * t);
       sc.vel = -k4pi * x * x * on * f;
       sc.dG = sgn * k4pi * x * x * x * on * f;
