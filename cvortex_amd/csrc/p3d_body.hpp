@@ -77,6 +77,14 @@ struct P3DKParams {
 // pair the caller repeats the tile with SELF_TEST (see p3d_block).
 enum SelfMode : int { SELF_NONE, SELF_TEST, SELF_WATCH };
 
+// A coordinate in the kernel's units.  One that overflows there (a particle parked
+// at FLT_MAX) stays as it is: the square of its distance to any other is infinite
+// in either unit, and its pairs give 0, where an infinite difference gives NaN.
+__device__ __forceinline__ float scaled(float x, float xs) {
+  const float y = x * xs;
+  return __builtin_isinf(y) ? x : y;
+}
+
 template <int REG, int MASK, int ACC, int SELF, bool DIRECT>
 __device__ __forceinline__ void p3d_pair(const float4 sp, const float4 sa, const double2* pxy,
                                          const double2* pzv, const float3 xt, const float3 at,
@@ -283,7 +291,8 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const P3DConsts& 
     i = i < tgt_end ? i : tgt_end - 1;
     if (p.tgt_perm) i = p.tgt_perm[i];
     const float4 q = p.tgt_pv[i];
-    xt[k] = SCALED ? make_float3(q.x * rc.xs, q.y * rc.xs, q.z * rc.xs) : make_float3(q.x, q.y, q.z);
+    xt[k] = SCALED ? make_float3(scaled(q.x, rc.xs), scaled(q.y, rc.xs), scaled(q.z, rc.xs))
+                   : make_float3(q.x, q.y, q.z);
     vt[k] = q.w;
     if constexpr (L::NEED_TA) {
       const float4 w = p.tgt_a[i];
@@ -315,9 +324,9 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const P3DConsts& 
       float4 q = p.src_pv[ts + tid];
       const float4 w = p.src_a[ts + tid];
       if constexpr (SCALED) {
-        q.x *= rc.xs;
-        q.y *= rc.xs;
-        q.z *= rc.xs;
+        q.x = scaled(q.x, rc.xs);
+        q.y = scaled(q.y, rc.xs);
+        q.z = scaled(q.z, rc.xs);
       }
       sm.xa[tid] = make_float4(q.x, q.y, q.z, w.x);
       if constexpr (P3DSmem<REG, MASK, ACC, WG>::VOL)
