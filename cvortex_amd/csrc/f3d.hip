@@ -608,6 +608,12 @@ __device__ __forceinline__ void inf_rows(const InfCols<NF>& c, const float4* s_x
                                          int nr, int j0, int n_fil, float* __restrict__ o) {
   using Vec = float __attribute__((ext_vector_type(NF)));
   using Vec4 = float __attribute__((ext_vector_type(NF), aligned(4)));  // any float's address
+  // Added to the squared distances (no instruction more): the reciprocal root of a
+  // denormal one is infinite, and the far form would turn that into NaN.
+  const float tiny = in_vgpr(0x1p-120f);
+  auto norm2 = [&](float3 r) {
+    return __builtin_fmaf(r.x, r.x, __builtin_fmaf(r.y, r.y, __builtin_fmaf(r.z, r.z, tiny)));
+  };
   int iv = in_vgpr(0);
   float4 xn = s_x[iv], en = s_e[iv];
   for (int i = 0; i < nr; ++i, o += n_fil) {
@@ -628,12 +634,12 @@ __device__ __forceinline__ void inf_rows(const InfCols<NF>& c, const float4* s_x
       float y1 = y2, n1 = n2;
       if (f == 0 || !SHARE) {
         r1 = sub3(x, c.a[f]);
-        const float ns = dot3(r1, r1);
+        const float ns = norm2(r1);
         y1 = __builtin_amdgcn_rsqf(ns);
         n1 = ns * y1;
       }
       r2 = sub3(x, c.b[f]);
-      const float ns = dot3(r2, r2);
+      const float ns = norm2(r2);
       y2 = __builtin_amdgcn_rsqf(ns);
       n2 = ns * y2;
       const float S = n1 + n2;
