@@ -240,7 +240,9 @@ __global__ __launch_bounds__(WG, (f3d_min_waves<MASK, T>())) void f3d_kernel(F3D
                  (int)(__float_as_uint(an.z) == __float_as_uint(b.z));
         }
         s_a[tid] = make_float4(a.x, a.y, a.z, g);
-        s_b[tid] = make_float4(b.x, b.y, b.z, -6.f * g / __builtin_sqrtf(l2));
+        // (a filament of no length contributes nothing: its factor, infinite
+        // here, times |c| = 0 would make the far loop's sum NaN)
+        s_b[tid] = make_float4(b.x, b.y, b.z, l2 > 0.f ? -6.f * g / __builtin_sqrtf(l2) : 0.f);
         s_r0[tid] = make_float4(rx, ry, rz, 0.5f * l2);
       }
       const unsigned long long links = __ballot(link != 0);
