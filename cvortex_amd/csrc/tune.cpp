@@ -175,8 +175,8 @@ LaunchCfg choose_cfg(int kind, int reg, int mask, int acc, int n_src, int n_tgt,
                              size_bucket(n_src), size_bucket(n_tgt)});
   const int cus = n_cu > 0 ? n_cu : 256;
   if (it != cache().end())
-    return it->second.q == 4 ? narrow_cfg(kind, reg, mask, n_src, n_tgt, cus)
-                             : launch_shape(it->second.T, it->second.n_split, n_src);
+    return it->second.q == 4 && n_tgt > 0 ? narrow_cfg(kind, reg, mask, n_src, n_tgt, cus)
+                                          : launch_shape(it->second.T, it->second.n_split, n_src);
   // Spatially ordered targets (Gaussian P3D, compensated sums).  One target
   // per lane: a 64-target wave of Morton-ordered targets is more compact
   // than a 128-target one, so fewer of its source rounds take the FP64
