@@ -35,7 +35,7 @@ void gather_p3d(const cvtx_P3D* const* src, int n, float4* pv, float4* a) {
     for (long i = b; i < e; ++i) {
       const cvtx_P3D* p = src[i];
       pv[i] = make_float4(p->coord.x[0], p->coord.x[1], p->coord.x[2], p->volume);
-      a[i] = make_float4(p->vorticity.x[0], p->vorticity.x[1], p->vorticity.x[2], 0.f);
+      if (a) a[i] = make_float4(p->vorticity.x[0], p->vorticity.x[1], p->vorticity.x[2], 0.f);
     }
   });
 }
