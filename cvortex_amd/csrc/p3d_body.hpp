@@ -101,7 +101,10 @@ __device__ __forceinline__ void p3d_pair(const float4 sp, const float4 sa, const
   auto same_place = [&] {
     if constexpr (REG == REG_GAUSSIAN && !DIRECT) return r2 == 0.f;
     // zeros of either sign: -0.0 - (+0.0) is -0.0
-    return __uint_as_float(__float_as_uint(dx) | __float_as_uint(dy) | __float_as_uint(dz)) == 0.f;
+    // (the larger of three that propagates NaN: one instruction and a compare)
+    const float x = __builtin_elementwise_abs(dx), y = __builtin_elementwise_abs(dy);
+    return __builtin_elementwise_maximum(__builtin_elementwise_maximum(x, y),
+                                         __builtin_elementwise_abs(dz)) == 0.f;
   };
   float Kv, Kh, eta, Kfar = 0.f;
   if constexpr (REG == REG_WINCKELMANS) {
