@@ -394,7 +394,7 @@ cvtx_hip_batch* cvtx_hip_batch_create(int n_clouds, const int* offsets, const fl
   for (int c = 0; c < n_clouds; ++c) {
     range[c] = make_int2(offsets[c], offsets[c + 1]);
     rc[c] = p3d_consts(regularisation, sigmas[c], outputs, accumulate, false);
-    sc[c] = p3d_scales(regularisation, sigmas[c], nu, false);
+    sc[c] = p3d_scales(regularisation, sigmas[c], nu, outputs, false);
   }
   bool ok = true;
   const size_t nc = std::max(1, n_clouds);

@@ -159,13 +159,14 @@ struct RegKernel<REG_WINCKELMANS> {
   // Positions come multiplied by a power of two (RegConsts::xs, exact) that
   // puts sigma in [1, 2), so that S = r^2 + sigma^2 can be formed in three
   // multiply-adds started from sigma^2 (rather than r^2 and then r^2/sigma^2
-  // + 1) and its powers stay in range.  With y = S^-1/2, in those units:
+  // + 1) and its powers stay in range; with the exchange (winckelmans_reduced)
+  // S = r^2/sigma^2 + 1 and sigma is 1 here.  With y = S^-1/2, in those units:
   //   Kv  = (r^2 + 2.5 sigma^2) y^5 = y^3 (1 + 1.5 sigma^2 y^2)
   //   Kh  = (r^2 + 3.5 sigma^2) y^7 = (Kv + sigma^2 y^5) y^2
   //   eta = y^9
-  // (x 3 and x 52.5 sigma^9 in the epilogue).  None is zero at r = 0: the
-  // caller drops coincident pairs where that matters.  k: s2 = sigma^2, c1 =
-  // 1.5 sigma^2.
+  // (x 3 and x 52.5 in the epilogue).  None is zero at r = 0: the caller drops
+  // coincident pairs where that matters.  k: s2 = sigma^2, c1 = 1.5 sigma^2, but
+  // for the rounding (p3d_consts).
   static __device__ __forceinline__ void eval(float S, const RegConsts& k, float& Kv, float& Kh,
                                               float& eta) {
     const float y = __builtin_amdgcn_rsqf(S);

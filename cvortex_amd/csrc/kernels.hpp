@@ -151,7 +151,12 @@ hipError_t launch_relax(float4* a, const float* omega, int n, float fdt, hipStre
 
 // Host-side helpers.
 // direct: which form of the Gaussian pair (GaussianKernel).
-Scales p3d_scales(int reg, float sigma, float nu, bool direct);
+// Winckelmans with the exchange: S = 1 + r^2 / sigma^2 in units of the radius, in
+// which S is rounded once.  (r^2 + sigma^2 formed in one chain rounds three times at
+// the size of S, which the exchange's S^-9/2 multiplies by 4.5: 23011 sources on
+// 9973 targets, against 64 bits, 1.7e-7, so 1.4e-7.)
+constexpr bool winckelmans_reduced(int mask) { return (mask & OUT_VISC) != 0; }
+Scales p3d_scales(int reg, float sigma, float nu, int mask, bool direct);
 P3DConsts p3d_consts(int reg, float sigma, int mask, int acc, bool direct);
 bool p3d_supported(int reg, int mask);
 bool p2d_supported(int reg, int mask);

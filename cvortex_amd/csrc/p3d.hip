@@ -81,6 +81,13 @@ static int radius_exponent(float sigma) {
   return std::min(126, std::max(-126, -std::ilogb(s)));
 }
 
+// Winckelmans in reduced units: the relative rounding a of 1/sigma^2 as the kernel
+// has it, S = 1 + a q.
+static double reduced_rounding(double s) {
+  const float inv = (float)(1.0 / (s * s));
+  return std::isfinite(inv) && inv > 0.f ? (double)inv * (s * s) : 1.0;
+}
+
 P3DConsts p3d_consts(int reg, float sigma, int mask, int acc, bool direct) {
   P3DConsts k{};
   const double s = std::fabs((double)sigma);
@@ -112,18 +119,28 @@ P3DConsts p3d_consts(int reg, float sigma, int mask, int acc, bool direct) {
     k.q_tab = (float)(k.q_tab * t2);
   }
   if (reg == REG_WINCKELMANS) {
-    k.xs = (float)std::ldexp(1.0, radius_exponent(sigma));
-    const double t = s * (double)k.xs;
-    // no field of a radius that is no length: 0 and NaN give NaN; an infinite
-    // one is scaled by 0 below
-    const double t2 = std::isinf(s) ? 1.0 : (s == 0.0 ? std::nan("") : t * t);
-    k.s2 = (float)t2;
-    k.c1 = (float)(1.5 * t2);
+    // sigma^2 or its reciprocal is rounded, one relative error for all pairs, and
+    // the constants are chosen so that Kv is exact far away and at r = 0 all the
+    // same (and Kh, in reduced units): the radii whose squares round most, error
+    // common to all pairs of a core, 1.0e-7 -> 4e-8.
+    if (winckelmans_reduced(mask)) {
+      const double a = reduced_rounding(s);
+      k.c1 = (float)(2.5 * std::pow(a, -1.5) - 1.0);
+      k.s2 = (float)(3.5 * std::pow(a, -2.5) - 1.0 - (double)k.c1);
+    } else {
+      k.xs = (float)std::ldexp(1.0, radius_exponent(sigma));
+      const double t = s * (double)k.xs;
+      // no field of a radius that is no length: 0 and NaN give NaN, an infinite
+      // one is scaled by 0 (p3d_scales)
+      const double t2 = std::isinf(s) ? 1.0 : (s == 0.0 ? std::nan("") : t * t);
+      k.s2 = (float)t2;
+      k.c1 = (float)((double)k.s2 * (2.5 * std::pow((double)k.s2 / t2, 1.5) - 1.0));
+    }
   }
   return k;
 }
 
-Scales p3d_scales(int reg, float sigma, float nu, bool direct) {
+Scales p3d_scales(int reg, float sigma, float nu, int mask, bool direct) {
   Scales sc;
   const double s = std::fabs((double)sigma);
   const double sgn = sigma < 0 ? -1.0 : 1.0;
@@ -143,14 +160,24 @@ Scales p3d_scales(int reg, float sigma, float nu, bool direct) {
       break;
     }
     case REG_WINCKELMANS: {
-      // in positions multiplied by x: Kv is x^-3 of the dimensional one, each
-      // position factor x
-      const double x = std::ldexp(1.0, radius_exponent(sigma)), t = s * x;
-      const double on = std::isinf(s) ? 0.0 : 1.0;
-      sc.vel = -k4pi * x * x * on;
-      sc.dG = sgn * k4pi * x * x * x * on;
-      sc.dH = 3.0 * sc.dG;
-      sc.visc = std::isinf(s) ? 0.0 : 2.0 * (double)nu / (s * s) * 52.5 * std::pow(t, 9);
+      const double on = std::isinf(s) ? 0.0 : (s > 0.0 ? 1.0 : std::nan(""));
+      if (winckelmans_reduced(mask)) {
+        // S^-3/2 and S^-5/2 far away; S^-9/2 on average over a uniform
+        // neighbourhood, where q / (1 + q) has the mean 1/3 under the weight
+        // (1 + q)^-4.5 q^1/2 dq
+        const double a = reduced_rounding(s);
+        sc.vel = -k4pi / s3 * on * std::pow(a, 1.5);
+        sc.dG = -sgn * sc.vel;
+        sc.dH = 3.0 * sgn * k4pi / s5 * on * std::pow(a, 2.5);
+        sc.visc = 2.0 * (double)nu / (s * s) * on * 52.5 * std::pow(a, 1.5);
+      } else {
+        // in positions multiplied by x: Kv is x^-3 of the dimensional one, each
+        // position factor x
+        const double x = std::ldexp(1.0, radius_exponent(sigma));
+        sc.vel = -k4pi * x * x * on;
+        sc.dG = sgn * k4pi * x * x * x * on;
+        sc.dH = 3.0 * sc.dG;
+      }
       break;
     }
     case REG_PLANETARY:
@@ -268,7 +295,7 @@ hipError_t launch_p3d(const P3DJob& j, const LaunchCfg& c, hipStream_t s) {
   p.n_src = j.n_src;
   p.n_tgt = j.n_tgt;
   p.rc = p3d_consts(j.reg, j.sigma, j.mask, j.acc, c.q == 1);
-  p.sc = p3d_scales(j.reg, j.sigma, j.nu, c.q == 1);
+  p.sc = p3d_scales(j.reg, j.sigma, j.nu, j.mask, c.q == 1);
 
   int n_split = c.n_split;
   int split_len = c.split_len;

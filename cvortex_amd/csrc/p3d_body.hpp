@@ -97,12 +97,13 @@ __device__ __forceinline__ void p3d_pair(const float4 sp, const float4 sa, const
   const float dx = xt.x - sp.x;
   const float dy = xt.y - sp.y;
   const float dz = xt.z - sp.z;
-  const float z2 = REG == REG_WINCKELMANS ? __builtin_fmaf(dz, dz, rc.s2)
+  constexpr bool REDUCED = REG == REG_WINCKELMANS && winckelmans_reduced(MASK);
+  const float z2 = REG == REG_WINCKELMANS && !REDUCED ? __builtin_fmaf(dz, dz, rc.s2)
                    : REG == REG_GAUSSIAN && DIRECT ? __builtin_fmaf(dz, dz, 1e-30f)
                                                    : dz * dz;
   const float r2 = __builtin_fmaf(dx, dx, __builtin_fmaf(dy, dy, z2));
   auto same_place = [&] {
-    if constexpr (REG == REG_GAUSSIAN && !DIRECT) return r2 == 0.f;
+    if constexpr (REDUCED || (REG == REG_GAUSSIAN && !DIRECT)) return r2 == 0.f;
     // zeros of either sign: -0.0 - (+0.0) is -0.0
     // (the larger of three that propagates NaN: one instruction and a compare)
     const float x = __builtin_elementwise_abs(dx), y = __builtin_elementwise_abs(dy);
@@ -111,7 +112,8 @@ __device__ __forceinline__ void p3d_pair(const float4 sp, const float4 sa, const
   };
   float Kv, Kh, eta, Kfar = 0.f;
   if constexpr (REG == REG_WINCKELMANS) {
-    RegKernel<REG_WINCKELMANS>::eval(r2, rc, Kv, Kh, eta);
+    const float S = REDUCED ? __builtin_fmaf(r2, rc.inv_s2, 1.f) : r2;
+    RegKernel<REG_WINCKELMANS>::eval(S, rc, Kv, Kh, eta);
     if constexpr (SELF == SELF_WATCH) smin = fminf(smin, r2);
     if constexpr (SELF == SELF_TEST) {
       const bool same = same_place();
@@ -285,7 +287,8 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const P3DConsts& 
   using R = P3DRegs<REG, MASK, ACC>;
   constexpr int NF = R::NF;
   constexpr int ND = R::ND > 0 ? R::ND : 1;
-  constexpr bool SCALED = REG == REG_WINCKELMANS || REG == REG_GAUSSIAN;  // P3DConsts::xs
+  // P3DConsts::xs
+  constexpr bool SCALED = (REG == REG_WINCKELMANS && !winckelmans_reduced(MASK)) || REG == REG_GAUSSIAN;
   constexpr bool DBL_ = P3DSmem<REG, MASK, ACC, WG>::DBL;
   const int tid = threadIdx.x;
   const int tl = Q == 1 ? tid : tid & 63;  // target within the group
@@ -406,7 +409,7 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const P3DConsts& 
 #pragma unroll
           for (int a = 0; a < ND; ++a) before[k][a] = dacc[k][a];
         tile(std::integral_constant<int, SELF_WATCH>());
-        if (__any(smin <= (REG == REG_SINGULAR ? 0.f : rc.s2))) {
+        if (__any(smin <= (REG == REG_SINGULAR || winckelmans_reduced(MASK) ? 0.f : rc.s2))) {
           test = true;
 #pragma unroll
           for (int k = 0; k < T; ++k)
