@@ -55,9 +55,10 @@ struct RegConsts {
 // suffer from a larger argument; the 2D planetary velocity with four targets per
 // lane takes 12.5 ms instead of 11.3 for 262144 particles.)
 struct P3DConsts : RegConsts {
-  // 3D gaussian, with t from GaussianKernel: 1/t^3, 1/t^5, t^3, -1/t,
-  // -1/(3 t^3), GTAB_PER_UNIT/t (used by the near ranges only)
-  float g3 = 1.f, h5 = 1.f, t3 = 1.f, nt1 = -1.f, nt3 = -1.f / 3.f, tp = GTAB_PER_UNIT;
+  // 3D gaussian, with t from GaussianKernel: -1/t, -1/(3 t^3), GTAB_PER_UNIT/t, and
+  // log(2) times what c1 lacks of its value in FP64 (used by the near ranges only)
+  float nt1 = -1.f, nt3 = -1.f / 3.f, tp = GTAB_PER_UNIT, c1_rest = 0.f;
+  double g3 = 1, h5 = 1;  // 1/t^3, 1/t^5: factors of the table's G and H/3
 };
 
 // A uniform value that a pair loop reads on every pair, held in a VGPR.  On
@@ -249,22 +250,26 @@ struct GaussianKernel {
     f.h = f.g * f.pinv2;
     return f;
   }
-  // (G itself in gr where the caller sums it in FP64: its product with 1/t^3
-  // would be rounded to FP32, so the epilogue multiplies the sum.)
-  template <class Same>
+  // The table's G and H/3 come multiplied by 1/t^3 and 1/t^5, in FP64 and each
+  // coefficient rounded by itself (table_entry): a factor rounded to FP32 would be off
+  // the same way for every near pair (velocity where all pairs are near, sigma 0.61:
+  // 4.8e-8 against 64 bits with such factors, 3.3e-8 so).
+  // ZETA: zeta itself is used: the rounding of c1, times rho^2/2, is common to all
+  // pairs too and made up for (exchange, sigma 0.013: 1.0e-7 -> 3.2e-8).  G and H,
+  // against which zeta is small, take it as it is, the same with and without ZETA.
+  template <bool ZETA, class Same>
   static __device__ __forceinline__ void near(const Far& f, float r2, const P3DConsts& k,
                                               const float4* tab, Same&& same, float& g, float& h,
-                                              float& z, float& gr) {
+                                              float& z) {
     z = k.c2 * __builtin_amdgcn_exp2f(r2 * k.c1);
     if constexpr (DIRECT) {
       g = f.pinv2 * __builtin_fmaf(z, k.nt1, f.pinv);
       h = __builtin_fmaf(z, k.nt3, g) * f.pinv2;
-      gr = g * k.t3;
     } else {
       g = f.pinv2 * (f.pinv - z);
       h = __builtin_fmaf(z, -1.f / 3.f, g) * f.pinv2;
-      gr = g;
     }
+    if constexpr (ZETA) z = __builtin_fmaf(z, r2 * k.c1_rest, z);
     if (r2 < k.q_tab) {
       float t = r2 * f.pinv * (DIRECT ? k.tp : (float)GTAB_PER_UNIT);  // rho * 16
       int i = (int)t;
@@ -273,14 +278,19 @@ struct GaussianKernel {
       float u = t - (float)i;
       float4 cg = tab[2 * i];
       float4 ch = tab[2 * i + 1];
-      gr = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(cg.w, u, cg.z), u, cg.y), u, cg.x);
+      g = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(cg.w, u, cg.z), u, cg.y), u, cg.x);
       h = __builtin_fmaf(__builtin_fmaf(__builtin_fmaf(ch.w, u, ch.z), u, ch.y), u, ch.x);
-      if constexpr (DIRECT) h *= k.h5;
       const bool zr = same();
-      gr = zr ? 0.f : gr;
+      g = zr ? 0.f : g;
       z = zr ? 0.f : z;
-      g = DIRECT ? gr * k.g3 : gr;
     }
+  }
+
+  // Entry i of the table in the kernel's units.
+  static __device__ __forceinline__ float4 table_entry(const float4 v, int i, const P3DConsts& k) {
+    if constexpr (!DIRECT) return v;
+    const double f = i & 1 ? k.h5 : k.g3;
+    return make_float4((float)(v.x * f), (float)(v.y * f), (float)(v.z * f), (float)(v.w * f));
   }
 
   // PIN: keep the near range a branch.  With no work of its own in
@@ -291,7 +301,7 @@ struct GaussianKernel {
   // compensated vel-only kernel 593 -> 515 ms with the pin; the plain FP32
   // vel+dvort kernel (two targets per lane) 680 -> 700 ms, so eval() does
   // not pin.
-  template <bool PIN = false, class Same, class Near>
+  template <bool ZETA, bool PIN = false, class Same, class Near>
   static __device__ __forceinline__ void eval_ranges(float r2, const P3DConsts& k,
                                                      const float4* tab, Same&& same, float& Kv,
                                                      float& Kh, float& eta, float& Kfar,
@@ -300,9 +310,8 @@ struct GaussianKernel {
     float g = f.g, h = f.h, z = 0.f, kf = f.g;
     if (r2 < k.q_far) {
       if constexpr (PIN) asm volatile("");
-      float gr;
-      near(f, r2, k, tab, same, g, h, z, gr);
-      near_cb(gr, z);
+      near<ZETA>(f, r2, k, tab, same, g, h, z);
+      near_cb(g, z);
       kf = 0.f;
     }
     Kv = g;
@@ -321,7 +330,7 @@ struct GaussianKernel {
   // the ring's rounds (a wave and a source) 9.4 % have a pair below 208 and 3.6 %
   // one below 46: 65536 2685 -> 2652 us, cube of 50000 1681 -> 1636 (targets not
   // ordered, where nearly every such round has both: 6000 59.8 -> 61.1 with it).
-  template <bool NEST, class Same, class Near, class FarCb>
+  template <bool ZETA, bool NEST, class Same, class Near, class FarCb>
   static __device__ __forceinline__ void eval_split(float r2, const P3DConsts& k,
                                                     const float4* tab, Same&& same, float& Kv,
                                                     float& Kh, float& eta, Near&& near_cb,
@@ -329,9 +338,8 @@ struct GaussianKernel {
     const Far f = far(r2, k);
     float g = f.g, h = f.h, z = 0.f;
     if (r2 < k.q_far) {
-      float gr = DIRECT ? f.g * k.t3 : f.g;
-      if (!NEST || r2 < k.q_exp) near(f, r2, k, tab, same, g, h, z, gr);
-      near_cb(gr, z);
+      if (!NEST || r2 < k.q_exp) near<ZETA>(f, r2, k, tab, same, g, h, z);
+      near_cb(g, z);
     } else {
       far_cb(f.g);
     }
@@ -340,11 +348,11 @@ struct GaussianKernel {
     eta = z;
   }
 
-  template <class Same>
+  template <bool ZETA, class Same>
   static __device__ __forceinline__ void eval(float r2, const P3DConsts& k, const float4* tab,
                                               Same&& same, float& Kv, float& Kh, float& eta) {
     float kf;
-    eval_ranges(r2, k, tab, same, Kv, Kh, eta, kf, [](float, float) {});
+    eval_ranges<ZETA>(r2, k, tab, same, Kv, Kh, eta, kf, [](float, float) {});
   }
 };
 

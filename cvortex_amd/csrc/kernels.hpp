@@ -30,7 +30,6 @@ struct LaunchCfg {
 // FP64 epilogue scale factors.
 struct Scales {
   double vel = 0, dG = 0, dH = 0, visc = 0;
-  double near = 1;  // 3D gaussian: Kv / G, applied to the FP64 near sums of G
 };
 
 struct P3DJob {

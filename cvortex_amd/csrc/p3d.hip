@@ -37,7 +37,8 @@ __global__ __launch_bounds__(WG) void p3d_kernel(P3DKParams p) {
   __shared__ P3DSmem<REG, MASK, ACC, WG> sm;
   __shared__ P3DShare<MASK, Q> share;
   if constexpr (REG == REG_GAUSSIAN) {
-    for (int i = threadIdx.x; i < 2 * GTAB_N; i += WG) sm.tab[i] = p.gtab[i];
+    for (int i = threadIdx.x; i < 2 * GTAB_N; i += WG)
+      sm.tab[i] = GaussianKernel<Q == 1>::table_entry(p.gtab[i], i, p.rc);
   }
   const int s0 = blockIdx.y * p.split_len;
   const int s1 = min(s0 + p.split_len, p.n_src);
@@ -99,11 +100,13 @@ P3DConsts p3d_consts(int reg, float sigma, int mask, int acc, bool direct) {
     const double sx = std::isinf(s) || s == 0.0 ? 1.0 : s * (double)k.xs;
     k.inv_s2 = (float)(1.0 / (sx * sx));
     const double t = direct ? sx : 1.0, t2 = t * t;
-    k.c1 = (float)(-0.5 / (std::log(2.0) * t2));
+    // (r^2 comes in the units of t, or multiplied by 1/sigma^2 as rounded)
+    const double c1 = -0.5 / (std::log(2.0) * (direct ? t2 : sx * sx * (double)k.inv_s2));
+    k.c1 = (float)c1;
+    k.c1_rest = (float)((c1 - (double)k.c1) * std::log(2.0));
     k.c2 = (float)std::sqrt(2.0 / M_PI);
-    k.g3 = (float)(1.0 / (t2 * t));
-    k.h5 = (float)(1.0 / (t2 * t2 * t));
-    k.t3 = (float)(t2 * t);
+    k.g3 = 1.0 / (t2 * t);
+    k.h5 = 1.0 / (t2 * t2 * t);
     k.nt1 = (float)(-1.0 / t);
     k.nt3 = (float)(-1.0 / (3.0 * t2 * t));
     k.tp = (float)(GTAB_PER_UNIT / t);
@@ -155,8 +158,8 @@ Scales p3d_scales(int reg, float sigma, float nu, int mask, bool direct) {
       sc.vel = -k4pi * x * x * on * f;
       sc.dG = sgn * k4pi * x * x * x * on * f;
       sc.dH = 3.0 * sc.dG * (direct ? 1.0 : 1.0 / (t * t));
-      sc.near = direct ? 1.0 / (t * t * t) : 1.0;
-      sc.visc = on * (2.0 * (double)nu / (s * s));
+      sc.visc = on * (2.0 * (double)nu / (s * s)) *
+                (std::sqrt(2.0 / M_PI) / (double)(float)std::sqrt(2.0 / M_PI));
       break;
     }
     case REG_WINCKELMANS: {

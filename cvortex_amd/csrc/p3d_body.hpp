@@ -37,8 +37,7 @@ struct P3DLayout {
 // inside the regularisation's near branch; the stretching terms of the
 // pairs beyond (Kv < 208^-3/2 in reduced units, and eta = 0 there) are
 // summed in FP32 tiles combined by TwoSum, in the F_A slots, on the far
-// branch (GaussianKernel::eval_split).  The near sum is of G itself,
-// the far one of Kv: Scales::near is the factor between them.
+// branch (GaussianKernel::eval_split).
 template <int REG, int MASK, int ACC>
 struct P3DRegs {
   static constexpr bool DBL = (ACC == ACC_COMP);
@@ -110,6 +109,7 @@ __device__ __forceinline__ void p3d_pair(const float4 sp, const float4 sa, const
     return __builtin_elementwise_maximum(__builtin_elementwise_maximum(x, y),
                                          __builtin_elementwise_abs(dz)) == 0.f;
   };
+  constexpr bool ZETA = (MASK & OUT_VISC) != 0;
   float Kv, Kh, eta, Kfar = 0.f;
   if constexpr (REG == REG_WINCKELMANS) {
     const float S = REDUCED ? __builtin_fmaf(r2, rc.inv_s2, 1.f) : r2;
@@ -121,7 +121,7 @@ __device__ __forceinline__ void p3d_pair(const float4 sp, const float4 sa, const
       eta = same ? 0.f : eta;
     }
   } else if constexpr (R::SPLIT && (MASK & OUT_DVORT) != 0) {
-    GaussianKernel<DIRECT>::template eval_split<DIRECT && (MASK & OUT_VISC) == 0>(
+    GaussianKernel<DIRECT>::template eval_split<ZETA, DIRECT && !ZETA>(
         r2, rc, tab, same_place, Kv, Kh, eta, [&](float kn, float en) {
       const double2 sxy = *pxy, szv = *pzv;
       const double k = (double)kn;
@@ -142,7 +142,7 @@ __device__ __forceinline__ void p3d_pair(const float4 sp, const float4 sa, const
     });
   } else if constexpr (R::SPLIT) {
     constexpr bool PIN = (MASK & (OUT_DVORT | OUT_VISC)) == 0;  // no FP64 near sums
-    GaussianKernel<DIRECT>::template eval_ranges<PIN>(r2, rc, tab, same_place, Kv, Kh, eta, Kfar,
+    GaussianKernel<DIRECT>::template eval_ranges<ZETA, PIN>(r2, rc, tab, same_place, Kv, Kh, eta, Kfar,
                                                        [&](float kn, float en) {
       // FP64 source strengths are read from LDS here, on the rare path (a
       // conversion of sa would be speculated out of the branch)
@@ -162,7 +162,7 @@ __device__ __forceinline__ void p3d_pair(const float4 sp, const float4 sa, const
       }
     });
   } else if constexpr (REG == REG_GAUSSIAN) {
-    GaussianKernel<DIRECT>::eval(r2, rc, tab, same_place, Kv, Kh, eta);
+    GaussianKernel<DIRECT>::template eval<ZETA>(r2, rc, tab, same_place, Kv, Kh, eta);
   } else if constexpr (REG == REG_SINGULAR) {
     RegKernel<REG_SINGULAR>::template eval<SELF != SELF_WATCH>(r2, rc, tab, Kv, Kh, eta);
     if constexpr (SELF == SELF_WATCH) smin = fminf(smin, r2);
@@ -446,7 +446,7 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const P3DConsts& 
 #pragma unroll
       for (int c = 0; c < 3; ++c) {
         if constexpr (R::SPLIT)
-          d[L::A + c] = sc.near * dacc[k][R::D_A + c] + fval(R::F_A + c);
+          d[L::A + c] = dacc[k][R::D_A + c] + fval(R::F_A + c);
         else
           d[L::A + c] = R::DBL ? dacc[k][R::D_A + c] : fval(R::F_A + c);
         d[L::H + c] = fval(R::F_H + c);
