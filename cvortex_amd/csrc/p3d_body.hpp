@@ -367,6 +367,12 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const P3DConsts& 
       // the LDS index runs in a VGPR too: an SGPR index would cost an
       // SGPR-reading move per source to form the ds_read address
       int jv = in_vgpr(part);
+      // The place of this loop in its 32 bytes matters where the issue is full: 128
+      // clouds take 41.9 ms with its start at 12 or 16 of them, where this puts it,
+      // 42.4 at 20 or 28 and 43.6 at 0, 4 or 8 (measured for this form only).
+      if constexpr (REG == REG_WINCKELMANS && MASK == (OUT_VEL | OUT_DVORT) && ACC == ACC_TILES &&
+                    T == 1 && decltype(mode)::value == SELF_WATCH)
+        asm volatile(".p2align 5");
 #pragma unroll kUnroll
       for (int j = part; j < end; ++j, ++jv) {
         const float4 xa = sm.xa[jv];
