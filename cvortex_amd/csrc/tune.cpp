@@ -147,6 +147,11 @@ LaunchCfg narrow_cfg(int kind, int reg, int mask, int n_src, int n_tgt, int cus)
   return c;
 }
 
+// Each partition's sums are read by one lane after another in the reduction: 2^20
+// 2D sources on 64 targets, us, with 256 / 512 / 1024 / 2048 partitions 106 / 92 / 99
+// / 120 (planetary).
+constexpr long long MOST_PARTITIONS = 512;
+
 // 2D problems that are not narrow.  One target per lane is bound by the LDS: a
 // source's 16 bytes take its port 8 cycles per wave, 32 for the four SIMDs of a
 // CU, as long as 16 issue slots, where a far pair needs 11.  So two targets per
@@ -161,6 +166,13 @@ LaunchCfg narrow_cfg(int kind, int reg, int mask, int n_src, int n_tgt, int cus)
 // with two.  More partitions alone:
 // Gaussian velocity and exchange 21000 particles 307 -> 208, singular 9000 34.3
 // -> 29.7.
+// Two targets per lane at least where that leaves 4 workgroups per CU, one for up to
+// 2048 targets; tiles halved among partitions below 2 workgroups per CU only, whose
+// partial sums cost more than an uneven end where targets are many; and at most
+// MOST_PARTITIONS.  us, without these lines -> with them: 1 source on 2^20 targets,
+// Gaussian with the exchange 14.5 -> 10.4, 250, Winckelmans with it 166 -> 156, 512,
+// planetary 136 -> 123; 2^20 sources on 64 targets, planetary 227 -> 92, on 1000 344
+// -> 264.
 LaunchCfg p2d_cfg(int reg, int mask, int n_src, int n_tgt, int cus) {
   const long long tiles = ((long long)n_src + 255) / 256;
   auto blocks = [&](int T) { return ((long long)n_tgt + 256LL * T - 1) / (256LL * T); };
@@ -171,10 +183,13 @@ LaunchCfg p2d_cfg(int reg, int mask, int n_src, int n_tgt, int cus) {
   else if (visc) T = work >= 24 ? 2 : 1;
   else if (reg == REG_PLANETARY || reg == REG_SINGULAR) T = work >= 1024 ? 4 : (work >= 16 ? 2 : 1);
   else T = work >= 1024 ? 4 : 1;
+  if (blocks(2) >= 4LL * cus) T = std::max(T, 2);
+  if (blocks(1) <= 8) T = 1;
   const long long nb = blocks(T);
   long long k = std::min((64LL * cus + nb - 1) / std::max(1LL, nb), std::max(1LL, tiles / 2));
-  if (nb * k < 32LL * cus) k = std::min((32LL * cus + nb - 1) / std::max(1LL, nb), tiles);
-  return launch_shape(T, (int)std::max(1LL, k), n_src);
+  if (nb * k < 32LL * cus && nb < 2LL * cus)
+    k = std::min((32LL * cus + nb - 1) / std::max(1LL, nb), tiles);
+  return launch_shape(T, (int)std::max(1LL, std::min(k, MOST_PARTITIONS)), n_src);
 }
 
 }  // namespace
