@@ -100,17 +100,21 @@ namespace {
 // box than one of 256, but its tiles are staged four times as often).
 // 2D velocities by the singular or the planetary kernel end at 16, where two
 // targets per lane win (planetary 15000 62.6 -> 56.2, 17000 68.4 -> 71.9).
-// Few sources on many targets don't go here either: with 4 blocks of 256 targets per
-// CU the chip is full as it is, and four times as many workgroups, each with its
-// own staging (and table), cost more than they share out; nor do up to 64 sources,
-// 16 for each wave, from half a block per CU on, nor less than 32.  256 targets per
-// workgroup -> 64, us, on 2^20 targets: 1 source, velocity 6.2 -> 12.0, Gaussian vel +
-// dvort 12 -> 29, 2D Gaussian 9.5 -> 45, filament 21 -> 71; 64 sources 33 -> 36, 68 -> 85,
-// 26 -> 59, 81 -> 87; 512, Gaussian 533 -> 596; on 65536 targets 1 filament 4.9 -> 8.2,
-// 16 6.7 -> 8.9; 64 on 131072 16.5 -> 18.8.
+// Few sources on many targets don't go here either: where blocks of 256 targets
+// fill the chip, four times as many workgroups, each with its own staging (and
+// table), cost more than they share out.  The line lies at 10 sources per block of
+// targets and CU (40 for the lighter 2D and the filament pairs), 32 at least, and 12
+// blocks per CU.  256 targets per workgroup -> 64, us: 1 source on 2^20 targets,
+// velocity 6.2 -> 12.0, 2D Gaussian 9.5 -> 45, filament 21 -> 71; on 65536 targets 1
+// filament 4.9 -> 8.2, 64 3D Gaussian 17.2 -> 10.0; on 131072 64 filaments 16.5 -> 18.8,
+// 64 3D Gaussian 18.1 -> 15.2; on 262144 64 2D Gaussian 12.3 -> 18.1, 250 3D Gaussian
+// 101 -> 72, 500 velocity 82 -> 60, 500 filaments 377 -> 322; on 600000 500 velocity
+// 176 -> 130, 500 filaments 587 -> 477; on 2^20 250 3D singular
+// 186 -> 198, 512 3D Gaussian 547 -> 596.
 bool narrow(int kind, int reg, int mask, int n_src, int n_tgt, int cus) {
   const long long nb = ((long long)n_tgt + 255) / 256, tiles = ((long long)n_src + 255) / 256;
-  if (nb >= 4LL * cus || n_src < 32 || (n_src <= 64 && 2 * nb >= cus)) return false;
+  if (nb >= 12LL * cus || n_src < 32 || (long long)n_src * cus < (kind == KIND_P3D ? 10 : 40) * nb)
+    return false;
   const bool light = kind == KIND_P2D && !(mask & OUT_VISC) &&
                      (reg == REG_PLANETARY || reg == REG_SINGULAR);
   return n_tgt > 0 && tiles > 0 && nb * tiles < (light ? 16LL : 24LL) * cus;
