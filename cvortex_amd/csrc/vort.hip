@@ -377,14 +377,13 @@ __global__ __launch_bounds__(256) void vort_sorted_kernel(VortKParams p) {
   }
 }
 
+// (One thread per target added up to 2048 partitions after one another: 2^20 sources
+// on 64 targets 297 -> 180 us, on 1000 582 -> 504, 300000 on 1000 206 -> 176.)
+template <int ROWS>
 __global__ __launch_bounds__(256) void vort_reduce(VortKParams p) {
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= p.n_tgt) return;
-  double d[3] = {0.0, 0.0, 0.0};
-#pragma unroll 4
-  for (int s = 0; s < p.n_split; ++s)
-#pragma unroll
-    for (int a = 0; a < 3; ++a) d[a] += p.partial[((size_t)s * 3 + a) * p.n_tgt + i];
+  int i;
+  double d[3];
+  if (!sum_partitions<3, ROWS>(p.partial, p.n_split, p.n_tgt, i, d)) return;
   const int o = p.tgt_perm ? p.tgt_perm[i] : i;
 #pragma unroll
   for (int a = 0; a < 3; ++a) p.out[3 * (size_t)o + a] = (float)(p.scale * d[a]);
@@ -578,7 +577,9 @@ hipError_t launch_vort(const VortJob& j, const LaunchCfg& c, void* ws, size_t ws
   hipLaunchKernelGGL(k, dim3(gx, n_split), dim3(256), 0, s, p);
   hipError_t e = hipGetLastError();
   if (e != hipSuccess || n_split == 1) return e;
-  hipLaunchKernelGGL(vort_reduce, dim3((j.n_tgt + 255) / 256), dim3(256), 0, s, p);
+  const int rows = reduce_rows(j.n_tgt), sums = 256 / rows;
+  hipLaunchKernelGGL(rows == 4 ? vort_reduce<4> : vort_reduce<1>, dim3((j.n_tgt + sums - 1) / sums),
+                     dim3(256), 0, s, p);
   return hipGetLastError();
 }
 
