@@ -701,6 +701,9 @@ __global__ __launch_bounds__(256) void f3d_inf_kernel(const float4* __restrict__
   }
   const bool whole = ((int)blockIdx.x + 1) * (256 * NF) <= n_fil;
   __syncthreads();
+  // a wave beyond the last column has nothing to do (no barrier below); us, its rows
+  // computed -> not: 1 column of 4 10^6 rows 1560 -> 444, 128 x 500000 210 -> 77
+  if ((int)(blockIdx.x * 256 + (tid & ~63)) * NF >= n_fil) return;
   float* o = out + (size_t)i0 * (size_t)n_fil;
   // one answer for the whole wave, so the row loop branches uniformly
   const bool share = __all(linked);
