@@ -345,7 +345,8 @@ extern "C" {
 
 // Autotune the launch shape of a device-resident P3D problem; the winner is
 // recorded in the shape cache for the problem's size bucket.  Returns 0 and
-// the winning shape, or -1.
+// the fastest shape that two numbers name (the winner, unless that shares its
+// targets among the waves of a workgroup), or -1.
 int cvtx_hip_autotune_p3d(const cvtx_hip_p3d_problem* p, int reps, int* best_T, int* best_split,
                           float* best_ms) {
   Runtime& rt = runtime();
@@ -376,8 +377,8 @@ int cvtx_hip_autotune_p3d(const cvtx_hip_p3d_problem* p, int reps, int* best_T, 
     j.tgt_perm = order_points(rt, *d, j.tgt_pv, j.n_tgt, SLOT_PERM, d->stream);
     if (!j.tgt_perm) return -1;
   }
-  float best = -1.f;
-  LaunchCfg win;
+  float best = -1.f, named_best = -1.f;
+  LaunchCfg win, named;  // the fastest, and the fastest that (T, n_split) names
   std::vector<LaunchCfg> shapes = candidates(j.n_src, j.n_tgt, d->n_cu);
   if (!j.tgt_perm && narrow(KIND_P3D, j.reg, j.mask, j.n_src, j.n_tgt, d->n_cu))
     shapes.push_back(narrow_cfg(KIND_P3D, j.reg, j.mask, j.n_src, j.n_tgt, d->n_cu));
@@ -393,13 +394,17 @@ int cvtx_hip_autotune_p3d(const cvtx_hip_p3d_problem* p, int reps, int* best_T, 
       best = ms;
       win = c;
     }
+    if (ms > 0.f && c.q == 1 && (named_best < 0.f || ms < named_best)) {
+      named_best = ms;
+      named = c;
+    }
   }
-  if (best < 0.f) return -1;
+  if (named_best < 0.f) return -1;
   cache()[Key{ordered_kind(KIND_P3D, j.reg, j.n_src, j.n_tgt), j.reg, j.mask, j.acc,
               size_bucket(j.n_src), size_bucket(j.n_tgt)}] = Entry{win.T, win.n_split, best, 256, win.q};
-  if (best_T) *best_T = win.T;
-  if (best_split) *best_split = win.n_split;
-  if (best_ms) *best_ms = best;
+  if (best_T) *best_T = named.T;
+  if (best_split) *best_split = named.n_split;
+  if (best_ms) *best_ms = named_best;
   return 0;
 }
 

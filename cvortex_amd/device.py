@@ -102,7 +102,8 @@ NOALLOC_SCRATCH_BYTES = 64 << 20
 def autotune_p3d(prob, reps=2):
     """Time the candidate launch shapes of a device problem and record the
     fastest for its size bucket (cvtx_hip_autotune_p3d).  Returns
-    (targets_per_lane, n_split, ms)."""
+    (targets_per_lane, n_split, ms) of the fastest that p3d_eval takes as a
+    shape."""
     L = lib()
     T, k, ms = ctypes.c_int(0), ctypes.c_int(0), ctypes.c_float(0.0)
     st = L.cvtx_hip_autotune_p3d(ctypes.byref(prob), reps, ctypes.byref(T), ctypes.byref(k),

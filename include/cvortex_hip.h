@@ -311,8 +311,9 @@ cvtx_hip_batch* cvtx_hip_batch_create(int n_clouds, const int* offsets, const fl
                                       int regularisation, int outputs, int accumulate, float nu);
 void cvtx_hip_batch_destroy(cvtx_hip_batch* batch);
 /* Targets per lane (1, 2, 4) and resident workgroups per CU of the
- * persistent launch (the workgroup size is kept); must precede
- * cvtx_hip_batch_rk4_init. */
+ * persistent launch (the workgroup size is kept; every wave gets targets of
+ * its own, also where the batch's shape so far was one target per lane shared
+ * by the waves of a workgroup); must precede cvtx_hip_batch_rk4_init. */
 int cvtx_hip_batch_set_shape(cvtx_hip_batch* batch, int targets_per_lane, int workgroups_per_cu);
 int cvtx_hip_batch_info(const cvtx_hip_batch* batch, int* n_units, int* grid, int* targets_per_lane);
 /* The batch's launch shape: targets per lane, workgroup size (128 or 256,
@@ -356,7 +357,9 @@ int cvtx_hip_batch_rk4_step(cvtx_hip_batch* batch, int n_steps, void* stream);
  * Times the candidate launch shapes of a device-resident problem on the
  * active device (the problem's outputs are overwritten) and records the
  * fastest for the problem's size bucket; later calls of any P3D entry point
- * in that bucket use it.  Returns 0 and the winner, or -1. */
+ * in that bucket use it.  Returns 0 and the fastest shape that
+ * cvtx_hip_p3d_eval_shape takes, with its time (a small problem's recorded one
+ * may be faster: 64 targets per workgroup, shared by its waves), or -1. */
 int cvtx_hip_autotune_p3d(const cvtx_hip_p3d_problem* p, int reps, int* best_T, int* best_split,
                           float* best_ms);
 /* Save / load the shape cache as text; load returns the number of entries. */
