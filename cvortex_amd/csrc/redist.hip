@@ -1062,9 +1062,9 @@ constexpr int kNotByBlocks = -2;
 
 // Nodes by blocks of the grid (see above): their number, -1 with the error
 // recorded, or kNotByBlocks where the grid's keys are too long for the
-// bitmaps or particles so scattered that the blocks' sums would take more
-// than kBlockBytes.
-constexpr size_t kBlockBytes = (size_t)4 << 30;
+// bitmaps or particles so scattered that the blocks' regions would make more
+// than kMostItems items, whose sums (1.5 KB each in 3D) take 1.5 GiB.
+constexpr size_t kMostItems = (size_t)1 << 20;
 
 template <int DIM>
 int by_blocks(Runtime& rt, Device& d, const RedistJob& j, const Grid& g, int key_bits, Nodes* out,
@@ -1082,7 +1082,7 @@ int by_blocks(Runtime& rt, Device& d, const RedistJob& j, const Grid& g, int key
                                                  key_bits, s);
   if (e == hipSuccess)
     e = rocprim::inclusive_scan(nullptr, scan_tmp, (int*)nullptr, (int*)nullptr,
-                                (size_t)std::max(cw, 1 << 20), rocprim::plus<int>(), s);
+                                std::max((size_t)cw, kMostItems), rocprim::plus<int>(), s);
   if (e != hipSuccess) return rd_fail(rt, "redistribution sort size", e);
   // ---- particles by cell, the bitmaps and their running counts ----
   const size_t need = al256(sizeof(unsigned) * n) * 2 + al256(sizeof(int) * n) * 2 +
@@ -1125,11 +1125,11 @@ int by_blocks(Runtime& rt, Device& d, const RedistJob& j, const Grid& g, int key
   if (nb == 0) return kNotByBlocks;
   // ---- items of each block's region, their sums ----
   const size_t most = (size_t)nb + (size_t)kRegionsOfACell * n / kItem + 1;
+  if (most > kMostItems) return kNotByBlocks;
   constexpr int SW = DIM == 3 ? 3 : 1;
   const size_t sneed = al256(sizeof(unsigned) * nb) + al256(sizeof(int) * nb) * 4 +
                        al256(sizeof(int2) * most) + al256(sizeof(double) * 64 * SW * most) +
                        al256(8 * most) + al256(8 * (size_t)nb) + al256(scan_tmp);
-  if (sneed > kBlockBytes || most > (1 << 20)) return kNotByBlocks;
   Arena sr;
   sr.base = (char*)device_buffer(rt, d, SLOT_RD, sneed);
   sr.cap = sneed;
