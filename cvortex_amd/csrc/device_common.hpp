@@ -59,6 +59,7 @@ struct P3DConsts : RegConsts {
   // log(2) times what c1 lacks of its value in FP64 (used by the near ranges only)
   float nt1 = -1.f, nt3 = -1.f / 3.f, tp = GTAB_PER_UNIT, c1_rest = 0.f;
   double g3 = 1, h5 = 1;  // 1/t^3, 1/t^5: factors of the table's G and H/3
+  double tp_error = 0;    // relative rounding of tp
 };
 
 // A uniform value that a pair loop reads on every pair, held in a VGPR.  On
@@ -286,11 +287,20 @@ struct GaussianKernel {
     }
   }
 
-  // Entry i of the table in the kernel's units.
-  static __device__ __forceinline__ float4 table_entry(const float4 v, int i, const P3DConsts& k) {
-    if constexpr (!DIRECT) return v;
-    const double f = i & 1 ? k.h5 : k.g3;
-    return make_float4((float)(v.x * f), (float)(v.y * f), (float)(v.z * f), (float)(v.w * f));
+  // Entry i of the table in the kernel's units.  DIRECT: from the FP64 copy behind
+  // the FP32 one, so that it is rounded once, and as a function of the argument
+  // that the kernel forms, 1 + d times the true one for the rounding d of tp:
+  // p(u) - d (i + u) p'(u) for the piece i, to first order in d, again a cubic.
+  static __device__ __forceinline__ float4 table_entry(const float4* __restrict__ gtab, int i,
+                                                       const P3DConsts& k) {
+    if constexpr (!DIRECT) return gtab[i];
+    const double2* d = reinterpret_cast<const double2*>(gtab + 2 * GTAB_N) + 2 * i;
+    const double f = i & 1 ? k.h5 : k.g3, e = k.tp_error, t = (double)(i >> 1);
+    const double2 a = d[0], b = d[1];  // p(u) = a.x + a.y u + b.x u^2 + b.y u^3
+    return make_float4((float)(f * (a.x - e * (t * a.y))),
+                       (float)(f * (a.y - e * (a.y + 2.0 * t * b.x))),
+                       (float)(f * (b.x - e * (2.0 * b.x + 3.0 * t * b.y))),
+                       (float)(f * (b.y - e * (3.0 * b.y))));
   }
 
   // PIN: keep the near range a branch.  With no work of its own in

@@ -66,7 +66,7 @@ void cubic_through(const double* u, const double* f, double* c) {
 
 }  // namespace
 
-void build_gaussian_table(float* out) {
+void build_gaussian_table(double* out) {
   // Chebyshev nodes on [0,1] make each cubic a near-minimax fit of its piece.
   double u[4];
   for (int j = 0; j < 4; ++j) u[j] = 0.5 - 0.5 * std::cos((2.0 * j + 1.0) * M_PI / 8.0);
@@ -80,8 +80,8 @@ void build_gaussian_table(float* out) {
     cubic_through(u, fg, cg);
     cubic_through(u, fh, ch);
     for (int c = 0; c < 4; ++c) {
-      out[8 * i + c] = (float)cg[c];
-      out[8 * i + 4 + c] = (float)ch[c];
+      out[8 * i + c] = cg[c];
+      out[8 * i + 4 + c] = ch[c];
     }
   }
 }

@@ -47,7 +47,7 @@ struct P3DJob {
   int acc = ACC_COMP;
   float sigma = 1.f;
   float nu = 0.f;
-  const float4* gtab = nullptr;  // Gaussian table (device), 2*GTAB_N float4
+  const float4* gtab = nullptr;  // Gaussian table (device), 2*GTAB_N float4, then in FP64
   double* partial = nullptr;     // workspace for n_split > 1
   const int* tgt_perm = nullptr; // optional target order: slot i handles target tgt_perm[i]
 };
@@ -162,7 +162,7 @@ bool p2d_supported(int reg, int mask);
 
 // Gaussian near-field table (2*GTAB_N float4): cubic pieces of G and H/3,
 // computed in FP64 on the host.
-void build_gaussian_table(float* out /* 8*GTAB_N floats */);
+void build_gaussian_table(double* out /* 8*GTAB_N */);
 
 // Copy of at most kStageMax bytes, a multiple of 4, between pinned host memory and
 // the device (stage.hip); both 16-byte aligned.  Larger ones go through HIP.

@@ -38,7 +38,7 @@ __global__ __launch_bounds__(WG) void p3d_kernel(P3DKParams p) {
   __shared__ P3DShare<MASK, Q> share;
   if constexpr (REG == REG_GAUSSIAN) {
     for (int i = threadIdx.x; i < 2 * GTAB_N; i += WG)
-      sm.tab[i] = GaussianKernel<Q == 1>::table_entry(p.gtab[i], i, p.rc);
+      sm.tab[i] = GaussianKernel<Q == 1>::table_entry(p.gtab, i, p.rc);
   }
   const int s0 = blockIdx.y * p.split_len;
   const int s1 = min(s0 + p.split_len, p.n_src);
@@ -110,6 +110,7 @@ P3DConsts p3d_consts(int reg, float sigma, int mask, int acc, bool direct) {
     k.nt1 = (float)(-1.0 / t);
     k.nt3 = (float)(-1.0 / (3.0 * t2 * t));
     k.tp = (float)(GTAB_PER_UNIT / t);
+    k.tp_error = (double)k.tp * t / GTAB_PER_UNIT - 1.0;
     // Where no pair's FP64 sum and no zeta depends on it, the far form is taken
     // from where the near one rounds to it: 1 - rho zeta = 1 from rho^2 = 38 on,
     // and G - zeta/3 = G from 44 on.  Bit for bit the same results; velocity, us:

@@ -111,10 +111,14 @@ static bool make_ready(Runtime& rt, Device& d) {
     o->own = d.stream;
   }
   if (!attach_scratch(rt, d)) return false;
-  float tab[8 * GTAB_N];
-  build_gaussian_table(tab);
+  struct {
+    float f[8 * GTAB_N];
+    double d[8 * GTAB_N];
+  } tab;
+  build_gaussian_table(tab.d);
+  for (int i = 0; i < 8 * GTAB_N; ++i) tab.f[i] = (float)tab.d[i];
   if (!check_hip(rt, hipMalloc(&d.gtab, sizeof(tab)), "hipMalloc(table)")) return false;
-  if (!check_hip(rt, hipMemcpy(d.gtab, tab, sizeof(tab), hipMemcpyHostToDevice), "hipMemcpy(table)"))
+  if (!check_hip(rt, hipMemcpy(d.gtab, &tab, sizeof(tab), hipMemcpyHostToDevice), "hipMemcpy(table)"))
     return false;
   d.ready = true;
   return true;

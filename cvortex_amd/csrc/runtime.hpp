@@ -65,7 +65,7 @@ struct Device {
   bool ready = false;
   int n_cu = 0;
   hipStream_t stream = nullptr;
-  float4* gtab = nullptr;  // Gaussian near-field table
+  float4* gtab = nullptr;  // Gaussian near-field table, in FP32 and then in FP64
   // The slot buffers are shared by every call on the device, whatever its
   // stream; so is the fixed scratch array of the no-allocation entry point
   // (noalloc.hip).  Each UseOrder marks the end of the last call's use of

@@ -448,7 +448,9 @@ void cvtx_hip_tune_clear(void) { cache().clear(); }
 
 int cvtx_hip_gaussian_table(float* out, int capacity) {
   if (out == nullptr || capacity < 8 * GTAB_N) return -1;
-  build_gaussian_table(out);
+  double tab[8 * GTAB_N];
+  build_gaussian_table(tab);
+  for (int i = 0; i < 8 * GTAB_N; ++i) out[i] = (float)tab[i];
   return 8 * GTAB_N;
 }
 
