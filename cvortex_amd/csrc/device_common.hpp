@@ -43,7 +43,7 @@ constexpr int GTAB_N = GTAB_PER_UNIT * GTAB_RHO_MAX;  // 96 pieces
 struct RegConsts {
   float s2;        // sigma^2
   float inv_s2;    // 1/sigma^2
-  float c1;        // gaussian: -log2(e)/2 | 2D winckelmans eta: 4 log2(e)
+  float c1;        // gaussian: -log2(e)/2 (3D: /t^2) | winckelmans: 2D eta 4 log2(e), 3D 1.5 sigma^2
   float c2;        // gaussian: sqrt(2/pi)
   float q_far = 208.f;  // gaussian: rho^2 from which the far form is taken (p3d_consts)
   float q_exp = 46.f;   // 3D gaussian: rho^2 from which 1 - rho zeta and G - zeta/3 round to 1 and G
@@ -214,9 +214,9 @@ struct GaussianKernel {
   // So !DIRECT (r^2 taken in units of sigma^2, t = 1) where most rounds (a wave
   // and a source) have a near pair: targets that are not ordered, that is clouds
   // and small problems (q = 4).  Reduced -> DIRECT: ring of 2^20 661.8 -> 635 ms,
-  // velocity of a ring of 100000 4005 -> 3953 us, its error against 64 bits
-  // 7.2e-8 -> 5.3e-8, of the ring of 65536 1.2e-7 -> 8.1e-8; but 48 clouds 16.3
-  // -> 17.0 ms and 3.3e-7 -> 3.4e-7.
+  // velocity of a ring of 100000 4005 -> 3953 us, the error of velocity and
+  // stretching of a ring of 65536 against 64 bits 1.2e-7 -> 5.4e-8; but 48 clouds
+  // 16.3 -> 17.0 ms.
   // Three ranges of rho^2 (limits in r^2), nested so that a wave runs only the ranges its
   // lanes need (for spatially ordered targets, order.hip, a wave's lanes
   // are close together and most sources fall in the first range for all):
@@ -333,7 +333,7 @@ struct GaussianKernel {
   // The same with the far range's own work in a callback on an else
   // branch, far_cb(G): the caller needs no copy of G that the near branch
   // would zero (a register copy per pair otherwise).  Ring of 2^20, fused
-  // vel + dvort: 694.5 -> 679.1 ms (three A/B pairs on one box).
+  // vel + dvort: 694.5 -> 679.1 ms (three runs of each in turn).
   // NEST: for callers that use neither zeta nor, below rho^2 = 208, anything
   // but FP64 sums of G: beyond q_exp (there 1 - rho zeta and 1 - zeta/(3 G) round
   // to 1) G and H are the far form's, bit for bit, and the exp is skipped.  Of

@@ -536,7 +536,8 @@ F3Fn f3_reduce(int mask) {
 // Influence matrix (cvtx_F3D_inf_mtrx, reference src/F3D.cpp:204-227):
 //   out[i * n_fil + j] = vel(filament j, point i) . dir_i
 // with the filament's own strength and, as in f3d_kernel, non-finite terms
-// flushed to zero.  Each lane owns NF adjacent filaments (columns) of its
+// flushed to zero (a strength that is not finite where the columns are loaded, the
+// rest by the general form below).  Each lane owns NF adjacent filaments (columns) of its
 // workgroup's block and the workgroup walks `rows` consecutive points, staged
 // in LDS (a broadcast read puts them in VGPRs; an SGPR operand would halve
 // the issue rate of every instruction that reads it).

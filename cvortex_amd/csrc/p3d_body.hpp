@@ -69,11 +69,12 @@ struct P3DKParams {
 };
 
 // How a Winckelmans pair with equal coordinates, or a singular one with r^2 = 0,
-// is dropped (the others test r^2 == 0 in their own kernels).  SELF_NONE: it need
+// is dropped (the others test for it in their own kernels).  SELF_NONE: it need
 // not be, the velocity term being Kv (d x a_s) with d = 0 and Kv finite.
-// SELF_TEST: a compare per pair.  SELF_WATCH: only the smallest r^2 (+ sigma^2)
-// of the tile is kept, a third as many instructions; where it is that of such a
-// pair the caller repeats the tile with SELF_TEST (see p3d_block).
+// SELF_TEST: a compare per pair.  SELF_WATCH: only the tile's smallest r^2 is kept
+// (r^2 + sigma^2 for Winckelmans without the exchange), a third as many
+// instructions; where it is that of such a pair the caller repeats the tile with
+// SELF_TEST (see p3d_block).
 enum SelfMode : int { SELF_NONE, SELF_TEST, SELF_WATCH };
 
 // A coordinate in the kernel's units.  Gaussian: one that overflows there (a particle
@@ -249,7 +250,7 @@ __device__ __forceinline__ void p3d_finish(const double* a, float3 at, float vt,
 // every pair: staged as {x, y, z, ax} and {ay, az} (with the viscous term
 // {ay, az, volume, -}), it is one 16-byte and one 8-byte read, where
 // {x, y, z, volume} and {ax, ay, az, -} took two 12-byte reads.  Measured on
-// the 2^20 ring, same box: fused vel + dvort 671.4 -> 659.7 ms, dvort alone
+// the 2^20 ring: fused vel + dvort 671.4 -> 659.7 ms, dvort alone
 // 595.0 -> 585.6 ms, vel + dvort + visc 695.4 -> 673.0 ms, identical results.
 template <int REG, int MASK, int ACC, int WG>
 struct P3DSmem {
@@ -391,14 +392,16 @@ __device__ __forceinline__ void p3d_block(const P3DKParams& p, const P3DConsts& 
     // Winckelmans with stretching or viscous terms: a target meets itself (or
     // another particle at its place) in one tile of many, so the tile's sums
     // are formed without a test and formed again with it only where some
-    // pair's S was sigma^2 (r below 2^-12 sigma).  Both give the same value
+    // pair's r^2 was 0 or, where S starts from sigma^2, S was (r below 2^-12
+    // sigma).  Both give the same value
     // for every other pair.  One FP32 running sum cannot be taken back.
     // With Q > 1 the partitions are of a few tiles, and it tests each pair
     // (4000 particles, vel + dvort, 31.0 -> 26.0 us).
     // With S formed from sigma^2 (RegKernel) 36 issue slots per pair instead
     // of 41, ms: 128 clouds, tile-compensated 51.1 -> 46.6; 64 clouds, FP64
-    // stretching 32.1 -> 30.8; 400000 particles with the viscous term 147.4 ->
-    // 141.0; velocity of 100000 (S alone) 4.38 -> 4.06.
+    // stretching 32.1 -> 30.8; velocity of 100000 (S alone) 4.40 -> 4.07.  With the
+    // exchange, where S is r^2/sigma^2 + 1, 400000 particles 146.7 -> 143.4 by the
+    // test per tile alone.
     // Singular, whose Kv is infinite there, likewise (r^2 = 0) for every output:
     // a compare and one or two selects less.  100000 particles on 300000, velocity
     // 11.95 -> 11.16 ms, with the stretching 20.50 -> 19.23.

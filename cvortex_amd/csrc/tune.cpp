@@ -132,7 +132,9 @@ bool narrow(int kind, int reg, int mask, int n_src, int n_tgt, int cus) {
 // sums are one group's reduction), and where one tile holds all sources, only
 // for pairs that cost more than the second launch: 256 particles by the Gaussian
 // 18.2 -> 10.4 and Winckelmans vel + dvort 8.5 -> 7.0, but velocity 5.7 -> 6.8
-// and 100 particles 5.2 -> 6.8.
+// and 100 particles 5.2 -> 6.8.  Without quarters a few targets' many partitions pay:
+// 2^20 sources on 64 targets, us, against 256 targets per workgroup: velocity 161 ->
+// 89, with stretching and exchange 541 -> 256, Gaussian 434 -> 203, filaments 593 -> 243.
 LaunchCfg narrow_cfg(int kind, int reg, int mask, int n_src, int n_tgt, int cus) {
   const long long groups = ((long long)n_tgt + 63) / 64, tiles = ((long long)n_src + 255) / 256;
   auto fill = [&](long long per_cu) { return std::max(1LL, (per_cu * cus + groups - 1) / groups); };
@@ -214,11 +216,11 @@ LaunchCfg choose_cfg(int kind, int reg, int mask, int acc, int n_src, int n_tgt,
   // leaving them as the launch's tail.  Enough partitions for about 64
   // workgroups per CU, and at least one per 65536 sources, but no more than
   // about 256 workgroups per CU.  Measured on the ring (vel+dvort, ms; one
-  // partition -> this rule, on different boxes):
+  // partition -> this rule, on different machines):
   //   2^14: 0.29 -> 0.26 (64 partitions),  2^16: 3.73 -> 2.85 (64),
   //   2^18: 58.0 -> 42.4 (16; 32 and 64 the same),
   //   2^20: 710.6 -> 665.5 (16; 4 partitions: 673.6, 32: 665.3),
-  //   2^22: 13742 -> 10564 (4; 1 partition on that box: 10703).
+  //   2^22: 13742 -> 10564 (4; 1 partition on that machine: 10703).
   // vel alone and vel+dvort+visc at 2^20 also gain 1.2-1.4 % from 4 to 16.
   // The plain FP32 kernel has no FP64 branch and keeps the general shape
   // (two targets per lane: 678 ms against 861 ms with one at 2^20).

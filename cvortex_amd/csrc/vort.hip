@@ -211,14 +211,17 @@ __global__ __launch_bounds__(WG) void vort_kernel(VortKParams p) {
 // finite is dropped and a target with one gets zero: the reference's box test
 // fails for all its pairs.
 //
-// Bound by vector issue: about 13 issue slots for an untested pair and 18 for
-// a tested one.  On the 2^20 ring (sigma 0.02) 2.3 % of all pairs are within
-// the box; chunk boxes alone leave 4.2 % to visit (20 % of them untested), the
-// per-source test 3.2 % (43 % untested).  A relaxation step there, ms: 22.9
-// with one box test per workgroup and tile, shared tiles and every pair
-// tested; 15.8 with a wave's own chunks; 11.85 with the queues and partitions
-// of interleaved chunks.  2^18: 2.29 -> 1.13, 2^16: 0.37 -> 0.225, 2^14:
-// 0.106 -> 0.077.
+// Bound by the LDS: with one target per lane a source's 24 bytes take its port
+// 12 cycles per wave, 48 for the four SIMDs of a CU, as long as 24 issue slots,
+// where an untested pair needs about 13 and a tested one 18.  On the 2^20 ring
+// the port is busy in 76 % of the cycles and the vector units issue 0.34
+// instructions per SIMD and cycle (68 % of the most they can), in 10.9 ms.
+// There (sigma 0.02) 2.3 % of all pairs are within the box; chunk boxes alone
+// leave 4.2 % to visit (20 % of them untested), the per-source test 3.2 % (43 %
+// untested).  A relaxation step, ms: 22.9 with one box test per workgroup and
+// tile, shared tiles and every pair tested; 15.8 with a wave's own chunks; 11.85
+// with the queues and partitions of interleaved chunks.  2^18: 2.29 -> 1.13,
+// 2^16: 0.37 -> 0.225, 2^14: 0.106 -> 0.077.
 template <int REG, int ACC, int T>
 __global__ __launch_bounds__(256) void vort_sorted_kernel(VortKParams p) {
   // queue entries {x, y, z, alpha x}, {alpha y, alpha z}: a ring of two
@@ -491,7 +494,7 @@ LaunchCfg vort_default_cfg(int n_src, int n_tgt, int n_cu, bool sorted) {
   // 32 of them even for many waves (ring 2^20, ms, 4 / 8 / 16 / 32 / 64:
   // 13.6 / 12.4 / 11.9 / 11.8 / 12.2; 2^16: 0.35 / 0.26 / 0.24 / 0.23 / 0.24),
   // more where the targets are too few to fill the chip (300000 sources on
-  // 20000 targets, 32 / 64: 0.48 / 0.44), but eight chunks each (2^14: 32
+  // 20000 targets, 32 / 64: 0.48 / 0.44), but eight chunks (two tiles) each (2^14: 32
   // partitions 77 us, 64 84 us).  The FP64 partial sums (24 B per target and
   // partition) are held to 2^26 target-partitions, 1.5 GiB.
   LaunchCfg c;
