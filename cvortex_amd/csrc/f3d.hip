@@ -692,9 +692,11 @@ __global__ __launch_bounds__(256) void f3d_inf_kernel(const float4* __restrict__
     c.b[f] = make_float3(fb4.x, fb4.y, fb4.z);
     c.r0[f] = make_float3(fb4.x - fa4.x, fb4.y - fa4.y, fb4.z - fa4.z);
     c.L2[f] = dot3(c.r0[f], c.r0[f]);
-    // (a strength that is not finite gives elements of 0, in either form)
+    // (a strength that is not finite and a filament of no length give elements of 0,
+    // in either form: c = 0 times a factor that overflows would be NaN)
     const float g = fa4.w * (float)(1.0 / (4.0 * M_PI));
-    c.g[f] = __builtin_isfinite(g) ? 2.f * g : 0.f;
+    const bool none = c.r0[f].x == 0.f && c.r0[f].y == 0.f && c.r0[f].z == 0.f;
+    c.g[f] = __builtin_isfinite(g) && !none ? 2.f * g : 0.f;
     if (f > 0)
       linked = linked && __float_as_uint(c.a[f].x) == __float_as_uint(c.b[f - 1].x) &&
                __float_as_uint(c.a[f].y) == __float_as_uint(c.b[f - 1].y) &&
